@@ -26,6 +26,11 @@ namespace cmbl {
 
 __host__ __device__ inline long moff(int L, int m) { return (long)m * (L + 1) - (long)m * (m - 1) / 2; }
 
+// The synthesis input alm has 16 zeros after each m's row: entry (l, m) at
+// aoff(L, m) + (l - m) (the synthesis runs whole blocks of 16 l-steps).
+constexpr int kAlmPad = 16;
+__host__ __device__ inline long aoff(int L, int m) { return moff(L, m) + (long)kAlmPad * m; }
+
 // ---------------------------------------------------------------- HEALPix NEST <-> RING
 // The 12 base pixels (faces) of the HEALPix sphere (Gorski et al. 2005): face
 // f spans rings around jrll[f] * nside and starts at longitude index
@@ -157,16 +162,11 @@ constexpr int kMaxFFT = 8192;          // largest LDS FFT (complex doubles)
 // layout (one spare slot per 16 values).
 constexpr int lds_bytes(int n) { return (n + n / 16) * 16; }
 constexpr int kMaxLds = lds_bytes(kMaxFFT);  // 136 KiB
-constexpr int kRedChunk = 8;           // l-steps per cross-lane reduction in the adjoint
-constexpr int kRedStride = 17;         // doubles per lane row in the reduction buffer
-constexpr int kChunk = 64;             // l-steps per LDS-staged coefficient chunk
-constexpr int kChunkPad = 8;           // padding for speculative reads past a chunk
-constexpr int kAdjChunk = 2 * kChunk;  // l-steps per staged chunk in the adjoint
-constexpr int kSynChunk = 2 * kChunk;  // l-steps per staged chunk in the synthesis
+constexpr int kSynChunk = 128;  // l-steps of one correction of x^2 in the synthesis
 
 struct MapDesc {
     int nside, L, npair, npair_pad, nring;
-    int nrb5;                 // ring blocks of the adjoint Legendre stage
+    int nrb5;                 // ring blocks (partial sums) of the adjoint
     long npix, nalm;
     // ring-pair tables [npair_pad]
     const double* ring_x;     // cos(theta) of the north ring
@@ -188,14 +188,12 @@ struct MapDesc {
     const double* seed_v;     // [(L+1) * npair_pad] scaled lambda_mm
     const int* seed_k;        // [(L+1) * npair_pad] scale count
     // recurrence state at each work item's first live l, per stage layout:
-    // (mu_{l-1}, mu_l) scaled, and the scale count; [(L+1) * npair_pad]
+    // (mu_{l-1}, mu_l) scaled, members of odd l - m divided by x, and the scale
+    // count; [(L+1) * npair_pad]
     const double* s1_prev;
     const double* s1_cur;
     const int* s1_k;
-    const double* s5_prev;
-    const double* s5_cur;
-    const int* s5_k;
-    const double* A;          // [nalm] recurrence coefficient of mu_l = A x mu_{l-1} - mu_{l-2}
+    const double* A;          // [nalm + 16] recurrence coefficient of mu_l = A x mu_{l-1} - mu_{l-2}
     const double* Nrm;        // [nalm] lambda_lm = Nrm * mu_lm
     const double* beam;       // [L+1]
     const double* invcl;      // [L+1] 1/C_l or 0
@@ -203,7 +201,7 @@ struct MapDesc {
     const double* d;          // [npix]
     const double* w;          // [npix]
     // per-evaluation workspace
-    double2* alm;             // [nalm] B_l N_lm a_lm, m-major
+    double2* alm;             // B_l N_lm a_lm, m-major with padded rows (aoff)
     double* P;                // [npair * (L+1) * 4] synthesis parity sums
     double* Q;                // [npair * (L+1) * 4] adjoint ring transforms
     double* upart;            // [nrb5 * nalm * 2]
@@ -222,9 +220,8 @@ struct WorkItem {
     int mcnt;
     int rb;
     int lfirst;
-    int lend;  // last l of the item (the adjoint's segments end before L)
-    int sidx;  // start-state slot of an adjoint segment (-1: indexed by m)
-    int pad_;
+    int sub;  // entry of MmaSub (matrix-core adjoint)
+    int pad_[2];
 };
 
 // Ring items of one launch: consecutive entries of the ring list that share
@@ -236,6 +233,32 @@ struct RingClass {
 struct ItemCost {
     WorkItem it;
     double cost;
+};
+
+// Adjoint work item: degree m, degrees l0 .. of one block of 64 K ring pairs
+// from p0, nrow rows of eight l-steps (l0 - m even; entries past lend are not
+// stored).  Group k of 64 pairs runs from row row[k] (non-increasing in k),
+// starting from st[64 k ..], sk[64 k ..].  nrow = 0 marks padding.
+struct AdjItem {
+    const double2* st;  // (mu_{l-2}, mu_{l-1}) at each group's first row
+    const int* sk;      // scale counts
+    const double* A;    // recurrence coefficients of degree m, by l
+    const double* x;    // cos theta of the ring pairs
+    const double* Q;    // Psi of degree m of ring pair 0, stride 4 (L + 1)
+    double* u;          // the block's partial sums of degree m, by l (re, im)
+    int map, m0, l0, lend, nrow;
+    int p0, npair, L, part, seg;
+    unsigned short row[8];
+};
+struct AdjCost {
+    AdjItem it;
+    double cost;
+};
+// Set-up of one group of 64 ring pairs from p0: its state at row start l.
+struct AdjCap {
+    double2* st;
+    int* sk;
+    int m, p0, l, pad_;
 };
 
 // A ring pair of a map; with pair2 >= 0 also a second ring pair (of map2) of
@@ -286,35 +309,34 @@ int hip_fail(hipError_t e, const char* what);
 // (defined in cmbl_kernels.hip)
 int launch_pre(const MapDesc& md, const MapDesc* d_md, const double* d_x, hipStream_t s);
 int launch_synth(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, hipStream_t s);
-// Shared-recurrence synthesis of groups of G maps of one geometry (G = 2, 4).
-int launch_synth_group(int K, int G, const WorkItem* items, int nitems, const MapDesc* d_maps, const int* d_groups,
+// Shared-recurrence synthesis of pairs of maps of one geometry (K = 1, 2);
+// d_groups: two map indices per pair.
+int launch_synth_pairs(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, const int* d_groups,
                        hipStream_t s);
-int launch_adj(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, hipStream_t s);
-// Shared adjoint of groups of kAdjG maps of one geometry on the FP64 matrix
-// cores: one ring pair per lane, a workgroup of kMmaWaves waves on
-// consecutive 64-pair blocks of one m; item.sidx indexes `subs` (each wave's
-// first live l and start-state slot); item.rb counts blocks of kMmaWaves * 64
-// pairs, whose partials the maps' descriptors address (nrb5 of them).
-constexpr int kAdjG = 8;
-constexpr int kAdjMinG = 3;  // fewest maps of a group (the rest of its columns empty, entry -1)
-constexpr int kSynMinG = 6;  // fewest maps of a matrix-core synthesis group (fewer share k_synth_g)
-constexpr int kMmaWaves = 4;
+int launch_adj(int K, const AdjItem* items, int nitems, hipStream_t s);
+constexpr int kSynG = 8;     // maps of a matrix-core group
+constexpr int kSynMinG = 6;  // fewest maps of such a group
+constexpr int kMmaWaves = 4;  // waves of a matrix-core adjoint workgroup, 64 ring pairs each
+// Its waves' first l (-1: none) and start states (AdjItem's form).
 struct MmaSub {
-    int lf[kMmaWaves];    // first live l of the wave's block, -1 if it has none
-    int sidx[kMmaWaves];  // its start-state slot
+    int lf[kMmaWaves];
+    const double2* st[kMmaWaves];
+    const int* sk[kMmaWaves];
 };
-// Shared synthesis of groups of up to kAdjG maps of one geometry (ring
-// pairs per lane K = 1 or 2) on the FP64 matrix cores; d_groups: kAdjG map
+// Shared adjoint of groups of up to kSynG maps of one geometry; item.rb counts
+// blocks of kMmaWaves * 64 ring pairs (the partial sums), item.sub indexes subs.
+int launch_adj_mma(const WorkItem* items, const MmaSub* subs, int nitems, const MapDesc* d_maps, const int* d_groups,
+                   hipStream_t s);
+// Shared synthesis of groups of up to kSynG maps of one geometry (ring
+// pairs per lane K = 1 or 2) on the FP64 matrix cores; d_groups: kSynG map
 // indices per group (-1: empty).
 int launch_synth_mma(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, const int* d_groups,
                      hipStream_t s);
-int launch_adj_mma(const WorkItem* items, const MmaSub* subs, int nitems, const MapDesc* d_maps, const int* d_groups,
-                   hipStream_t s);
 int lm_tiles(int L);  // blocks of k_pre / k_post (prior partial sums)
 int launch_ldiv(double* y, const double* x, const double* dl, int L, hipStream_t s);
-// spin-2 synthesis: kPolRec complex coefficients per (l, m); parity sums of
+// spin-2 synthesis: kPolRec doubles of coefficients per (l, m); parity sums of
 // T, Q and U in three buffers laid out as MapDesc::P
-constexpr int kPolRec = 5;
+constexpr int kPolRec = 14;
 int launch_pre_pol(const MapDesc& md, const MapDesc* d_md, const double* t, const double* e, const double* b,
                    double2* d_rec, hipStream_t s);
 int launch_synth_pol(int K, const WorkItem* items, int nitems, const MapDesc* d_md, const double2* d_rec,
@@ -343,6 +365,7 @@ int launch_post_batch(const MapDesc* d_mds, const BatchArgs& a, int mode, hipStr
 int launch_final_batch(const MapDesc* d_mds, const BatchArgs& a, hipStream_t s);
 int launch_bluestein_setup(const MapDesc* d_md, const int* d_pairs, int npairs_bs, double2* d_out,
                            double2* d_chirp, int lds_bytes, const double2* d_tw, hipStream_t s);
+int launch_adj_capture(const AdjCap* caps, int n, const MapDesc* d_md, hipStream_t s);
 int launch_scan(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, int* d_lstart,
                 hipStream_t s);
 int launch_capture(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, double* d_prev, double* d_cur,
@@ -377,14 +400,16 @@ struct cmbl_map {
     cmbl::MapDesc desc{};
     cmbl::MapDesc* d_desc = nullptr;
     cmbl::WorkItem* d_items1 = nullptr;
-    cmbl::WorkItem* d_items5 = nullptr;
+    cmbl::AdjItem* d_items5 = nullptr;
     cmbl::RingItem* d_ring_items = nullptr;
     int nitems1 = 0, nitems5 = 0, nring_items = 0;
     std::vector<cmbl::RingClass> ring_classes;
     std::vector<int> ring_M;  // transform length per pair
     std::vector<int> ring_two;  // n for power-of-two unsplit pairs with n > lmax (two may share a workgroup), else 0
-    std::vector<cmbl::WorkItem> items1, items5;   // launch order (XCD-interleaved)
-    std::vector<cmbl::ItemCost> cost1, cost5;      // live items with cost estimates
+    std::vector<cmbl::WorkItem> items1;      // launch order (XCD-interleaved)
+    std::vector<cmbl::ItemCost> cost1;       // live items with cost estimates
+    std::vector<cmbl::AdjCost> cost5;
+    std::vector<int> lmin64;      // first live l (L + 1: none) per m and 64 ring pairs
     std::vector<cmbl::RingItem> ring_items;
     double2* d_tw = nullptr;
     double* d_f = nullptr;
@@ -433,27 +458,24 @@ struct cmbl_batch {
     cmbl::MapDesc* d_descs = nullptr;
     // work lists grouped by K (index = log2 K)
     cmbl::WorkItem* d_items1[4] = {nullptr, nullptr, nullptr, nullptr};
-    cmbl::WorkItem* d_items5[4] = {nullptr, nullptr, nullptr, nullptr};
-    int n1[4] = {0, 0, 0, 0}, n5[4] = {0, 0, 0, 0};
-    // shared-recurrence synthesis: groups of G maps of one geometry, their
-    // items by (K, G) (index log2 K, G = 2 or 4) and the group table
-    struct SynGroupList {
-        int K = 0, G = 0, n = 0;
-        cmbl::WorkItem* d_items = nullptr;
-    };
-    std::vector<SynGroupList> syn_groups;
-    int* d_gmaps = nullptr;
-    int ngroups = 0;
-    // shared adjoint on the matrix cores: groups of kAdjG maps of one
-    // geometry with one ring pair per lane, their items and group table
-    // matrix-core synthesis: groups of up to kAdjG maps of one geometry, items by K - 1
-    cmbl::WorkItem* d_items_smma[2] = {nullptr, nullptr};
-    int n_smma[2] = {0, 0};
-    int* d_smaps = nullptr;
+    int n1[4] = {0, 0, 0, 0};
+    // adjoint items by log2 K
+    cmbl::AdjItem* d_items5[4] = {nullptr, nullptr, nullptr, nullptr};
+    int n5[4] = {0, 0, 0, 0};
+    // matrix-core adjoint: groups of up to kSynG maps of one geometry
     cmbl::WorkItem* d_items_mma = nullptr;
     cmbl::MmaSub* d_subs_mma = nullptr;
     int n_mma = 0;
     int* d_amaps = nullptr;
+    // shared-recurrence synthesis: pairs of maps of one geometry, items by
+    // K - 1, and the table of the pairs
+    cmbl::WorkItem* d_items_pair[2] = {nullptr, nullptr};
+    int n_pair[2] = {0, 0};
+    int* d_gmaps = nullptr;
+    // matrix-core synthesis: groups of up to kSynG maps of one geometry, items by K - 1
+    cmbl::WorkItem* d_items_smma[2] = {nullptr, nullptr};
+    int n_smma[2] = {0, 0};
+    int* d_smaps = nullptr;
     cmbl::RingItem* d_ring_items = nullptr;
     int nring_items = 0;
     int lds_ring = 0;

@@ -63,6 +63,8 @@ __device__ __forceinline__ void wave_sync()
 typedef __attribute__((address_space(1))) double gdouble;
 typedef const __attribute__((address_space(1))) double gcdouble;
 typedef double __attribute__((ext_vector_type(2))) dvec2;
+// Wave-uniform coefficients through the scalar cache.
+typedef const __attribute__((address_space(4))) double scdouble;
 
 // Views of double2 arrays in global memory (16-byte loads and stores).
 struct GCView2 {
@@ -174,8 +176,7 @@ __device__ __forceinline__ void pre_tile(const MapDesc& md, const double* __rest
         const int l = l0 + lr, m = m0 + mr;
         if (l <= L && m <= l) {
             const double re = T[lr][2 * mr], im = T[lr][2 * mr + 1];
-            const long k = moff(L, m) + (l - m);
-            md.alm[k] = make_double2(sc[e] * re, sc[e] * im);
+            md.alm[aoff(L, m) + (l - m)] = make_double2(sc[e] * re, sc[e] * im);
             pr += ic[e] * ((m == 0) ? re * re : 2.0 * (re * re + im * im));
         }
     }
@@ -327,16 +328,18 @@ __global__ __launch_bounds__(256) void k_ldiv(double* y, const double* x, const 
 // c = cos(theta), s2 = sin^2(theta) and lambda_lm = Y_lm(theta, 0):
 //   F1_lm = kappa_l [-((l - m^2)/s2 + l(l-1)/2) lambda_lm + c q_lm lambda_{l-1,m} / s2]
 //   F2_lm = kappa_l (m/s2) [-(l-1) c lambda_lm + q_lm lambda_{l-1,m}].
-// Per field the sums over l need four scalar Legendre sums of one recursion:
-//   Sa = sum kappa a lambda_l,  Sb = sum l kappa a lambda_l,  Sc = sum l^2 kappa a lambda_l,
-//   D3 = sum kappa q a lambda_{l-1}  (coefficients shifted by one l),
-// and with D1 = Sb - m^2 Sa, D2 = (Sc - Sb)/2, D4 = Sb - Sa:
-//   sum_l a F1 = -D1/s2 - D2 + c D3/s2,   sum_l a F2 = m (D3 - c D4)/s2.
+// The sums over l of a field need three scalar Legendre
+// sums of one recursion,
+//   S1 = sum kappa a g lambda_l,  g = (m^2 - l) / s2 - l (l - 1) / 2,
+//   S2 = sum kappa q a lambda_{l-1}  (coefficients shifted by one l),
+//   S3 = sum (l - 1) kappa a lambda_l:
+//   sum_l a F1 = S1 + c S2/s2,   sum_l a F2 = m (S2 - c S3)/s2.
 // k_synth_pol runs the recursion once per (m, ring block) for the T sum and
-// the eight field sums and forms Q_m, U_m per ring in its epilogue.
+// the six field sums and forms Q_m, U_m per ring in its epilogue.
 
-// Record of (l, m) (m-major, kPolRec complex): N a^T, N kappa_l a^E,
-// N kappa_{l+1} q_{l+1,m} a^E_{l+1,m}, and the same two for B.
+// Record of (l, m) (m-major with padded rows, kPolRec doubles): complex N a^T;
+// N kappa_l a^E, the same of B; N kappa_{l+1} q_{l+1,m} a^E_{l+1,m}, B;
+// (l - 1) N kappa_l a^E, B.
 __global__ __launch_bounds__(256) void k_pre_pol(const MapDesc* __restrict__ md_, const double* __restrict__ t,
                                                  const double* __restrict__ e, const double* __restrict__ b,
                                                  double2* __restrict__ rec)
@@ -370,12 +373,16 @@ __global__ __launch_bounds__(256) void k_pre_pol(const MapDesc* __restrict__ md_
                               ? nr * 2.0 / sqrt((l1 - 1.0) * l1 * (l1 + 1.0) * (l1 + 2.0)) *
                                     sqrt((2.0 * l1 + 1.0) / (2.0 * l1 - 1.0) * (l1 * l1 - m2))
                               : 0.0;
-        double2* o = rec + k * kPolRec;
+        double2* o = rec + (aoff(L, m) + (l - m)) * (kPolRec / 2);
+        const double e0 = ck * T[1][lr][2 * mr], e1 = ck * T[1][lr][2 * mr + 1];
+        const double b0 = ck * T[2][lr][2 * mr], b1 = ck * T[2][lr][2 * mr + 1];
         o[0] = make_double2(nr * T[0][lr][2 * mr], nr * T[0][lr][2 * mr + 1]);
-        o[1] = make_double2(ck * T[1][lr][2 * mr], ck * T[1][lr][2 * mr + 1]);
-        o[2] = make_double2(dk * T[1][lr + 1][2 * mr], dk * T[1][lr + 1][2 * mr + 1]);
-        o[3] = make_double2(ck * T[2][lr][2 * mr], ck * T[2][lr][2 * mr + 1]);
+        o[1] = make_double2(e0, e1);
+        o[2] = make_double2(b0, b1);
+        o[3] = make_double2(dk * T[1][lr + 1][2 * mr], dk * T[1][lr + 1][2 * mr + 1]);
         o[4] = make_double2(dk * T[2][lr + 1][2 * mr], dk * T[2][lr + 1][2 * mr + 1]);
+        o[5] = make_double2((fl - 1.0) * e0, (fl - 1.0) * e1);
+        o[6] = make_double2((fl - 1.0) * b0, (fl - 1.0) * b1);
     }
 }
 
@@ -445,13 +452,30 @@ __global__ __launch_bounds__(256) void k_reorder(const double* __restrict__ in, 
 // of one map.  Lane `lane` handles ring pairs p_k = rb*64*K + k*64 + lane,
 // k < K.  The recurrence mu_l = A_lm x mu_{l-1} - mu_{l-2} runs in registers,
 // starting from the state precomputed at set-up for the item's first live l.
+//
+// Its odd members (l - m odd) are carried divided by x = cos theta, which
+// takes x out of every second step,
+//   odd:  mu_l / x = A_lm mu_{l-1} - mu_{l-2} / x
+//   even: mu_l     = A_lm x^2 (mu_{l-1} / x) - mu_{l-2},
+// so a pair of l-steps costs 3 FP64 instructions instead of 4; the sums over
+// odd l - m are multiplied by x once, at the end (synthesis) or in their
+// inputs (adjoint).  x^2 is rounded, and that one relative error, the same at
+// every step, would be a phase error growing with l: of the eight even steps
+// of every 16 l-steps the first takes x^2 plus eight times the rounding error
+// (rounded again: Ring::ya), and of every eighth 16 also eight times what that
+// rounding left (yb), so that the mean multiplier is x^2 to 2^-60 and the
+// phase never drifts by more than a few steps' rounding.  The error against
+// higher precision is then that of the plain recurrence (rms over rings,
+// nside 64 to 1024: 0.9 to 1.2 times).
 // The wave-uniform coefficients (A_lm and, for the synthesis, B_l N_lm a_lm)
-// are staged through a per-wave LDS double buffer, kChunk l-steps at a time:
-// every lane issues one vector load of the next chunk before the current
-// chunk is processed, so the loads overlap kChunk steps of FP64 work.
+// come through the scalar cache, or from a row of 16 lanes, a step group ahead:
+// read from LDS by every wave they kept its port (128 bytes per clock) as busy
+// as the multipliers (2.45 ns per instruction and SIMD, scalar operands 2.1).
 // Lanes whose scale count is > 0 are negligible (|lambda| < 2^-100): the wave
 // runs a "scaled" path with rescale checks until every lane is live, then a
-// check-free path of 4 FP64 VALU operations per (l, ring pair).
+// check-free path of 3.5 FP64 VALU operations per (l, ring pair).
+//
+// nside 1024 / lmax 2048: synthesis 527 -> 408, adjoint 650 -> 531 us.
 
 template <int K>
 __device__ __forceinline__ bool all_live(const int (&sc)[K])
@@ -488,11 +512,22 @@ __device__ __forceinline__ bool rescale(double (&mu1)[K], double (&mu2)[K], int 
     return true;
 }
 
-// Phase state shared by both Legendre kernels.
+// x^2 of a ring pair and its corrected values, from x = cos theta.
+struct Ring {
+    double y, ya, yb;
+    __device__ __forceinline__ explicit Ring(double x)
+    {
+        y = x * x;
+        const double d = fma(x, x, -y);
+        ya = fma(8.0, d, y);
+        yb = fma(8.0, fma(8.0, d, y - ya), ya);
+    }
+};
+
+// Recurrence state of the spin-2 and set-up kernels.
 template <int K>
 struct LegState {
-    double x[K];
-    double mu1[K], mu2[K];  // mu_l, mu_{l-1}
+    double mu1[K], mu2[K];  // mu_l, mu_{l-1}, odd ones divided by x (k_scan: not)
     double gate[K];         // 1 for live lanes, 0 otherwise (scaled path only)
     int sc[K];
     bool live, all;
@@ -503,309 +538,8 @@ struct LegState {
 #pragma unroll
         for (int k = 0; k < K; ++k) gate[k] = sc[k] == 0 ? 1.0 : 0.0;
     }
-    __device__ __forceinline__ void advance(double Al)
-    {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const double nu = fma(Al * x[k], mu1[k], -mu2[k]);
-            mu2[k] = mu1[k];
-            mu1[k] = nu;
-        }
-    }
 };
 
-// -------------------------------------------------------------- synthesis
-template <int K>
-struct SynAcc {
-    double er[K], ei[K], orr[K], oi[K];
-};
-
-template <int K, bool ODD>
-__device__ __forceinline__ void syn_live(LegState<K>& st, SynAcc<K>& ac, double Al, double ar, double ai)
-{
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const double nu = fma(Al * st.x[k], st.mu1[k], -st.mu2[k]);
-        st.mu2[k] = st.mu1[k];
-        st.mu1[k] = nu;
-        if (ODD) {
-            ac.orr[k] = fma(nu, ar, ac.orr[k]);
-            ac.oi[k] = fma(nu, ai, ac.oi[k]);
-        } else {
-            ac.er[k] = fma(nu, ar, ac.er[k]);
-            ac.ei[k] = fma(nu, ai, ac.ei[k]);
-        }
-    }
-}
-
-// Scaled lanes (count > 0) accumulate like live ones: their scaled mu
-// (|mu| < 2^945 between rescale checks) makes meaningless sums, which are
-// cleared when the lane turns live (its count reaching 0 at a rescale check)
-// and never stored while it is scaled, so the result equals gating each term
-// by the lane's state at the last check, without the multiplies.
-
-// The item's first l (the recurrence state is already at it).
-template <int K, bool ODD>
-__device__ __forceinline__ void syn_first(const LegState<K>& st, SynAcc<K>& ac, double ar, double ai)
-{
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        if (ODD) {
-            ac.orr[k] = fma(st.mu1[k], ar, ac.orr[k]);
-            ac.oi[k] = fma(st.mu1[k], ai, ac.oi[k]);
-        } else {
-            ac.er[k] = fma(st.mu1[k], ar, ac.er[k]);
-            ac.ei[k] = fma(st.mu1[k], ai, ac.ei[k]);
-        }
-    }
-}
-
-// Rescale check of the synthesis' scaled path: lanes above 2^900 drop by
-// 2^-1000; a lane whose count reaches 0 clears its sums.
-template <int K>
-__device__ __forceinline__ void syn_rescale(LegState<K>& st, SynAcc<K>& ac)
-{
-    int need = 0;
-#pragma unroll
-    for (int k = 0; k < K; ++k) need |= (st.sc[k] > 0) & (fabs(st.mu1[k]) > kScaleHi);
-    if (!__any(need)) return;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const bool r = st.sc[k] > 0 && fabs(st.mu1[k]) > kScaleHi;
-        st.mu1[k] = r ? st.mu1[k] * kScaleDn : st.mu1[k];
-        st.mu2[k] = r ? st.mu2[k] * kScaleDn : st.mu2[k];
-        st.sc[k] -= r ? 1 : 0;
-        const bool join = r && st.sc[k] == 0;
-        ac.er[k] = join ? 0.0 : ac.er[k];
-        ac.ei[k] = join ? 0.0 : ac.ei[k];
-        ac.orr[k] = join ? 0.0 : ac.orr[k];
-        ac.oi[k] = join ? 0.0 : ac.oi[k];
-    }
-    st.all = all_live<K>(st.sc);
-}
-
-// Four live steps with coefficients c (A), r/i (B_l N_lm a_lm), parity
-// pattern ODD0, !ODD0, ODD0, !ODD0.
-template <int K, bool ODD0>
-__device__ __forceinline__ void syn_live4(LegState<K>& st, SynAcc<K>& ac, const double (&c)[4], const double (&r)[4],
-                                          const double (&i)[4])
-{
-    syn_live<K, ODD0>(st, ac, c[0], r[0], i[0]);
-    syn_live<K, !ODD0>(st, ac, c[1], r[1], i[1]);
-    syn_live<K, ODD0>(st, ac, c[2], r[2], i[2]);
-    syn_live<K, !ODD0>(st, ac, c[3], r[3], i[3]);
-}
-
-template <int K, bool ODD0>
-__device__ __forceinline__ void syn_load4(int j, const double* cA, const double2* ca, double (&c)[4], double (&r)[4],
-                                          double (&i)[4])
-{
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        c[q] = cA[j + q];
-        r[q] = ca[j + q].x;
-        i[q] = ca[j + q].y;
-    }
-}
-
-// Groups of four live steps.  Two register sets alternate: each iteration
-// does eight steps (compute X while Y loads, compute Y while the next X
-// loads), so loads overlap arithmetic without register copies.  The speculative load of the
-// next X may read up to kChunkPad entries past the chunk; the LDS rows are
-// padded for it and the values are not used.
-template <int K, bool ODD0>
-__device__ __forceinline__ void syn_live_run(LegState<K>& st, SynAcc<K>& ac, int& l, int cend, int cb,
-                                             const double* cA, const double2* ca)
-{
-    if (l + 3 > cend) return;
-    double xc[4], xr[4], xi[4], yc[4], yr[4], yi[4];
-    syn_load4<K, ODD0>(l - cb, cA, ca, xc, xr, xi);
-    for (; l + 7 <= cend; l += 8) {
-        // each set's loads are issued after the first step that uses the
-        // other set, so the wait before that step covers only loads issued
-        // half an iteration earlier
-        syn_live<K, ODD0>(st, ac, xc[0], xr[0], xi[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        syn_load4<K, ODD0>(l + 4 - cb, cA, ca, yc, yr, yi);
-        syn_live<K, !ODD0>(st, ac, xc[1], xr[1], xi[1]);
-        syn_live<K, ODD0>(st, ac, xc[2], xr[2], xi[2]);
-        syn_live<K, !ODD0>(st, ac, xc[3], xr[3], xi[3]);
-        syn_live<K, ODD0>(st, ac, yc[0], yr[0], yi[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        syn_load4<K, ODD0>(l + 8 - cb, cA, ca, xc, xr, xi);
-        syn_live<K, !ODD0>(st, ac, yc[1], yr[1], yi[1]);
-        syn_live<K, ODD0>(st, ac, yc[2], yr[2], yi[2]);
-        syn_live<K, !ODD0>(st, ac, yc[3], yr[3], yi[3]);
-    }
-    if (l + 3 <= cend) {
-        syn_live4<K, ODD0>(st, ac, xc, xr, xi);
-        l += 4;
-    }
-}
-
-// Rows of eight steps (parity pattern ODD0, !ODD0, ...) while some lane is
-// scaled, with one rescale check per row.  Eight steps multiply |mu| by at
-// most prod (A_l + 1) < 2^45 (A_{m+1} = sqrt(2m + 2) is the largest factor),
-// so from 2^900 nothing overflows between checks; a lane whose scale count
-// reaches 0 inside a row joins at the row's end, dropping terms below 2^-55
-// of O(1).
-template <int K, bool ODD0>
-__device__ __forceinline__ void syn_scaled_rows(LegState<K>& st, SynAcc<K>& ac, int& l, int cend, int cb,
-                                                const double* cA, const double2* ca)
-{
-    for (; !st.all && l + 7 <= cend; l += 8) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const double2 al = ca[l + q - cb];
-            if (ODD0 ^ (q & 1))
-                syn_live<K, true>(st, ac, cA[l + q - cb], al.x, al.y);
-            else
-                syn_live<K, false>(st, ac, cA[l + q - cb], al.x, al.y);
-        }
-        syn_rescale<K>(st, ac);
-    }
-}
-
-// Steps l = l .. cend of one staged chunk (coefficients cA[l - cb], ca[l - cb]).
-// Scaled path: rows while eight steps remain, then single steps with a
-// rescale check after every second step.
-template <int K>
-__device__ __forceinline__ void syn_chunk(LegState<K>& st, SynAcc<K>& ac, int& l, int cend, int cb, int m,
-                                          const double* cA, const double2* ca)
-{
-    if (!st.all && l + 7 <= cend) {
-        if ((l - m) & 1)
-            syn_scaled_rows<K, true>(st, ac, l, cend, cb, cA, ca);
-        else
-            syn_scaled_rows<K, false>(st, ac, l, cend, cb, cA, ca);
-    }
-    while (!st.all && l <= cend) {
-        for (int rep = 0; rep < 2 && l <= cend; ++rep, ++l) {
-            const double2 al = ca[l - cb];
-            if ((l - m) & 1)
-                syn_live<K, true>(st, ac, cA[l - cb], al.x, al.y);
-            else
-                syn_live<K, false>(st, ac, cA[l - cb], al.x, al.y);
-        }
-        syn_rescale<K>(st, ac);
-    }
-    if (l > cend) return;
-    // all lanes live: parity pattern fixed by (l - m)
-    if ((l - m) & 1)
-        syn_live_run<K, true>(st, ac, l, cend, cb, cA, ca);
-    else
-        syn_live_run<K, false>(st, ac, l, cend, cb, cA, ca);
-    for (; l <= cend; ++l) {
-        const int j = l - cb;
-        if ((l - m) & 1)
-            syn_live<K, true>(st, ac, cA[j], ca[j].x, ca[j].y);
-        else
-            syn_live<K, false>(st, ac, cA[j], ca[j].x, ca[j].y);
-    }
-}
-
-template <int K>
-__global__ __launch_bounds__(64) void k_synth(const WorkItem* __restrict__ items, const MapDesc* __restrict__ maps)
-{
-    constexpr int CH = kSynChunk, NC = kSynChunk / 64;
-    __shared__ double sA[2][CH + kChunkPad];
-    __shared__ double2 sa[2][CH + kChunkPad];
-    const WorkItem it = items[blockIdx.x];
-    if (it.mcnt == 0) return;
-    const MapDesc& md = maps[it.map];
-    const int L = md.L;
-    const int npad = md.npair_pad;
-    const int lane = threadIdx.x;
-    const int m = it.m0;
-    const int l0 = it.lfirst;
-    const long base = moff(L, m) - m;
-    gcdouble* __restrict__ A = (gcdouble*)(md.A + base);
-    gcdouble* __restrict__ a = (gcdouble*)(md.alm + base);  // (re, im) interleaved
-
-    LegState<K> st;
-    SynAcc<K> ac;
-    int p[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        p[k] = it.rb * 64 * K + k * 64 + lane;
-        const long q = (long)m * npad + p[k];
-        st.x[k] = md.ring_x[p[k]];
-        st.mu1[k] = md.s1_cur[q];
-        st.mu2[k] = md.s1_prev[q];
-        st.sc[k] = md.s1_k[q];
-        ac.er[k] = ac.ei[k] = ac.orr[k] = ac.oi[k] = 0.0;
-    }
-    st.all = all_live<K>(st.sc);
-    {
-        const double ar = a[2 * l0], ai = a[2 * l0 + 1];
-        if ((l0 - m) & 1)
-            syn_first<K, true>(st, ac, ar, ai);
-        else
-            syn_first<K, false>(st, ac, ar, ai);
-    }
-    // staged chunks of CH steps from l0+1 to L, NC coefficients per lane
-    int cb = l0 + 1;
-    double tA[NC];
-    double2 ta[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const int j = cb + 64 * c + lane;
-        tA[c] = 0.0;
-        ta[c] = make_double2(0.0, 0.0);
-        if (j <= L) {
-            tA[c] = A[j];
-            ta[c] = make_double2(a[2 * j], a[2 * j + 1]);
-        }
-        sA[0][64 * c + lane] = tA[c];
-        sa[0][64 * c + lane] = ta[c];
-    }
-    wave_sync();
-    int buf = 0;
-    int l = cb;
-    while (cb <= L) {
-        const int nb = cb + CH;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int j = nb + 64 * c + lane;
-            if (j <= L) {
-                tA[c] = A[j];
-                ta[c] = make_double2(a[2 * j], a[2 * j + 1]);
-            }
-        }
-        const int cend = min(L, nb - 1);
-        syn_chunk<K>(st, ac, l, cend, cb, m, sA[buf], sa[buf]);
-        if (nb <= L) {
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                sA[buf ^ 1][64 * c + lane] = tA[c];
-                sa[buf ^ 1][64 * c + lane] = ta[c];
-            }
-        }
-        wave_sync();
-        buf ^= 1;
-        cb = nb;
-    }
-    // lanes still scaled at L store zeros
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        if (p[k] < md.npair) {
-            const bool z = st.sc[k] != 0;
-            double2* dst = reinterpret_cast<double2*>(md.P + ((long)p[k] * (L + 1) + m) * 4);
-            dst[0] = make_double2(z ? 0.0 : ac.er[k], z ? 0.0 : ac.ei[k]);
-            dst[1] = make_double2(z ? 0.0 : ac.orr[k], z ? 0.0 : ac.oi[k]);
-        }
-    }
-}
-
-// -------------------------------------------------------------- shared-recurrence synthesis
-// G maps of one geometry (same nside, lmax and ring pairs per lane, so the
-// same ring tables, recurrence coefficients, work items and start states)
-// in one wave: the recurrence runs once per (l, ring pair) and feeds the G
-// maps' parity sums, 2K + 2KG FP64 instructions per l-step against 4KG for
-// the maps one by one.  Item.map indexes the group table (rows of four map
-// indices, the first G used);
-// the first map supplies the geometry.  Each map's sums are formed by the
-// same operations in the same order as in k_synth, so its P is the same.
 // Compile-time loops over the maps of a group: every index is a constant
 // when the accumulators are laid out, so they stay in registers (a runtime
 // loop, even one that is unrolled later, left them in scratch).
@@ -815,52 +549,95 @@ __device__ __forceinline__ void for_each_map(std::integer_sequence<int, I...>, F
     (f(std::integral_constant<int, I>{}), ...);
 }
 
-template <int K, int G, bool ODD>
-__device__ __forceinline__ void syng_step(LegState<K>& st, SynAcc<K> (&ac)[G], double Al, const double2 (&av)[G])
+// -------------------------------------------------------------- synthesis
+template <int K>
+struct SynAcc {
+    double er[K], ei[K], orr[K], oi[K];
+};
+
+// acc += c x (or -= c x), c taken from lane N of the lane's row of 16.  The
+// rows hold the same 16 coefficients, so one register pair feeds 16 steps.  A
+// DPP operand must not have been written by the VALU in the last two
+// instructions: coefficients come straight from memory.
+template <int N, bool NEG>
+__device__ __forceinline__ void fmac_row(double& acc, double c, double x)
 {
+    if (NEG)
+        asm("v_fmac_f64_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(N));
+    else
+        asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(N));
+}
+
+// Synthesis state of a lane's K ring pairs.  With step q = l - l0 of the item,
+// the recurrence runs in place on v_q = s_q mu_{l0 + q}, s = + + - - + + - -
+// from q = 0 (v_-1 = -mu_{l0-1}), which turns mu_q = c mu_{q-1} - mu_{q-2} into
+//   u += c w (q odd),  w -= c u (q even),
+// u holding the odd and w the even members.
+template <int K>
+struct SynState {
+    double y[K], ya[K], yb[K];  // x^2 and its corrected values (Ring)
+    double u[K], w[K];
+    int sc[K];
+    bool all;
+};
+
+// Steps J + 1 + q, q = Q0 .. Q1 - 1 (J a multiple of 4), of the 16 whose A the
+// lanes hold, with scalar coefficients r, i of the G maps; x multiplies the
+// steps of even l - m.  P1: parity of the odd steps' l - m.
+template <int K, int G, bool P1, int J, int Q0, int Q1, int NS>
+__device__ __forceinline__ void syn_steps(SynState<K>& st, SynAcc<K> (&ac)[G], const double (&x)[K], double A,
+                                          const double (&r)[G][NS], const double (&i)[G][NS])
+{
+    for_each_map(std::make_integer_sequence<int, Q1 - Q0>{}, [&](auto qi) {
+        constexpr int q = Q0 + decltype(qi)::value, j = J + q;
+        constexpr bool qodd = (j & 1) == 0;       // step q = j + 1 of the item's 16
+        constexpr bool odd = qodd ? P1 : !P1;     // parity of l - m
+        constexpr bool minus = ((j + 1) & 2) != 0;  // s_q
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const double nu = fma(Al * st.x[k], st.mu1[k], -st.mu2[k]);
-        st.mu2[k] = st.mu1[k];
-        st.mu1[k] = nu;
+        for (int k = 0; k < K; ++k) {
+            double& n = qodd ? st.u[k] : st.w[k];
+            const double& p = qodd ? st.w[k] : st.u[k];
+            fmac_row<j, !qodd>(n, A, odd ? p : x[k] * p);
+        }
         for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
             constexpr int g = decltype(gi)::value;
-            if (ODD) {
-                ac[g].orr[k] = fma(nu, av[g].x, ac[g].orr[k]);
-                ac[g].oi[k] = fma(nu, av[g].y, ac[g].oi[k]);
-            } else {
-                ac[g].er[k] = fma(nu, av[g].x, ac[g].er[k]);
-                ac[g].ei[k] = fma(nu, av[g].y, ac[g].ei[k]);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const double nu = minus ? -(qodd ? st.u[k] : st.w[k]) : (qodd ? st.u[k] : st.w[k]);
+                if (odd) {
+                    ac[g].orr[k] = fma(nu, r[g][q], ac[g].orr[k]);
+                    ac[g].oi[k] = fma(nu, i[g][q], ac[g].oi[k]);
+                } else {
+                    ac[g].er[k] = fma(nu, r[g][q], ac[g].er[k]);
+                    ac[g].ei[k] = fma(nu, i[g][q], ac[g].ei[k]);
+                }
             }
         });
-    }
-}
-
-template <int K, int G, bool ODD>
-__device__ __forceinline__ void syng_stepj(LegState<K>& st, SynAcc<K> (&ac)[G], int j, const double* cA,
-                                           const double2 (*ca)[kSynChunk / 2 + kChunkPad])
-{
-    double2 av[G];
-    for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-        constexpr int g = decltype(gi)::value;
-        av[g] = ca[g][j];
     });
-    syng_step<K, G, ODD>(st, ac, cA[j], av);
 }
 
-// Rescale check: as syn_rescale, a joining lane clears every map's sums.
+// Rescale check after a row of eight steps while some lane is scaled: lanes
+// above 2^900 drop by 2^-1000; a lane whose count reaches 0 clears its sums.
+// Scaled lanes (count > 0) accumulate like live ones: their scaled mu
+// (|mu| < 2^958 between checks) makes meaningless sums, which are cleared when
+// the lane turns live and never stored while it is scaled, so the result
+// equals gating each term by the lane's state at the last check, without the
+// multiplies.  Eight steps multiply |mu| by at most prod (A_l + 1) < 2^45
+// (A_{m+1} = sqrt(2m + 2) is the largest factor), so from 2^900 nothing
+// overflows between checks; a lane whose scale count reaches 0 inside a row
+// joins at the row's end, dropping terms below 2^-42 of O(1) 2^-45.
 template <int K, int G>
-__device__ __forceinline__ void syng_rescale(LegState<K>& st, SynAcc<K> (&ac)[G])
+__device__ __forceinline__ void syn_rescale(SynState<K>& st, SynAcc<K> (&ac)[G])
 {
     int need = 0;
 #pragma unroll
-    for (int k = 0; k < K; ++k) need |= (st.sc[k] > 0) & (fabs(st.mu1[k]) > kScaleHi);
+    for (int k = 0; k < K; ++k) need |= (st.sc[k] > 0) & (fabs(st.w[k]) > kScaleHi);
     if (!__any(need)) return;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const bool r = st.sc[k] > 0 && fabs(st.mu1[k]) > kScaleHi;
-        st.mu1[k] = r ? st.mu1[k] * kScaleDn : st.mu1[k];
-        st.mu2[k] = r ? st.mu2[k] * kScaleDn : st.mu2[k];
+        const bool r = st.sc[k] > 0 && fabs(st.w[k]) > kScaleHi;
+        st.w[k] = r ? st.w[k] * kScaleDn : st.w[k];
+        st.u[k] = r ? st.u[k] * kScaleDn : st.u[k];
         st.sc[k] -= r ? 1 : 0;
         const bool join = r && st.sc[k] == 0;
         for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
@@ -874,492 +651,468 @@ __device__ __forceinline__ void syng_rescale(LegState<K>& st, SynAcc<K> (&ac)[G]
     st.all = all_live<K>(st.sc);
 }
 
-// One step of either parity, the parity by value (both parities' sums take an
-// fma, the other one's with zero coefficients: fma(nu, 0, s) = s for s != -0).
-template <int K, int G>
-__device__ __forceinline__ void syng_step_any(LegState<K>& st, SynAcc<K> (&ac)[G], bool odd, int j, const double* cA,
-                                              const double2 (*ca)[kSynChunk / 2 + kChunkPad])
+// Scalar loads of NS coefficients of the G maps.
+template <int G, int NS>
+__device__ __forceinline__ void syn_coef(scdouble* const (&a)[G], long o, double (&r)[G][NS], double (&i)[G][NS])
 {
-    const double Al = cA[j];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const double nu = fma(Al * st.x[k], st.mu1[k], -st.mu2[k]);
-        st.mu2[k] = st.mu1[k];
-        st.mu1[k] = nu;
-    }
-    for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-        constexpr int g = decltype(gi)::value;
-        const double2 a = ca[g][j];
-        const double er = odd ? 0.0 : a.x, ei = odd ? 0.0 : a.y, orr = odd ? a.x : 0.0, oi = odd ? a.y : 0.0;
+    for (int g = 0; g < G; ++g)
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            ac[g].er[k] = fma(st.mu1[k], er, ac[g].er[k]);
-            ac[g].ei[k] = fma(st.mu1[k], ei, ac[g].ei[k]);
-            ac[g].orr[k] = fma(st.mu1[k], orr, ac[g].orr[k]);
-            ac[g].oi[k] = fma(st.mu1[k], oi, ac[g].oi[k]);
+        for (int q = 0; q < NS; ++q) {
+            r[g][q] = a[g][2 * (o + q)];
+            i[g][q] = a[g][2 * (o + q) + 1];
         }
-    });
 }
 
-// Steps l..cend of one staged chunk.  Every run of steps starts at an even
-// l - m (an odd first step is taken on its own, parity by value), so all
-// paired steps are (even, odd) in one code path: two paths that differ only
-// in which parity's sums a step updates get merged by the compiler into a
-// choice of sums by address, which keeps them in scratch.  While some lane
-// is scaled: rows of eight steps with a rescale check after each, and pairs
-// with a check after each near the chunk's end (a lane joining inside a row
-// drops terms below 2^-55 of O(1), as in k_synth); then live pairs.
-template <int K, int G>
-__device__ __forceinline__ void syng_chunk(LegState<K>& st, SynAcc<K> (&ac)[G], int& l, int cend, int cb, int m,
-                                           const double* cA, const double2 (*ca)[kSynChunk / 2 + kChunkPad])
+// A group of NS steps on coefficients r, i; the next group's (nr, ni, at o of
+// the rows) are loaded after the first step, whose wait would otherwise cover
+// them: scalar loads return out of order, so any wait for one waits for all
+// (and nothing else in the loop, such as LDS, may share their counter).
+template <int K, int G, bool P1, int J, int NS>
+__device__ __forceinline__ void syn_group(SynState<K>& st, SynAcc<K> (&ac)[G], const double (&x)[K], double A,
+                                          const double (&r)[G][NS], const double (&i)[G][NS], scdouble* const (&a)[G],
+                                          long o, double (&nr)[G][NS], double (&ni)[G][NS])
 {
-    while (l <= cend) {
-        if ((l - m) & 1) {
-            syng_step_any<K, G>(st, ac, true, l - cb, cA, ca);
-            ++l;
-            if (!st.all) syng_rescale<K, G>(st, ac);
-            continue;
+    // x is for the group's first even step (q = 0 or 1)
+    syn_steps<K, G, P1, J, 0, 1, NS>(st, ac, x, A, r, i);
+    __builtin_amdgcn_sched_barrier(0);
+    syn_coef<G, NS>(a, o, nr, ni);
+    syn_steps<K, G, P1, J, 1, 2, NS>(st, ac, x, A, r, i);
+    syn_steps<K, G, P1, J, 2, NS, NS>(st, ac, st.y, A, r, i);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// 16 steps (two rows of eight) from step o of the rows; SCALED: a rescale
+// check after each row.  xa multiplies the first even step (Ring).
+template <int K, int G, bool P1, bool SCALED, int NS>
+__device__ __forceinline__ void syn_block(SynState<K>& st, SynAcc<K> (&ac)[G], const double (&xa)[K], double A,
+                                          scdouble* const (&a)[G], long o, double (&xr)[G][NS], double (&xi)[G][NS])
+{
+    double yr[G][NS], yi[G][NS];
+    if constexpr (NS == 8) {
+        syn_group<K, G, P1, 0, NS>(st, ac, xa, A, xr, xi, a, o + 8, yr, yi);
+        if (SCALED) syn_rescale<K, G>(st, ac);
+        syn_group<K, G, P1, 8, NS>(st, ac, st.y, A, yr, yi, a, o + 16, xr, xi);
+    } else {
+        syn_group<K, G, P1, 0, NS>(st, ac, xa, A, xr, xi, a, o + 4, yr, yi);
+        syn_group<K, G, P1, 4, NS>(st, ac, st.y, A, yr, yi, a, o + 8, xr, xi);
+        if (SCALED) syn_rescale<K, G>(st, ac);
+        syn_group<K, G, P1, 8, NS>(st, ac, st.y, A, xr, xi, a, o + 12, yr, yi);
+        syn_group<K, G, P1, 12, NS>(st, ac, st.y, A, yr, yi, a, o + 16, xr, xi);
+    }
+    if (SCALED) syn_rescale<K, G>(st, ac);
+}
+
+// Steps l0 + 1 .. L in blocks of 16 (the rows of a are zero past L and A is
+// loaded as zero there, so the last block needs no remainder): with rescale
+// checks until every lane is live, then without.  A of the next block is
+// loaded while a block runs.
+template <int K, int G, bool P1>
+__device__ __forceinline__ void syn_run(SynState<K>& st, SynAcc<K> (&ac)[G], gcdouble* __restrict__ A,
+                                        scdouble* const (&a)[G], int l0, int L, int lane)
+{
+    constexpr int NS = G == 1 ? 8 : 4, PER = kSynChunk / 16;
+    const int nblk = (L - l0 + 15) / 16;
+    int l = l0 + 1 + (lane & 15);
+    double A0 = l <= L ? A[l] : 0.0;
+    double xr[G][NS], xi[G][NS];
+    long o = l0 + 1;
+    syn_coef<G, NS>(a, o, xr, xi);
+    int b = 0;
+    for (; b < nblk && !st.all; ++b, o += 16) {
+        l += 16;
+        const double A1 = l <= L ? A[l] : 0.0;
+        double xa[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) xa[k] = b % PER == 0 ? st.yb[k] : st.ya[k];
+        syn_block<K, G, P1, true, NS>(st, ac, xa, A0, a, o, xr, xi);
+        A0 = A1;
+    }
+    while (b < nblk) {
+        if (b % PER == 0) {
+            l += 16;
+            const double A1 = l <= L ? A[l] : 0.0;
+            syn_block<K, G, P1, false, NS>(st, ac, st.yb, A0, a, o, xr, xi);
+            A0 = A1;
+            ++b;
+            o += 16;
         }
-        if (!st.all) {
-            const int n = (l + 7 <= cend) ? 8 : 2;
-#pragma unroll 1
-            for (int q = 0; q < n && l + 1 <= cend; q += 2, l += 2) {
-                syng_stepj<K, G, false>(st, ac, l - cb, cA, ca);
-                syng_stepj<K, G, true>(st, ac, l + 1 - cb, cA, ca);
-            }
-            if (l == cend && n == 2) {
-                syng_stepj<K, G, false>(st, ac, l - cb, cA, ca);
-                ++l;
-            }
-            syng_rescale<K, G>(st, ac);
-            continue;
-        }
-#pragma unroll 1
-        for (; l + 1 <= cend; l += 2) {
-            syng_stepj<K, G, false>(st, ac, l - cb, cA, ca);
-            syng_stepj<K, G, true>(st, ac, l + 1 - cb, cA, ca);
-        }
-        if (l <= cend) {
-            syng_stepj<K, G, false>(st, ac, l - cb, cA, ca);
-            ++l;
+        const int e = min(nblk, b / PER * PER + PER);
+        for (; b < e; ++b, o += 16) {
+            l += 16;
+            const double A1 = l <= L ? A[l] : 0.0;
+            syn_block<K, G, P1, false, NS>(st, ac, st.ya, A0, a, o, xr, xi);
+            A0 = A1;
         }
     }
 }
 
+// Legendre synthesis of G maps of one geometry (G > 1: the recurrence runs
+// once for them; item.map is then a row of gmaps).
 template <int K, int G>
-__global__ __launch_bounds__(64) void k_synth_g(const WorkItem* __restrict__ items, const MapDesc* __restrict__ maps,
-                                                const int* __restrict__ gmaps)
+__global__ __launch_bounds__(64) void k_synth(const WorkItem* __restrict__ items, const MapDesc* __restrict__ maps,
+                                              const int* __restrict__ gmaps)
 {
-    constexpr int CH = kSynChunk / 2;  // 64 steps: the G coefficient rows share the LDS budget
-    __shared__ double sA[2][CH + kChunkPad];
-    __shared__ double2 sa[2][G][CH + kChunkPad];
     const WorkItem it = items[blockIdx.x];
     if (it.mcnt == 0) return;
-    const int* gm = gmaps + (long)it.map * 4;  // group table rows of four entries
-    const MapDesc& md = maps[gm[0]];
+    const MapDesc* mds[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) mds[g] = maps + (G == 1 ? it.map : gmaps[G * it.map + g]);
+    const MapDesc& md = *mds[0];
     const int L = md.L;
-    const int npad = md.npair_pad;
     const int lane = threadIdx.x;
     const int m = it.m0;
     const int l0 = it.lfirst;
-    const long base = moff(L, m) - m;
-    gcdouble* __restrict__ A = (gcdouble*)(md.A + base);
-    gcdouble* a[G];
-    for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-        constexpr int g = decltype(gi)::value;
-        a[g] = (gcdouble*)(maps[gm[g]].alm + base);
-    });
+    gcdouble* __restrict__ A = (gcdouble*)(md.A + (moff(L, m) - m));
+    scdouble* a[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) a[g] = (scdouble*)(mds[g]->alm + (aoff(L, m) - m));
 
-    LegState<K> st;
+    SynState<K> st;
     SynAcc<K> ac[G];
     int p[K];
+    const bool odd0 = ((l0 - m) & 1) != 0;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         p[k] = it.rb * 64 * K + k * 64 + lane;
-        const long q = (long)m * npad + p[k];
-        st.x[k] = md.ring_x[p[k]];
-        st.mu1[k] = md.s1_cur[q];
-        st.mu2[k] = md.s1_prev[q];
+        const long q = (long)m * md.npair_pad + p[k];
+        const Ring c(md.ring_x[p[k]]);
+        st.y[k] = c.y;
+        st.ya[k] = c.ya;
+        st.yb[k] = c.yb;
+        st.w[k] = md.s1_cur[q];
+        st.u[k] = -md.s1_prev[q];
         st.sc[k] = md.s1_k[q];
-        for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-            constexpr int g = decltype(gi)::value;
-            ac[g].er[k] = ac[g].ei[k] = ac[g].orr[k] = ac[g].oi[k] = 0.0;
-        });
     }
     st.all = all_live<K>(st.sc);
-    // the item's first l, its parity by value (a branch here would be merged
-    // into a choice of accumulator by address, which keeps the sums in
-    // scratch); fma(mu, 0, +0) = +0 leaves the other parity's sums as they are
-    const bool odd0 = ((l0 - m) & 1) != 0;
-    for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-        constexpr int g = decltype(gi)::value;
-        const double ar = a[g][2 * l0], ai = a[g][2 * l0 + 1];
-        const double er = odd0 ? 0.0 : ar, ei = odd0 ? 0.0 : ai, orr = odd0 ? ar : 0.0, oi = odd0 ? ai : 0.0;
+    // the item's first l, its parity by value
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const double ar = a[g][2 * (long)l0], ai = a[g][2 * (long)l0 + 1];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            ac[g].er[k] = fma(st.mu1[k], er, ac[g].er[k]);
-            ac[g].ei[k] = fma(st.mu1[k], ei, ac[g].ei[k]);
-            ac[g].orr[k] = fma(st.mu1[k], orr, ac[g].orr[k]);
-            ac[g].oi[k] = fma(st.mu1[k], oi, ac[g].oi[k]);
+            ac[g].er[k] = odd0 ? 0.0 : st.w[k] * ar;
+            ac[g].ei[k] = odd0 ? 0.0 : st.w[k] * ai;
+            ac[g].orr[k] = odd0 ? st.w[k] * ar : 0.0;
+            ac[g].oi[k] = odd0 ? st.w[k] * ai : 0.0;
         }
-    });
-    int cb = l0 + 1;
-    double tA = 0.0;
-    double2 ta[G];
-    {
-        const int j = cb + lane;
-        tA = j <= L ? A[j] : 0.0;
-        for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-            constexpr int g = decltype(gi)::value;
-            ta[g] = j <= L ? make_double2(a[g][2 * j], a[g][2 * j + 1]) : make_double2(0.0, 0.0);
-            sa[0][g][lane] = ta[g];
-        });
-        sA[0][lane] = tA;
     }
-    wave_sync();
-    int buf = 0;
-    int l = cb;
-    while (cb <= L) {
-        const int nb = cb + CH;
-        const int j = nb + lane;
-        if (j <= L) {
-            tA = A[j];
-            for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-                constexpr int g = decltype(gi)::value;
-                ta[g] = make_double2(a[g][2 * j], a[g][2 * j + 1]);
-            });
-        }
-        syng_chunk<K, G>(st, ac, l, min(L, nb - 1), cb, m, sA[buf], sa[buf]);
-        if (nb <= L) {
-            sA[buf ^ 1][lane] = tA;
-            for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-                constexpr int g = decltype(gi)::value;
-                sa[buf ^ 1][g][lane] = ta[g];
-            });
-        }
-        wave_sync();
-        buf ^= 1;
-        cb = nb;
-    }
+    if (odd0)
+        syn_run<K, G, false>(st, ac, A, a, l0, L, lane);
+    else
+        syn_run<K, G, true>(st, ac, A, a, l0, L, lane);
     // lanes still scaled at L store zeros
-    for_each_map(std::make_integer_sequence<int, G>{}, [&](auto gi) {
-        constexpr int g = decltype(gi)::value;
-        const MapDesc& mg = maps[gm[g]];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             if (p[k] < md.npair) {
                 const bool z = st.sc[k] != 0;
-                double2* dst = reinterpret_cast<double2*>(mg.P + ((long)p[k] * (L + 1) + m) * 4);
+                const double x = md.ring_x[p[k]];
+                double2* dst = reinterpret_cast<double2*>(mds[g]->P + ((long)p[k] * (L + 1) + m) * 4);
                 dst[0] = make_double2(z ? 0.0 : ac[g].er[k], z ? 0.0 : ac[g].ei[k]);
-                dst[1] = make_double2(z ? 0.0 : ac[g].orr[k], z ? 0.0 : ac[g].oi[k]);
+                dst[1] = make_double2(z ? 0.0 : x * ac[g].orr[k], z ? 0.0 : x * ac[g].oi[k]);
             }
         }
-    });
 }
 
 // -------------------------------------------------------------- fused spin-2 synthesis
-// Accumulators of one ring pair, per slot (0: steps at even offsets from the
-// item's first l, 1: odd offsets), 18 doubles: T (re, im), then per field f
-// (E, B) at 2 + 8 f: Sa, Sb, Sc, D3.
-template <int K>
+//
+// One ring pair per lane: recurrence 1.5, T 2, field sums 12 and g 3 FP64
+// instructions per l, which bound it.  The 14 coefficients of a step are
+// wave-uniform; 16 steps of them sit in one row of 16 lanes, one step per lane,
+// loaded a block ahead, and feed the sums through the DPP operand (fmac_row).
+// Read from LDS instead they kept its read port busy longer than the multiplier
+// (8 KB per wave and step), and scalar loads, of which only one step fits the
+// scalar registers ahead, waited for memory.  nside 512 / lmax 1024, scalar
+// loads 620, two ring pairs per lane (half the waves) 399, this form 330 us;
+// with four sums per field (no g), two ring pairs and LDS 476 us.
+
+// Sums of a ring pair by parity of l - m (0: even), one per number of a
+// record: T (re, im), then S1, S2, S3 at 2, 6, 10, each E.re, E.im, B.re, B.im.
 struct PolAcc {
-    double v[2][K][18];
+    double v[2][kPolRec];
 };
 
-template <int K, int SLOT>
-__device__ __forceinline__ void pol_accum(PolAcc<K>& ac, int k, double nu, double fl, double fl2,
-                                          const double2 (&c)[kPolRec])
-{
-    double* a = ac.v[SLOT][k];
-    a[0] = fma(nu, c[0].x, a[0]);
-    a[1] = fma(nu, c[0].y, a[1]);
+// The coefficients of 16 l-steps, one step per lane of a row of 16: A, the
+// records, l - m^2 and l (l - 1) / 2.
+struct PolRow {
+    double A, c[kPolRec], e, h;
+    __device__ __forceinline__ void load(gcdouble* Am, gcdouble* R, int l, int L)
+    {
+        A = l <= L ? Am[l] : 0.0;
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
-        double* q = a + 2 + 8 * f;
-        const double ur = nu * c[1 + 2 * f].x, ui = nu * c[1 + 2 * f].y;
-        q[0] += ur;
-        q[1] += ui;
-        q[2] = fma(fl, ur, q[2]);
-        q[3] = fma(fl, ui, q[3]);
-        q[4] = fma(fl2, ur, q[4]);
-        q[5] = fma(fl2, ui, q[5]);
-        q[6] = fma(nu, c[2 + 2 * f].x, q[6]);
-        q[7] = fma(nu, c[2 + 2 * f].y, q[7]);
+        for (int i = 0; i < kPolRec; ++i) c[i] = R[(long)l * kPolRec + i];
+    }
+    // two wait states between these VALU writes and the first DPP read
+    __device__ __forceinline__ void ready(int l, double m2)
+    {
+        const double fl = l;
+        e = fl - m2;
+        h = 0.5 * (fl * (fl - 1.0));
+        asm volatile("s_nop 1" : "+v"(A), "+v"(e), "+v"(h));
+    }
+};
+
+// c of lane N of the lane's row of 16.
+template <int N>
+__device__ __forceinline__ double mov_row(double c)
+{
+    double r;
+    asm("v_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(c), "n"(N));
+    return r;
+}
+
+// Step J + 1 of a block of 16 as in syn_steps (the recurrence and the T sums
+// are those of k_synth, operation by operation).
+template <bool P1, int J>
+__device__ __forceinline__ void pol_step(SynState<1>& st, PolAcc& ac, double x, double is2, const PolRow& r)
+{
+    constexpr bool qodd = (J & 1) == 0, odd = qodd ? P1 : !P1, minus = ((J + 1) & 2) != 0;
+    double& v = qodd ? st.u[0] : st.w[0];
+    const double& p = qodd ? st.w[0] : st.u[0];
+    fmac_row<J, !qodd>(v, r.A, odd ? p : x * p);
+    double(&a)[kPolRec] = ac.v[odd];
+    fmac_row<J, minus>(a[0], r.c[0], v);
+    fmac_row<J, minus>(a[1], r.c[1], v);
+    double g = mov_row<J>(r.h);  // -g
+    fmac_row<J, false>(g, r.e, is2);
+    g *= v;
+#pragma unroll
+    for (int i = 2; i < kPolRec; ++i) fmac_row<J, minus>(a[i], r.c[i], i < 6 ? g : v);
+}
+
+// syn_rescale for the spin-2 sums.
+__device__ __forceinline__ void pol_rescale(SynState<1>& st, PolAcc& ac)
+{
+    const bool r = st.sc[0] > 0 && fabs(st.w[0]) > kScaleHi;
+    if (!__any(r)) return;
+    st.w[0] = r ? st.w[0] * kScaleDn : st.w[0];
+    st.u[0] = r ? st.u[0] * kScaleDn : st.u[0];
+    st.sc[0] -= r ? 1 : 0;
+    const bool join = r && st.sc[0] == 0;
+#pragma unroll
+    for (int i = 0; i < kPolRec; ++i) {
+        ac.v[0][i] = join ? 0.0 : ac.v[0][i];
+        ac.v[1][i] = join ? 0.0 : ac.v[1][i];
+    }
+    st.all = all_live<1>(st.sc);
+}
+
+// A block of 16 steps; xa multiplies the first even step (Ring).
+template <bool P1, bool SCALED>
+__device__ __forceinline__ void pol_block(SynState<1>& st, PolAcc& ac, double xa, double is2, const PolRow& r)
+{
+    for_each_map(std::make_integer_sequence<int, 16>{}, [&](auto ji) {
+        constexpr int j = decltype(ji)::value;
+        pol_step<P1, j>(st, ac, j < 2 ? xa : st.y[0], is2, r);
+        if (SCALED && (j & 7) == 7) pol_rescale(st, ac);
+    });
+}
+
+// syn_run for the spin-2 sums: the same blocks, x^2 corrections and checks.
+template <bool P1>
+__device__ __forceinline__ void pol_run(SynState<1>& st, PolAcc& ac, gcdouble* __restrict__ A,
+                                        gcdouble* __restrict__ R, double is2, double m2, int l0, int L, int lane)
+{
+    constexpr int PER = kSynChunk / 16;
+    const int nblk = (L - l0 + 15) / 16;
+    int l = l0 + 1 + (lane & 15);
+    PolRow r0, r1;
+    r0.load(A, R, min(l, L + 16), L);
+    int b = 0;
+    auto run = [&](auto scaled, PolRow& r, PolRow& n) {
+        r.ready(l, m2);
+        l += 16;
+        n.load(A, R, min(l, L + 16), L);
+        pol_block<P1, decltype(scaled)::value>(st, ac, b % PER == 0 ? st.yb[0] : st.ya[0], is2, r);
+        ++b;
+    };
+    while (b < nblk && !st.all) {
+        run(std::true_type{}, r0, r1);
+        r0 = r1;
+    }
+    // two blocks at a time: their rows change places without copies
+    while (b < nblk) {
+        run(std::false_type{}, r0, r1);
+        if (b >= nblk) break;
+        run(std::false_type{}, r1, r0);
     }
 }
 
-template <int K, int SLOT>
-__device__ __forceinline__ void pol_live(LegState<K>& st, PolAcc<K>& ac, double Al, int l,
-                                         const double2 (&c)[kPolRec])
-{
-    const double fl = l, fl2 = fl * fl;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const double nu = fma(Al * st.x[k], st.mu1[k], -st.mu2[k]);
-        st.mu2[k] = st.mu1[k];
-        st.mu1[k] = nu;
-        pol_accum<K, SLOT>(ac, k, nu, fl, fl2, c);
-    }
-}
-
-// Gated step: negligible lanes contribute gate 0 (no branch, so the
-// accumulators stay in place across steps).
-template <int K, int SLOT>
-__device__ __forceinline__ void pol_gated(const LegState<K>& st, PolAcc<K>& ac, int l, const double2 (&c)[kPolRec])
-{
-    const double fl = l, fl2 = fl * fl;
-#pragma unroll
-    for (int k = 0; k < K; ++k) pol_accum<K, SLOT>(ac, k, st.gate[k] * st.mu1[k], fl, fl2, c);
-}
-
-template <int K>
-__device__ __forceinline__ void pol_load(const double2 (*cr)[kPolRec], int j, double2 (&c)[kPolRec])
-{
-#pragma unroll
-    for (int i = 0; i < kPolRec; ++i) c[i] = cr[j][i];
-}
-
-// Steps l .. cend of one staged chunk in pairs: the accumulators are indexed
-// by the step's position relative to the item's first l (slot 0 for even
-// offsets), so no parity decision sits between accumulator updates.  Chunks
-// start at odd offsets and hold an even number of steps except the last,
-// whose extra step reads the zero coefficients staged beyond lmax.  Scaled
-// pairs carry a rescale check each, then live pairs.
-template <int K>
-__device__ __forceinline__ void pol_chunk(LegState<K>& st, PolAcc<K>& ac, int& l, int cend, int cb,
-                                          const double* cA, const double2 (*cr)[kPolRec])
-{
-    double2 c[kPolRec];
-    while (!st.all && l <= cend) {
-        pol_load<K>(cr, l - cb, c);
-        st.advance(cA[l - cb]);
-        pol_gated<K, 1>(st, ac, l, c);
-        pol_load<K>(cr, l + 1 - cb, c);
-        st.advance(cA[l + 1 - cb]);
-        pol_gated<K, 0>(st, ac, l + 1, c);
-        l += 2;
-        if (rescale<K>(st.mu1, st.mu2, st.sc)) st.refresh();
-    }
-    for (; l <= cend; l += 2) {
-        pol_load<K>(cr, l - cb, c);
-        pol_live<K, 1>(st, ac, cA[l - cb], l, c);
-        pol_load<K>(cr, l + 1 - cb, c);
-        pol_live<K, 0>(st, ac, cA[l + 1 - cb], l + 1, c);
-    }
-}
-
-// One (m, ring block) item of the synthesis work list: T, Q, U parity sums of
-// its ring pairs into pt, pq, pu ([pair][m] (E.re, E.im, O.re, O.im), the
-// form the ring stage reads; Q and U as ((north + south)/2, (north - south)/2)).
-template <int K>
+// One block of 64 ring pairs (blockIdx.y) of a (m, ring block) item of the
+// synthesis work list, from the item's first l: T, Q, U parity sums of its
+// ring pairs into pt, pq, pu ([pair][m] (E.re, E.im, O.re, O.im), the form the
+// ring stage reads; Q and U as ((north + south)/2, (north - south)/2)).
 __global__ __launch_bounds__(64) void k_synth_pol(const WorkItem* __restrict__ items, const MapDesc* __restrict__ maps,
                                                   const double2* __restrict__ rec, double* __restrict__ pt,
                                                   double* __restrict__ pq, double* __restrict__ pu)
 {
-    __shared__ double sA[2][kChunk + kChunkPad];
-    __shared__ double2 sr[2][kChunk + kChunkPad][kPolRec];
     const WorkItem it = items[blockIdx.x];
     if (it.mcnt == 0) return;
     const MapDesc& md = maps[it.map];
     const int L = md.L;
-    const int npad = md.npair_pad;
     const int lane = threadIdx.x;
     const int m = it.m0;
     const int l0 = it.lfirst;
-    const long base = moff(L, m) - m;
-    gcdouble* __restrict__ A = (gcdouble*)(md.A + base);
-    gcdouble* __restrict__ R = (gcdouble*)(rec + base * kPolRec);  // 2 kPolRec doubles per l
+    gcdouble* __restrict__ A = (gcdouble*)(md.A + (moff(L, m) - m));
+    gcdouble* __restrict__ R = (gcdouble*)(rec + (aoff(L, m) - m) * (kPolRec / 2));
 
-    LegState<K> st;
-    PolAcc<K> ac;
-    int p[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        p[k] = it.rb * 64 * K + k * 64 + lane;
-        const long q = (long)m * npad + p[k];
-        st.x[k] = md.ring_x[p[k]];
-        st.mu1[k] = md.s1_cur[q];
-        st.mu2[k] = md.s1_prev[q];
-        st.sc[k] = md.s1_k[q];
-#pragma unroll
-        for (int i = 0; i < 18; ++i) ac.v[0][k][i] = ac.v[1][k][i] = 0.0;
-    }
-    st.refresh();
+    const int p = (it.rb * (int)gridDim.y + (int)blockIdx.y) * 64 + lane;
+    const long q = (long)m * md.npair_pad + p;
+    const double x = md.ring_x[p], is2 = 1.0 / md.ring_s2[p];
+    const bool odd0 = ((l0 - m) & 1) != 0;
+    SynState<1> st;
+    PolAcc ac;
+    const Ring c(x);
+    st.y[0] = c.y;
+    st.ya[0] = c.ya;
+    st.yb[0] = c.yb;
+    st.w[0] = md.s1_cur[q];
+    st.u[0] = -md.s1_prev[q];
+    st.sc[0] = md.s1_k[q];
+    st.all = all_live<1>(st.sc);
+    const double m2 = (double)m * m;
+    // the item's first l, its parity by value
     {
-        double2 c[kPolRec];
+        const double fl = l0, h = 0.5 * (fl * (fl - 1.0));
+        const double g = st.w[0] * fma(fl - m2, is2, h);
 #pragma unroll
-        for (int i = 0; i < kPolRec; ++i)
-            c[i] = make_double2(R[(long)l0 * 2 * kPolRec + 2 * i], R[(long)l0 * 2 * kPolRec + 2 * i + 1]);
-        pol_gated<K, 0>(st, ac, l0, c);
-    }
-    // staged chunks of steps l0+1 .. L
-    int cb = l0 + 1;
-    double tA = 0.0;
-    double2 tc[kPolRec];
-#pragma unroll
-    for (int i = 0; i < kPolRec; ++i) tc[i] = make_double2(0.0, 0.0);
-    if (cb + lane <= L) {
-        tA = A[cb + lane];
-#pragma unroll
-        for (int i = 0; i < kPolRec; ++i)
-            tc[i] = make_double2(R[(long)(cb + lane) * 2 * kPolRec + 2 * i], R[(long)(cb + lane) * 2 * kPolRec + 2 * i + 1]);
-    }
-    sA[0][lane] = tA;
-#pragma unroll
-    for (int i = 0; i < kPolRec; ++i) sr[0][lane][i] = tc[i];
-    wave_sync();
-    int buf = 0;
-    int l = cb;
-    while (cb <= L) {
-        const int nb = cb + kChunk;
-        // entries beyond lmax stage zeros: the last chunk's extra step reads one
-        tA = 0.0;
-#pragma unroll
-        for (int i = 0; i < kPolRec; ++i) tc[i] = make_double2(0.0, 0.0);
-        if (nb + lane <= L) {
-            tA = A[nb + lane];
-#pragma unroll
-            for (int i = 0; i < kPolRec; ++i)
-                tc[i] = make_double2(R[(long)(nb + lane) * 2 * kPolRec + 2 * i],
-                                     R[(long)(nb + lane) * 2 * kPolRec + 2 * i + 1]);
+        for (int i = 0; i < kPolRec; ++i) {
+            const double t = (i >= 2 && i < 6 ? g : st.w[0]) * R[(long)l0 * kPolRec + i];
+            ac.v[0][i] = odd0 ? 0.0 : t;
+            ac.v[1][i] = odd0 ? t : 0.0;
         }
-        pol_chunk<K>(st, ac, l, min(L, nb - 1), cb, sA[buf], sr[buf]);
-        if (nb <= L) {
-            sA[buf ^ 1][lane] = tA;
-#pragma unroll
-            for (int i = 0; i < kPolRec; ++i) sr[buf ^ 1][lane][i] = tc[i];
-        }
-        wave_sync();
-        buf ^= 1;
-        cb = nb;
     }
-    // epilogue: per ring pair, north (E + O at c) and south (E - O at -c)
-    const double fm = m, fm2 = fm * fm;
+    if (odd0)
+        pol_run<false>(st, ac, A, R, is2, m2, l0, L, lane);
+    else
+        pol_run<true>(st, ac, A, R, is2, m2, l0, L, lane);
+    // epilogue: north (E + O at c) and south (E - O at -c); lanes still scaled
+    // at L store zeros
+    if (p >= md.npair) return;
+    const double fm = m;
+    const long o = ((long)p * (L + 1) + m) * 4;
+    const bool z = st.sc[0] != 0;
+    double e[kPolRec], d[kPolRec];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        if (p[k] >= md.npair) continue;
-        const long o = ((long)p[k] * (L + 1) + m) * 4;
-        const bool swap = ((l0 - m) & 1) != 0;  // slot 0 holds the parity of l0 - m
-        double e[18], d[18];
+    for (int i = 0; i < kPolRec; ++i) {
+        e[i] = z ? 0.0 : ac.v[0][i];
+        d[i] = z ? 0.0 : x * ac.v[1][i];
+    }
+    *reinterpret_cast<double4*>(pt + o) = make_double4(e[0], e[1], d[0], d[1]);
+    double W[2][2][2], X[2][2][2];  // [field][north/south][re/im]
 #pragma unroll
-        for (int i = 0; i < 18; ++i) {
-            e[i] = swap ? ac.v[1][k][i] : ac.v[0][k][i];
-            d[i] = swap ? ac.v[0][k][i] : ac.v[1][k][i];
-        }
-        *reinterpret_cast<double4*>(pt + o) = make_double4(e[0], e[1], d[0], d[1]);
-        const double c = st.x[k], is2 = 1.0 / md.ring_s2[p[k]];
-        double W[2][2][2], X[2][2][2];  // [field][north/south][re/im]
+    for (int f = 0; f < 2; ++f) {
 #pragma unroll
-        for (int f = 0; f < 2; ++f) {
+        for (int s = 0; s < 2; ++s) {
+            const double sg = s ? -1.0 : 1.0;  // south: E - O, c -> -c
+            const double ch = sg * x;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const double sg = h ? -1.0 : 1.0;  // south: E - O, c -> -c
-                const double ch = sg * c;
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    const int b = 2 + 8 * f + r;
-                    const double Sa = e[b] + sg * d[b], Sb = e[b + 2] + sg * d[b + 2];
-                    const double Sc = e[b + 4] + sg * d[b + 4], D3 = e[b + 6] + sg * d[b + 6];
-                    const double D1 = Sb - fm2 * Sa, D2 = 0.5 * (Sc - Sb), D4 = Sb - Sa;
-                    W[f][h][r] = -is2 * D1 - D2 + ch * is2 * D3;
-                    X[f][h][r] = fm * is2 * (D3 - ch * D4);
-                }
+            for (int r = 0; r < 2; ++r) {
+                const int b = 2 + 2 * f + r;
+                const double S1 = e[b] + sg * d[b], S2 = e[b + 4] + sg * d[b + 4];  // S1: its negative
+                const double S3 = e[b + 8] + sg * d[b + 8];
+                W[f][s][r] = ch * is2 * S2 - S1;
+                X[f][s][r] = fm * is2 * (S2 - ch * S3);
             }
         }
-        // Q = -(W_E + i X_B), U = -(W_B - i X_E)
-        double Q[2][2], U[2][2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            Q[h][0] = -(W[0][h][0] - X[1][h][1]);
-            Q[h][1] = -(W[0][h][1] + X[1][h][0]);
-            U[h][0] = -(W[1][h][0] + X[0][h][1]);
-            U[h][1] = -(W[1][h][1] - X[0][h][0]);
-        }
-        *reinterpret_cast<double4*>(pq + o) = make_double4(0.5 * (Q[0][0] + Q[1][0]), 0.5 * (Q[0][1] + Q[1][1]),
-                                                           0.5 * (Q[0][0] - Q[1][0]), 0.5 * (Q[0][1] - Q[1][1]));
-        *reinterpret_cast<double4*>(pu + o) = make_double4(0.5 * (U[0][0] + U[1][0]), 0.5 * (U[0][1] + U[1][1]),
-                                                           0.5 * (U[0][0] - U[1][0]), 0.5 * (U[0][1] - U[1][1]));
     }
+    // Q = -(W_E + i X_B), U = -(W_B - i X_E)
+    double Q[2][2], U[2][2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        Q[s][0] = -(W[0][s][0] - X[1][s][1]);
+        Q[s][1] = -(W[0][s][1] + X[1][s][0]);
+        U[s][0] = -(W[1][s][0] + X[0][s][1]);
+        U[s][1] = -(W[1][s][1] - X[0][s][0]);
+    }
+    *reinterpret_cast<double4*>(pq + o) = make_double4(0.5 * (Q[0][0] + Q[1][0]), 0.5 * (Q[0][1] + Q[1][1]),
+                                                       0.5 * (Q[0][0] - Q[1][0]), 0.5 * (Q[0][1] - Q[1][1]));
+    *reinterpret_cast<double4*>(pu + o) = make_double4(0.5 * (U[0][0] + U[1][0]), 0.5 * (U[0][1] + U[1][1]),
+                                                       0.5 * (U[0][0] - U[1][0]), 0.5 * (U[0][1] - U[1][1]));
 }
 
 // -------------------------------------------------------------- adjoint
-// Per l-step each lane forms sum_k mu_l(p_k) Psi^{parity}(p_k); every
-// kRedChunk steps the wave reduces the 64 lanes (register folds and an LDS
-// tile) and writes the ring-block partial u_lm (re, im) with one coalesced
-// store.  Steps outside whole rows (the item's last partial row) go through a
-// per-lane LDS buffer reduced when it holds kRedChunk steps or at the end.
+// u_lm = sum over ring pairs of lambda_lm Psi_m.  One wavefront takes one
+// degree m of a block of 64 K ring pairs, lane j holding the pairs 64 k + j,
+// and walks l in rows of eight steps; each lane adds its K products per step
+// and the row's 16 sums (8 steps, real and imaginary) are then reduced over
+// the 64 lanes and stored as the block's partial u.
+//
+// What bounds it: FP64 VALU issue, 3.5 instructions per (l, ring pair) plus
+// about 60 issue slots per row for the reduction, whatever K: K = 8 halves
+// the reduction's share against K = 4 (28 K against 60 slots per row).  Its
+// 512-pair blocks would start all their pairs at the earliest live l of the
+// block; instead each group k of 64 pairs joins at the row of its own first
+// live l (AdjItem::row), so the skipped range is that of 64-pair blocks.  The
+// registers of K = 8 (about 200) allow two waves per SIMD, enough here: eight
+// independent chains per wave.  The recurrence coefficients are wave-uniform
+// and come through the scalar cache a row ahead; LDS carries the reduction
+// tile and the ring constants.
 
-// A lane's ring-stage inputs Psi_m (even and odd parts) of its K ring pairs.
-// Lanes whose scale count is > 0 hold zeros, so that the same four-operation
-// step serves the scaled and the live path: their scaled mu (|mu| < 2^945
-// between rescale checks) times 0 contributes exactly 0.  A lane that turns
-// live loads its inputs at the rescale check where its count reaches 0.
+// A lane's ring-stage inputs Psi_m (even and odd parts, the odd one times x)
+// of its K ring pairs.  Lanes whose scale count is > 0 hold
+// zeros, so that the same step serves the scaled and the live path: their
+// scaled mu (|mu| < 2^958 between rescale checks) times 0 contributes exactly
+// 0.  A lane that turns live loads its inputs at the rescale check where its
+// count reaches 0.
 template <int K>
-struct AdjIn {
+struct AdjState {
+    double y[K];           // x^2
+    double mu1[K], mu2[K]; // mu_{l-1}, mu_{l-2} before step l, odd ones divided by x
     double per[K], pei[K], por[K], poi[K];
-};
-
-// Where the inputs of lane `lane`'s ring pair pbase + 64 k + lane live:
-// Q + p * row + 4 m (row = 4 (L + 1) doubles per ring pair); pairs past npair
-// (padding) have none.
-struct AdjSrc {
-    const double* Q;
-    long row;
-    int m, pbase, npair, lane;
+    int sc[K];
 };
 
 template <int K>
-__device__ __forceinline__ void adj_load_in(AdjIn<K>& in, int k, const AdjSrc& s)
+__device__ __forceinline__ void adj_load_in(AdjState<K>& st, int k, const AdjItem& it, int lane)
 {
-    const int p = s.pbase + k * 64 + s.lane;
+    const int p = it.p0 + k * 64 + lane;
     double v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
-    if (p < s.npair) {
-        gcdouble* src = (gcdouble*)(s.Q + (long)p * s.row + 4 * (long)s.m);
+    if (p < it.npair) {
+        gcdouble* src = gview(it.Q) + (long)p * 4 * (it.L + 1);
+        const double x = gview(it.x)[p];
         v0 = src[0];
         v1 = src[1];
-        v2 = src[2];
-        v3 = src[3];
+        v2 = x * src[2];
+        v3 = x * src[3];
     }
     // one unconditional store per field: stores in both arms of a branch
     // would be merged through a pointer and keep the inputs in memory
-    in.per[k] = v0;
-    in.pei[k] = v1;
-    in.por[k] = v2;
-    in.poi[k] = v3;
+    st.per[k] = v0;
+    st.pei[k] = v1;
+    st.por[k] = v2;
+    st.poi[k] = v3;
 }
 
-// Rescale check of the adjoint's scaled path: lanes above 2^900 drop by
-// 2^-1000; a lane whose count reaches 0 loads its inputs.
-template <int K>
-__device__ __forceinline__ void adj_rescale(LegState<K>& st, AdjIn<K>& in, const AdjSrc& s)
+// Rescale check of the groups k >= K - KA: lanes above 2^900 drop by 2^-1000;
+// a lane whose count reaches 0 loads its inputs.  Returns whether all are live.
+// (Checking only the groups that still hold scaled lanes, by a branch each,
+// made the register allocator copy the state at every merge: 40 more VGPRs at
+// K = 8, spills, 115 against 105 us at nside 512.)
+template <int K, int KA>
+__device__ __forceinline__ bool adj_rescale(AdjState<K>& st, const AdjItem& it, int lane)
 {
     int need = 0;
 #pragma unroll
-    for (int k = 0; k < K; ++k) need |= (st.sc[k] > 0) & (fabs(st.mu1[k]) > kScaleHi);
-    if (!__any(need)) return;
+    for (int k = K - KA; k < K; ++k) need |= (st.sc[k] > 0) & (fabs(st.mu1[k]) > kScaleHi);
+    if (__any(need)) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        if (st.sc[k] > 0 && fabs(st.mu1[k]) > kScaleHi) {
-            st.mu1[k] *= kScaleDn;
-            st.mu2[k] *= kScaleDn;
-            st.sc[k] -= 1;
-            if (st.sc[k] == 0) adj_load_in<K>(in, k, s);
+        for (int k = K - KA; k < K; ++k) {
+            if (st.sc[k] > 0 && fabs(st.mu1[k]) > kScaleHi) {
+                st.mu1[k] *= kScaleDn;
+                st.mu2[k] *= kScaleDn;
+                st.sc[k] -= 1;
+                if (st.sc[k] == 0) adj_load_in<K>(st, k, it, lane);
+            }
         }
     }
-    st.all = all_live<K>(st.sc);
+    int ok = 1;
+#pragma unroll
+    for (int k = K - KA; k < K; ++k) ok &= (st.sc[k] == 0);
+    return __all(ok);
 }
-
-// Psi (re, im) of parity o of ring pair k.  All four inputs are read and the
-// values selected: selecting array elements, or merging the even and odd
-// variants of a step, would keep the inputs in addressable memory.
-template <int K>
-__device__ __forceinline__ void adj_psi(const AdjIn<K>& in, int k, bool o, double& pr, double& pi)
-{
-    const double er = in.per[k], ei = in.pei[k], orr = in.por[k], oi = in.poi[k];
-    pr = o ? orr : er;
-    pi = o ? oi : ei;
-}
-
 
 // Lanes 0..31 get a summed over lanes (j, j + 32), lanes 32..63 get b summed
 // likewise (v_permlane32_swap exchanges lanes 32..63 of its first operand
@@ -1395,389 +1148,214 @@ __device__ __forceinline__ double ror_add(double s)
     return s + __hiloint2double(hi, lo);
 }
 
-// the row tile (records 33 q + u, q < 8, u < 32) fits in the lane rows
-static_assert(2 * (33 * 7 + 32) <= 64 * kRedStride, "row tile exceeds the reduction buffer");
+// Rows of eight steps.  Steps 2p and 2p + 1 are folded as soon as both exist,
+// once over lane pairs (j, j + 32) with permlane32 swaps (fold_pair): z[2p + c]
+// then holds step 2p in lanes 0..31 and step 2p + 1 in lanes 32..63 (c = 0
+// real, 1 imaginary).  tile_store puts lane L's four (re, im) records as
+// records (q, L & 31), q = 2p + (L >> 5), at index 33 q + (L & 31); tile_load
+// gives lane j the records (j & 7, 4 (j >> 3) + r), r < 4 (the skew of one
+// record per q puts the eight lanes of a read on distinct banks); finish_row
+// sums them and completes the sum over the eight lanes that share j & 7
+// (distances 32, 16, 8): the real part ends in lanes 0..31, the imaginary part
+// in lanes 32..63.  A permlane swap costs about 1.2 to 1.6 FP64 issue slots, so
+// the tile carries the second fold: 20 swaps per row instead of 28, for 4 KB of
+// LDS traffic each way.
+constexpr int kAdjTile = 33 * 7 + 32;  // records of the row tile
 
 struct AdjRed {
-    double* red;   // [64 * kRedStride]
-    double* mine;  // this lane's row
-    double* dst;   // output row, dst[2l], dst[2l+1] (global memory)
-    int cnt, lbase, lane;
-    __device__ __forceinline__ void flush()
-    {
-        wave_sync();
-        const int c = lane & 15;
-        const int q = lane >> 4;
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s += red[(16 * q + i) * kRedStride + c];
-        s += __shfl_xor(s, 16);
-        s += __shfl_xor(s, 32);
-        if (lane < 2 * cnt) ((gdouble*)dst)[2 * lbase + lane] = s;
-        wave_sync();
-        lbase += cnt;
-        cnt = 0;
-    }
-    __device__ __forceinline__ void push(double sr, double si)
-    {
-        mine[2 * cnt] = sr;
-        mine[2 * cnt + 1] = si;
-        if (++cnt == kRedChunk) flush();
-    }
-    // Rows of kRedChunk = 8 steps.  Steps 2p and 2p + 1 are folded as soon as
-    // both exist, once over lane pairs (j, j + 32) with permlane32 swaps
-    // (fold_pair): z[2p + c] then holds step 2p in lanes 0..31 and step 2p + 1
-    // in lanes 32..63 (c = 0 real, 1 imaginary).  tile_store puts lane L's four
-    // (re, im) records as records (q, L & 31), q = 2p + (L >> 5), at index
-    // 33 q + (L & 31); tile_load gives lane j the records (j & 7, 4 (j >> 3)
-    // + r), r < 4 (the skew of one record per q puts the eight lanes of a read
-    // on distinct banks); finish_row sums them and completes the sum over the
-    // eight lanes that share j & 7 (distances 32, 16, 8): the real part ends in
-    // lanes 0..31, the imaginary part in lanes 32..63.  A permlane swap costs
-    // about two FP64 issue slots, so the tile carries the second fold: 20 swaps
-    // per row instead of 28, for 4 KB of LDS traffic each way.
-    __device__ __forceinline__ static void fold_pair(double are, double aim, double bre, double bim, double& z0,
-                                                     double& z1)
-    {
-        z0 = swap32_add(are, bre);
-        z1 = swap32_add(aim, bim);
-    }
+    double2* tile;
+    gdouble* dst;  // output row, dst[2 l], dst[2 l + 1]
+    int l, lend, lane;
     __device__ __forceinline__ void tile_store(const double (&z)[8])
     {
-        double2* t = reinterpret_cast<double2*>(red) + 33 * (lane >> 5) + (lane & 31);
+        double2* t = tile + 33 * (lane >> 5) + (lane & 31);
 #pragma unroll
         for (int p = 0; p < 4; ++p) t[66 * p] = make_double2(z[2 * p], z[2 * p + 1]);
         wave_sync();
     }
     __device__ __forceinline__ void tile_load(double2 (&t4)[4]) const
     {
-        const double2* t = reinterpret_cast<const double2*>(red) + 33 * (lane & 7) + 4 * (lane >> 3);
+        const double2* t = tile + 33 * (lane & 7) + 4 * (lane >> 3);
 #pragma unroll
         for (int r = 0; r < 4; ++r) t4[r] = t[r];
     }
     __device__ __forceinline__ void finish_row(const double2 (&t4)[4])
     {
-        double re = (t4[0].x + t4[1].x) + (t4[2].x + t4[3].x);
-        double im = (t4[0].y + t4[1].y) + (t4[2].y + t4[3].y);
+        const double re = (t4[0].x + t4[1].x) + (t4[2].x + t4[3].x);
+        const double im = (t4[0].y + t4[1].y) + (t4[2].y + t4[3].y);
         double s = swap32_add(re, im);
         s = swap16_add(s, s);
         s = ror_add<8>(s);
-        // four lanes hold each value and store it (no branch, so the store
-        // stays in the loop's block)
-        gdouble* g = (gdouble*)dst;
-        g[2 * lbase + 2 * (lane & 7) + (lane >> 5)] = s;
-        lbase += kRedChunk;
-    }
-    // One l on its own (the item's first): the whole-wave sum of (sr, si),
-    // the real part in lanes 0..31 and the imaginary part in lanes 32..63, all
-    // in registers, stored at lbase.  Keeping it out of the push buffer lets
-    // the staged chunks (64 steps from the next l) fall on row boundaries.
-    __device__ __forceinline__ void store_one(double sr, double si)
-    {
-        double s = swap32_add(sr, si);
-        s = swap16_add(s, s);
-        s = ror_add<8>(s);
-        s = ror_add<4>(s);
-        s = ror_add<2>(s);
-        s = ror_add<1>(s);
-        gdouble* g = (gdouble*)dst;
-        g[2 * lbase + (lane >> 5)] = s;
-        lbase += 1;
+        // four lanes hold each value and store it
+        const int lr = l + (lane & 7);
+        if (lr <= lend) dst[2 * (long)lr + (lane >> 5)] = s;
+        l += 8;
     }
 };
 
-template <int K, bool ODD>
-__device__ __forceinline__ void adj_live(LegState<K>& st, const AdjIn<K>& in, AdjRed& rd, double Al)
-{
-    double sr = 0.0, si = 0.0;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const double nu = fma(Al * st.x[k], st.mu1[k], -st.mu2[k]);
-        st.mu2[k] = st.mu1[k];
-        st.mu1[k] = nu;
-        double pr, pi;
-        adj_psi<K>(in, k, ODD, pr, pi);
-        sr = fma(nu, pr, sr);
-        si = fma(nu, pi, si);
-    }
-    rd.push(sr, si);
-}
-
-// The item's first l (the recurrence state is already at it).
-template <int K, bool ODD>
-__device__ __forceinline__ void adj_first(const LegState<K>& st, const AdjIn<K>& in, AdjRed& rd)
-{
-    double sr = 0.0, si = 0.0;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        double pr, pi;
-        adj_psi<K>(in, k, ODD, pr, pi);
-        sr = fma(st.mu1[k], pr, sr);
-        si = fma(st.mu1[k], pi, si);
-    }
-    rd.store_one(sr, si);
-}
-
-// One live step returning its (real, imaginary) lane sums; o = parity of l - m.
-template <int K>
-__device__ __forceinline__ void adj_step_v(LegState<K>& st, const AdjIn<K>& in, bool o, double Al, double& sr,
-                                           double& si)
+// Step j of a row on the groups k >= K - KA, returning the lane's sums.  Rows
+// start at even l - m, so j's parity is that of l - m.
+template <int K, int KA>
+__device__ __forceinline__ void adj_step(AdjState<K>& st, bool odd, double A, const double (&y)[K], double& sr,
+                                         double& si)
 {
     sr = 0.0;
     si = 0.0;
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const double nu = fma(Al * st.x[k], st.mu1[k], -st.mu2[k]);
+    for (int k = K - KA; k < K; ++k) {
+        const double nu = fma(odd ? A : A * y[k], st.mu1[k], -st.mu2[k]);
         st.mu2[k] = st.mu1[k];
         st.mu1[k] = nu;
-        double pr, pi;
-        adj_psi<K>(in, k, o, pr, pi);
-        sr = fma(nu, pr, sr);
-        si = fma(nu, pi, si);
+        sr = fma(nu, odd ? st.por[k] : st.per[k], sr);
+        si = fma(nu, odd ? st.poi[k] : st.pei[k], si);
     }
 }
 
-template <int K>
-__device__ __forceinline__ void adj_step(LegState<K>& st, const AdjIn<K>& in, AdjRed& rd, int l, int m, double Al)
+// Rows r .. rend - 1 with KA groups; SCALED: with a rescale check after each
+// row, until every lane is live.  a holds row r's coefficients; a row loads
+// the next one's after its first step (scalar loads return out of order: the
+// wait before that step would otherwise cover them), and reads the previous
+// row's tile there, which it finishes halfway.  Eight steps multiply |mu| by
+// at most prod (A_l + 1) < 2^45 (A_{m+1} = sqrt(2m + 2) is the largest
+// factor), so from 2^900 no value overflows between checks; a lane whose scale
+// count reaches 0 inside a row joins at the row's end, dropping terms below
+// 2^-42 of O(1).
+template <int K, int KA, bool SCALED>
+__device__ __forceinline__ bool adj_rows(AdjState<K>& st, AdjRed& rd, const AdjItem& it, scdouble* A, double (&a)[8],
+                                         const double* yl, int& r, int rend, bool all)
 {
-    if ((l - m) & 1)
-        adj_live<K, true>(st, in, rd, Al);
-    else
-        adj_live<K, false>(st, in, rd, Al);
-}
-
-// Steps l..cend of one staged chunk while some lane is still scaled: single
-// steps up to a row boundary (rescale check after each), then rows of
-// kRedChunk = 8 steps reduced like the live rows with one rescale check per
-// row, then (at the item's end) the rest one step at a time.  It returns once
-// every lane is live; the caller finishes the chunk with live rows.  Eight steps multiply |mu| by at most prod (A_l + 1) < 2^45
-// (A_{m+1} = sqrt(2m + 2) is the largest factor), so from 2^900 no value
-// overflows between checks; a lane whose scale count reaches 0 inside a row
-// joins at the row's end, dropping terms below 2^-55 of O(1).
-template <int K, bool ODD0>
-__device__ __forceinline__ void adj_scaled_rows(LegState<K>& st, AdjIn<K>& in, AdjRed& rd, int& l, int cend, int cb,
-                                                const double* cA, const AdjSrc& s)
-{
-    for (; !st.all && l + 7 <= cend; l += 8) {
-        double z[8];
-        double2 t4[4];
+    double2 t4[4];
+    bool pend = false;
+    const int lane = rd.lane;
+    // multipliers of a row's first step: x^2, in every second row its
+    // corrected values (Ring)
+    double y0[K];
+    auto load_y0 = [&](int row) {
+        const double* src = yl + ((row & 1) ? 0 : (row & 15) ? 64 * K : 128 * K) + lane;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            double are, aim, bre, bim;
-            adj_step_v<K>(st, in, ODD0, cA[l + 2 * p - cb], are, aim);
-            adj_step_v<K>(st, in, !ODD0, cA[l + 2 * p + 1 - cb], bre, bim);
-            AdjRed::fold_pair(are, aim, bre, bim, z[2 * p], z[2 * p + 1]);
-        }
+        for (int k = K - KA; k < K; ++k) y0[k] = src[64 * k];
+    };
+    load_y0(r);
+    while (r < rend && !(SCALED && all)) {
+        double z[8], are, aim, bre, bim, an[8];
+        adj_step<K, KA>(st, false, a[0], y0, are, aim);
+        __builtin_amdgcn_sched_barrier(0);
+        if (pend) rd.tile_load(t4);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) an[q] = A[8 * (long)(r + 1) + q];
+        adj_step<K, KA>(st, true, a[1], st.y, bre, bim);
+        z[0] = swap32_add(are, bre);
+        z[1] = swap32_add(aim, bim);
+        adj_step<K, KA>(st, false, a[2], st.y, are, aim);
+        adj_step<K, KA>(st, true, a[3], st.y, bre, bim);
+        z[2] = swap32_add(are, bre);
+        z[3] = swap32_add(aim, bim);
+        if (pend) rd.finish_row(t4);
+        adj_step<K, KA>(st, false, a[4], st.y, are, aim);
+        __builtin_amdgcn_sched_barrier(0);
+        load_y0(r + 1);
+        adj_step<K, KA>(st, true, a[5], st.y, bre, bim);
+        z[4] = swap32_add(are, bre);
+        z[5] = swap32_add(aim, bim);
+        adj_step<K, KA>(st, false, a[6], st.y, are, aim);
+        adj_step<K, KA>(st, true, a[7], st.y, bre, bim);
+        z[6] = swap32_add(are, bre);
+        z[7] = swap32_add(aim, bim);
         rd.tile_store(z);
-        rd.tile_load(t4);
-        rd.finish_row(t4);
-        wave_sync();
-        adj_rescale<K>(st, in, s);
-    }
-}
-
-template <int K>
-__device__ __forceinline__ void adj_chunk_scaled(LegState<K>& st, AdjIn<K>& in, AdjRed& rd, int& l, int cend,
-                                                 int cb, int m, const double* cA, const AdjSrc& s)
-{
-    while (!st.all && rd.cnt != 0 && l <= cend) {
-        adj_step<K>(st, in, rd, l, m, cA[l - cb]);
-        ++l;
-        adj_rescale<K>(st, in, s);
-    }
-    if (!st.all && l + 7 <= cend) {
-        if ((l - m) & 1)
-            adj_scaled_rows<K, true>(st, in, rd, l, cend, cb, cA, s);
-        else
-            adj_scaled_rows<K, false>(st, in, rd, l, cend, cb, cA, s);
-    }
-    while (!st.all && l <= cend) {
-        adj_step<K>(st, in, rd, l, m, cA[l - cb]);
-        ++l;
-        adj_rescale<K>(st, in, s);
-    }
-}
-
-// Steps l..cend of one staged chunk with every lane live: single steps up to
-// the next reduction row boundary, then rows of kRedChunk = 8 steps with two
-// 4-coefficient register sets alternating (the speculative load of the next
-// set may read up to 4 entries past the chunk, into the row padding).  A
-// row's tile is stored at its end and read back after the next row's first
-// step, and the sum finishes halfway through that row, so the LDS round trip
-// overlaps FP64 work.
-template <int K>
-__device__ __forceinline__ void adj_chunk_live(LegState<K>& st, const AdjIn<K>& in, AdjRed& rd, int& l, int cend,
-                                               int cb, int m, const double* cA)
-{
-    for (; rd.cnt != 0 && l <= cend; ++l) adj_step<K>(st, in, rd, l, m, cA[l - cb]);
-    if (l + 7 <= cend) {
-        const bool odd = ((l - m) & 1) != 0;
-        double x[4], y[4];
-        double2 t4[4];
-        bool pend = false;  // the tile holds a row not yet summed
+        pend = true;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = cA[l - cb + q];
-        for (; l + 7 <= cend; l += 8) {
-            double z[8], are, aim, bre, bim;
-            // each set's loads are issued after the first step that uses the
-            // other set, so the wait before that step covers only LDS traffic
-            // issued half an iteration earlier; the previous row's tile read
-            // rides along with the Y loads
-            adj_step_v<K>(st, in, odd, x[0], are, aim);
-            __builtin_amdgcn_sched_barrier(0);
-            if (pend) rd.tile_load(t4);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) y[q] = cA[l - cb + 4 + q];
-            adj_step_v<K>(st, in, !odd, x[1], bre, bim);
-            AdjRed::fold_pair(are, aim, bre, bim, z[0], z[1]);
-            adj_step_v<K>(st, in, odd, x[2], are, aim);
-            adj_step_v<K>(st, in, !odd, x[3], bre, bim);
-            AdjRed::fold_pair(are, aim, bre, bim, z[2], z[3]);
-            if (pend) rd.finish_row(t4);
-            adj_step_v<K>(st, in, odd, y[0], are, aim);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) x[q] = cA[l - cb + 8 + q];
-            adj_step_v<K>(st, in, !odd, y[1], bre, bim);
-            AdjRed::fold_pair(are, aim, bre, bim, z[4], z[5]);
-            adj_step_v<K>(st, in, odd, y[2], are, aim);
-            adj_step_v<K>(st, in, !odd, y[3], bre, bim);
-            AdjRed::fold_pair(are, aim, bre, bim, z[6], z[7]);
-            rd.tile_store(z);
-            pend = true;
-        }
+        for (int q = 0; q < 8; ++q) a[q] = an[q];
+        ++r;
+        if (SCALED) all = adj_rescale<K, KA>(st, it, lane);
+    }
+    if (pend) {
         rd.tile_load(t4);
         rd.finish_row(t4);
         wave_sync();
     }
-    for (; l <= cend; ++l) adj_step<K>(st, in, rd, l, m, cA[l - cb]);
+    return all;
 }
 
-// K = 4 (the adjoint's ring pairs per lane from nside 512 up) runs three
-// waves per SIMD: it needs 166 VGPRs (168 fit three waves); a four-wave bound
-// (128) spills around the step loops and measured slower.
-template <int K>
-__global__ __launch_bounds__(64, K == 4 ? 3 : 1) void k_adj(const WorkItem* __restrict__ items, const MapDesc* __restrict__ maps)
+// The rows in which KA groups of ring pairs run, then those with more.
+template <int K, int KA>
+__device__ __forceinline__ void adj_phase(AdjState<K>& st, AdjRed& rd, const AdjItem& it, scdouble* A, double (&a)[8],
+                                          const double* yl, int& r)
 {
-    __shared__ __align__(16) double red[64 * kRedStride];
-    __shared__ double sA[2][kAdjChunk + kChunkPad];
-    const WorkItem it = items[blockIdx.x];
-    if (it.mcnt == 0) return;
-    const MapDesc& md = maps[it.map];
-    const int L = md.L;
-    const int lend = it.lend;  // last l of this segment
+    const int rend = KA < K ? it.row[K - KA - 1] : it.nrow;
+    if (r < rend) {
+        int ok = 1;
+#pragma unroll
+        for (int k = K - KA; k < K; ++k) ok &= (st.sc[k] == 0);
+        bool all = __all(ok);
+        if (!all) all = adj_rows<K, KA, true>(st, rd, it, A, a, yl, r, rend, all);
+        if (r < rend) adj_rows<K, KA, false>(st, rd, it, A, a, yl, r, rend, all);
+    }
+    if constexpr (KA < K) adj_phase<K, KA + 1>(st, rd, it, A, a, yl, r);
+}
+
+template <int K>
+__global__ __launch_bounds__(64, K == 8 ? 2 : K == 4 ? 3 : 4) void k_adj(const AdjItem* __restrict__ items)
+{
+    __shared__ double2 tile[kAdjTile];
+    __shared__ double yl[3 * K * 64];
+    const AdjItem it = items[blockIdx.x];
+    if (it.nrow == 0) return;
     const int lane = threadIdx.x;
-    const int m = it.m0;
-    const int l0 = it.lfirst;
-    const long base = moff(L, m) - m;
-    gcdouble* __restrict__ A = (gcdouble*)(md.A + base);
-
-    LegState<K> st;
-    AdjIn<K> in;
-    AdjSrc src;
-    src.Q = md.Q;
-    src.row = 4 * (long)(L + 1);
-    src.m = m;
-    src.pbase = it.rb * 64 * K;
-    src.npair = md.npair;
-    src.lane = lane;
+    AdjState<K> st;
+    const auto sv = gview(it.st) + lane;
+    const __attribute__((address_space(1))) int* sk = (const __attribute__((address_space(1))) int*)it.sk + lane;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const int p = src.pbase + k * 64 + lane;
-        const long q = (long)it.sidx * 64 * K + k * 64 + lane;  // the segment's start state
-        st.x[k] = md.ring_x[p];
-        st.mu1[k] = md.s5_cur[q];
-        st.mu2[k] = md.s5_prev[q];
-        st.sc[k] = md.s5_k[q];
-        adj_load_in<K>(in, k, src);
+        const double2 v = sv[64 * k];
+        st.mu2[k] = v.x;
+        st.mu1[k] = v.y;
+        st.sc[k] = sk[64 * k];
+        const Ring c(gview(it.x)[it.p0 + 64 * k + lane]);
+        st.y[k] = c.y;
+        yl[64 * k + lane] = c.y;
+        yl[64 * (K + k) + lane] = c.ya;
+        yl[64 * (2 * K + k) + lane] = c.yb;
+        adj_load_in<K>(st, k, it, lane);
     }
     // lanes still scaled start from zero inputs
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const bool z = st.sc[k] != 0;
-        in.per[k] = z ? 0.0 : in.per[k];
-        in.pei[k] = z ? 0.0 : in.pei[k];
-        in.por[k] = z ? 0.0 : in.por[k];
-        in.poi[k] = z ? 0.0 : in.poi[k];
+        st.per[k] = z ? 0.0 : st.per[k];
+        st.pei[k] = z ? 0.0 : st.pei[k];
+        st.por[k] = z ? 0.0 : st.por[k];
+        st.poi[k] = z ? 0.0 : st.poi[k];
     }
-    st.all = all_live<K>(st.sc);
-    AdjRed rd;
-    rd.red = red;
-    rd.mine = red + lane * kRedStride;
-    rd.dst = md.upart + 2 * (long)it.rb * md.nalm + 2 * base;
-    rd.cnt = 0;
-    rd.lbase = l0;
-    rd.lane = lane;
-    if ((l0 - m) & 1)
-        adj_first<K, true>(st, in, rd);
-    else
-        adj_first<K, false>(st, in, rd);
-
-    // staged chunks of kAdjChunk = 128 steps, two coefficients per lane (each
-    // chunk ends with one unpipelined row reduction, so longer chunks drain
-    // the pipeline less often)
-    int cb = l0 + 1;
-    double tA0 = (cb + lane <= lend) ? A[cb + lane] : 0.0;
-    double tA1 = (cb + 64 + lane <= lend) ? A[cb + 64 + lane] : 0.0;
-    sA[0][lane] = tA0;
-    sA[0][64 + lane] = tA1;
     wave_sync();
-    int buf = 0;
-    int l = cb;
-    // two loops so that the scaled-path state is dead in the second
-    while (cb <= lend && !st.all) {
-        const int nb = cb + kAdjChunk;
-        if (nb + lane <= lend) tA0 = A[nb + lane];
-        if (nb + 64 + lane <= lend) tA1 = A[nb + 64 + lane];
-        adj_chunk_scaled<K>(st, in, rd, l, min(lend, nb - 1), cb, m, sA[buf], src);
-        // every lane turned live inside the chunk: its rest runs as live rows
-        if (st.all && l <= min(lend, nb - 1)) adj_chunk_live<K>(st, in, rd, l, min(lend, nb - 1), cb, m, sA[buf]);
-        if (nb <= lend) {
-            sA[buf ^ 1][lane] = tA0;
-            sA[buf ^ 1][64 + lane] = tA1;
-        }
-        wave_sync();
-        buf ^= 1;
-        cb = nb;
-    }
-    while (cb <= lend) {
-        const int nb = cb + kAdjChunk;
-        if (nb + lane <= lend) tA0 = A[nb + lane];
-        if (nb + 64 + lane <= lend) tA1 = A[nb + 64 + lane];
-        adj_chunk_live<K>(st, in, rd, l, min(lend, nb - 1), cb, m, sA[buf]);
-        if (nb <= lend) {
-            sA[buf ^ 1][lane] = tA0;
-            sA[buf ^ 1][64 + lane] = tA1;
-        }
-        wave_sync();
-        buf ^= 1;
-        cb = nb;
-    }
-    if (rd.cnt > 0) rd.flush();
+    AdjRed rd;
+    rd.tile = tile;
+    rd.dst = (gdouble*)it.u;
+    rd.l = it.l0;
+    rd.lend = it.lend;
+    rd.lane = lane;
+    scdouble* A = (scdouble*)(it.A + it.l0);
+    double a[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) a[q] = A[q];
+    int r = 0;
+    adj_phase<K, 1>(st, rd, it, A, a, yl, r);
 }
 
-// -------------------------------------------------------------- shared adjoint on the matrix cores
+// -------------------------------------------------------------- Legendre stages on the matrix cores
 //
-// Maps of one geometry share lambda_lm(theta).  For a group of up to kAdjG = 8
-// such maps (a smaller group leaves columns empty) the adjoint of one
-// (m, block of 64 ring pairs) is a matrix product,
-//   U[l][c] = sum_p Lambda[l][p] Psi[p][c],  c = (map, re / im),
-// the ring-pair sum of 16 l-rows by 16 columns taking one FP64 matrix
-// instruction per 4 ring pairs (v_mfma_f64_16x16x4f64): the sum over ring
-// pairs happens inside the instruction (no cross-lane reduction) and the
-// recurrence runs once for the 8 maps.  Lane layout of that instruction:
-// A[i][k] comes from lane i + 16 k, B[k][j] from lane j + 16 k, and D[i][j]
-// lands in lane j + 16 (i % 4), register i / 4.
-// Each lane runs the recurrence of one ring pair and writes lambda_l (times a
-// gate that is 0 while the lane is scaled) into an LDS tile of kMmaSteps
-// l-steps; the 16 rows of one parity (l - m even pairs with Psi_E, odd with
-// Psi_O) are the A operands, and the Psi of the block's 64 ring pairs stay in
-// registers as B operands for the whole item.  A workgroup is kMmaWaves
-// waves on consecutive 64-pair blocks of one m, each starting at its own
-// first live l on a common grid of tiles; their products are added in LDS
-// in wave order, so one partial per kMmaWaves blocks goes to memory.
+// Maps of one geometry share lambda_lm(theta), so the Legendre sums of a group
+// of up to kSynG = 8 such maps are matrix products with 16 columns c = (map,
+// re / im), done by v_mfma_f64_16x16x4f64: lane layout A[i][k] from lane
+// i + 16 k, B[k][j] from lane j + 16 k, D[i][j] in lane j + 16 (i % 4),
+// register i / 4.  The recurrence of each 64 ring pairs runs once for the group
+// into an LDS tile of kMmaSteps l-steps.  FP64 matrix and vector instructions
+// share the multipliers (a mixture takes the sum of both times), so the gain is
+// the shared recurrence and, in the adjoint, the sum over ring pairs inside
+// the instruction: 16 maps of nside 256 / lmax 512 take 158 us against 285 us
+// map by map (k_adj<8>), the synthesis 134 against 160 us in pairs.
 constexpr int kMmaSteps = 32;
-constexpr int kMmaRow = 65;  // doubles per tile row: the 16 rows of one parity start 4 banks apart
+constexpr int kMmaRow = 65;   // adjoint tile row: the 16 rows of one parity start 4 banks apart
+constexpr int kMmaRowS = 72;  // synthesis tile row: rows two apart start 32 banks apart
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
@@ -1795,7 +1373,12 @@ __device__ __forceinline__ void mma_rescale(double& mu1, double& mu2, int& sc, d
 // kMmaSteps recurrence steps of one ring pair into tile column `lane`: row s
 // holds lambda at l = c0 + s.  SCALED: times the gate, rescale checks every 8
 // steps.  Coefficients are read from LDS eight steps ahead of their use.
-template <bool SCALED, int RS = kMmaRow>
+// The matrix-core kernels run the recursion in its plain form, mu_l = A_l x
+// mu_{l-1} - mu_{l-2} (the states' odd values times x): between matrix
+// instructions the products A_l x are free, and the divided form with its
+// direct coefficients was slower (8 maps, nside 256: synthesis 134 and 141 us,
+// adjoint 158 and 163 us).
+template <bool SCALED, int RS>
 __device__ __forceinline__ void mma_fill(double* __restrict__ T, const double* __restrict__ cA, int lane, double x,
                                          double& mu1, double& mu2, int& sc, double& g, bool& all)
 {
@@ -1821,25 +1404,45 @@ __device__ __forceinline__ void mma_fill(double* __restrict__ T, const double* _
     }
 }
 
-// The tile holding a wave's first live l at row r0: rows below it are zero,
-// row r0 is the start state itself, later rows advance.  (Rescale checks
-// before r0 find nothing: start states are at most 2^900.)
-template <int RS = kMmaRow>
+// The synthesis' first tile: row 0 is the start state itself, later rows advance.
 __device__ __forceinline__ void mma_fill_first(double* __restrict__ T, const double* __restrict__ cA, int lane,
-                                               int r0, double x, double& mu1, double& mu2, int& sc, double& g,
-                                               bool& all)
+                                               double x, double& mu1, double& mu2, int& sc, double& g, bool& all)
 {
 #pragma unroll
     for (int s = 0; s < kMmaSteps; ++s) {
-        const bool adv = s > r0;
-        const double nu = fma(cA[s] * x, mu1, -mu2);
-        mu2 = adv ? mu1 : mu2;
-        mu1 = adv ? nu : mu1;
-        T[s * RS + lane] = s >= r0 ? mu1 * g : 0.0;
+        if (s > 0) {
+            const double nu = fma(cA[s] * x, mu1, -mu2);
+            mu2 = mu1;
+            mu1 = nu;
+        }
+        T[s * kMmaRowS + lane] = mu1 * g;
         if ((s & 7) == 7) mma_rescale(mu1, mu2, sc, g, all);
     }
 }
 
+// A wave's first tile of the adjoint: rows below its first row r0 (even) are
+// zero, later rows advance from (mu_{l-2}, mu_{l-1}) at row r0.
+__device__ __forceinline__ void mma_fill_from(double* __restrict__ T, const double* __restrict__ cA, int lane, int r0,
+                                              double x, double& mu1, double& mu2, int& sc, double& g, bool& all)
+{
+#pragma unroll
+    for (int s = 0; s < kMmaSteps; ++s) {
+        const bool adv = s >= r0;
+        const double nu = fma(cA[s] * x, mu1, -mu2);
+        mu2 = adv ? mu1 : mu2;
+        mu1 = adv ? nu : mu1;
+        T[s * kMmaRow + lane] = adv ? mu1 * g : 0.0;
+        if ((s & 7) == 7) mma_rescale(mu1, mu2, sc, g, all);
+    }
+}
+
+// Shared adjoint: U[l][c] = sum_p Lambda[l][p] Psi[p][c] for one (m, block of 64
+// ring pairs) per wave; the 16 rows of one parity of a tile are the A operands
+// and the Psi of the block's ring pairs stay in registers as B operands for
+// the whole item.  A workgroup is kMmaWaves waves on consecutive blocks of
+// one m, each starting at its own first live l (even l - m) on a common grid
+// of tiles; their products are added in LDS in wave order, so one partial per
+// kMmaWaves blocks goes to memory.
 __global__ __launch_bounds__(64 * kMmaWaves, 2) void k_adj_mma(const WorkItem* __restrict__ items,
                                                                const MmaSub* __restrict__ subs,
                                                                const MapDesc* __restrict__ maps,
@@ -1850,36 +1453,35 @@ __global__ __launch_bounds__(64 * kMmaWaves, 2) void k_adj_mma(const WorkItem* _
     const WorkItem it = items[blockIdx.x];
     if (it.mcnt == 0) return;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int* __restrict__ gm = groups + kAdjG * it.map;
+    const int* __restrict__ gm = groups + kSynG * it.map;
     const MapDesc& md = maps[gm[0]];
     const int L = md.L;
-    const int lend = it.lend;
     const int m = it.m0;
-    const int l0 = it.lfirst;  // the earliest first live l of the workgroup's blocks
+    const int l0 = it.lfirst;  // the earliest start of the workgroup's blocks, even l - m
     const long base = moff(L, m) - m;
     gcdouble* __restrict__ A = (gcdouble*)(md.A + base);
-    const int lfw = subs[it.sidx].lf[w];  // this wave's first live l, -1: no live item
+    const MmaSub& sub = subs[it.sub];
+    const int lfw = sub.lf[w];             // this wave's first l, -1: no live item
     const int rb = it.rb * kMmaWaves + w;  // this wave's 64-pair block
     double* __restrict__ Tw = T[w];
 
     // the recurrence of ring pair rb * 64 + lane, from the wave's start state
-    // (a wave without a live item may lie past the ring tables: npair_pad
-    // need not be a multiple of kMmaWaves * 64)
+    // (a wave without a live item may lie past the ring tables)
     double x = 0.0, mu1 = 0.0, mu2 = 0.0;
     int sc = 1;
     if (lfw >= 0) {
         x = md.ring_x[rb * 64 + lane];
-        const long q = (long)subs[it.sidx].sidx[w] * 64 + lane;
-        mu1 = md.s5_cur[q];
-        mu2 = md.s5_prev[q];
-        sc = md.s5_k[q];
+        const double2 v = sub.st[w][lane];
+        mu2 = v.x;
+        mu1 = v.y * x;  // l - m odd
+        sc = sub.sk[w][lane];
     }
     double g = sc == 0 ? 1.0 : 0.0;
     bool all = __all(sc == 0);
 
     // B operands: B[k][j] = Psi of ring pair rb * 64 + 4 b + k, column j =
-    // (map j / 2 of the group, re / im j % 2); a group's empty columns
-    // (entry -1) hold zeros and are not stored
+    // (map j / 2 of the group, re / im j % 2); a group's empty columns (entry
+    // -1) hold zeros and are not stored
     const int j = lane & 15, kq = lane >> 4;
     const int mapj = gm[j >> 1];
     const MapDesc& mj = maps[mapj >= 0 ? mapj : gm[0]];
@@ -1889,7 +1491,7 @@ __global__ __launch_bounds__(64 * kMmaWaves, 2) void k_adj_mma(const WorkItem* _
     if (lfw >= 0 && mapj >= 0) {
         const long row = 4 * (long)(L + 1);
         // padding pairs (past npair) read the last ring pair's row and are
-        // zeroed afterwards, so that all 32 loads are issued together
+        // zeroed afterwards, so that all loads are issued together
 #pragma unroll
         for (int b = 0; b < 16; ++b) {
             const int pp = min(rb * 64 + 4 * b + kq, md.npair - 1);
@@ -1911,30 +1513,29 @@ __global__ __launch_bounds__(64 * kMmaWaves, 2) void k_adj_mma(const WorkItem* _
     const int t = threadIdx.x;
     double tA = 0.0;
     if (t < kMmaSteps) {
-        sA[0][t] = (l0 + t <= lend) ? A[l0 + t] : 0.0;
-        tA = (l0 + kMmaSteps + t <= lend) ? A[l0 + kMmaSteps + t] : 0.0;
+        sA[0][t] = (l0 + t <= L) ? A[l0 + t] : 0.0;
+        tA = (l0 + kMmaSteps + t <= L) ? A[l0 + kMmaSteps + t] : 0.0;
     }
     __syncthreads();
     int buf = 0;
-    for (int c0 = l0; c0 <= lend; c0 += kMmaSteps) {
+    for (int c0 = l0; c0 <= L; c0 += kMmaSteps) {
         const int n2 = c0 + 2 * kMmaSteps;
-        // tile rows past lend hold finite values that no stored output uses
+        // tile rows past L hold finite values that no stored output uses
         const bool active = lfw >= 0 && lfw < c0 + kMmaSteps;
         if (active) {
             if (lfw >= c0)
-                mma_fill_first(Tw, sA[buf], lane, lfw - c0, x, mu1, mu2, sc, g, all);
+                mma_fill_from(Tw, sA[buf], lane, lfw - c0, x, mu1, mu2, sc, g, all);
             else if (all)
-                mma_fill<false>(Tw, sA[buf], lane, x, mu1, mu2, sc, g, all);
+                mma_fill<false, kMmaRow>(Tw, sA[buf], lane, x, mu1, mu2, sc, g, all);
             else
-                mma_fill<true>(Tw, sA[buf], lane, x, mu1, mu2, sc, g, all);
+                mma_fill<true, kMmaRow>(Tw, sA[buf], lane, x, mu1, mu2, sc, g, all);
         }
         wave_sync();
-        const int sE = (c0 - m) & 1;  // first tile row with l - m even
         dbl4 dE = {0.0, 0.0, 0.0, 0.0}, dO = {0.0, 0.0, 0.0, 0.0};
         if (active) {
-            // the ring-pair sums on the matrix cores, 16 l-rows of each parity
-            const double* tE = Tw + (sE + 2 * j) * kMmaRow + kq;
-            const double* tO = Tw + ((sE ^ 1) + 2 * j) * kMmaRow + kq;
+            // the ring-pair sums, 16 l-rows of each parity (even rows first)
+            const double* tE = Tw + 2 * j * kMmaRow + kq;
+            const double* tO = tE + kMmaRow;
             double aE[16], aO[16];
 #pragma unroll
             for (int b = 0; b < 16; ++b) {
@@ -1966,18 +1567,17 @@ __global__ __launch_bounds__(64 * kMmaWaves, 2) void k_adj_mma(const WorkItem* _
                     dO[r] += T[v][(4 + r) * 64 + lane];
                 }
             }
-            // row i = kq + 4 r of each parity: l = c0 + s0 + 2 i
+            // row i = kq + 4 r of each parity: l = c0 + 2 i (+ 1)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int lE = c0 + sE + 2 * (kq + 4 * r);
-                const int lO = c0 + (sE ^ 1) + 2 * (kq + 4 * r);
-                if (mapj >= 0 && lE <= lend) dst[2 * (long)lE] = dE[r];
-                if (mapj >= 0 && lO <= lend) dst[2 * (long)lO] = dO[r];
+                const int lE = c0 + 2 * (kq + 4 * r);
+                if (mapj >= 0 && lE <= L) dst[2 * (long)lE] = dE[r];
+                if (mapj >= 0 && lE + 1 <= L) dst[2 * (long)lE + 2] = dO[r];
             }
         }
         if (t < kMmaSteps) {
             sA[buf ^ 1][t] = tA;
-            tA = (n2 + t <= lend) ? A[n2 + t] : 0.0;
+            tA = (n2 + t <= L) ? A[n2 + t] : 0.0;
         }
         __syncthreads();
         buf ^= 1;
@@ -1986,20 +1586,18 @@ __global__ __launch_bounds__(64 * kMmaWaves, 2) void k_adj_mma(const WorkItem* _
 
 // -------------------------------------------------------------- shared synthesis on the matrix cores
 //
-// The synthesis of a group of up to kAdjG = 8 maps of one geometry (a smaller
+// The synthesis of a group of up to kSynG = 8 maps of one geometry (a smaller
 // group leaves columns empty) as matrix products: for a block of 64 ring
 // pairs, P[p][c] = sum_l Lambda[l][p] a_l[c] per parity, c = (map, re / im),
 // accumulated over the item's l range in registers.  Each lane runs the
 // recurrence of one ring pair (once for the group) into an LDS tile of
-// kMmaSteps l-steps as in k_adj_mma; an instruction takes 16 ring pairs by 4
+// kMmaSteps l-steps; an instruction takes 16 ring pairs by 4
 // l-steps of one parity (A, read across the tile's rows) times those 4
 // l-steps' a_lm of the 8 maps (B, from global memory, a tile ahead).  A tile
 // is 2 parities x 4 groups of 4 l-steps x 4 blocks of 16 pairs = 32
 // instructions; the item's sums (E, O per pair and map) are stored once at
 // its end.  No sums cross waves, so a workgroup is one wave; an item of K
 // ring pairs per lane runs as K workgroups, all from the item's first l.
-constexpr int kMmaRowS = 72;  // tile row stride: rows two apart start 32 banks apart
-
 template <int K>
 __global__ __launch_bounds__(64, 2) void k_synth_mma(const WorkItem* __restrict__ items,
                                                      const MapDesc* __restrict__ maps, const int* __restrict__ groups)
@@ -2009,7 +1607,7 @@ __global__ __launch_bounds__(64, 2) void k_synth_mma(const WorkItem* __restrict_
     const WorkItem it = items[blockIdx.x / K];
     if (it.mcnt == 0) return;
     const int w = blockIdx.x % K;
-    const int* __restrict__ gm = groups + kAdjG * it.map;
+    const int* __restrict__ gm = groups + kSynG * it.map;
     const MapDesc& md = maps[gm[0]];
     const int L = md.L;
     const int m = it.m0;
@@ -2023,6 +1621,10 @@ __global__ __launch_bounds__(64, 2) void k_synth_mma(const WorkItem* __restrict_
     const long q = (long)m * md.npair_pad + pbase + lane;
     const double x = md.ring_x[pbase + lane];
     double mu1 = md.s1_cur[q], mu2 = md.s1_prev[q];
+    if ((l0 - m) & 1)
+        mu1 *= x;
+    else
+        mu2 *= x;
     int sc = md.s1_k[q];
     double g = sc == 0 ? 1.0 : 0.0;
     bool all = __all(sc == 0);
@@ -2031,7 +1633,7 @@ __global__ __launch_bounds__(64, 2) void k_synth_mma(const WorkItem* __restrict_
     // the k-th l-step of a group; empty columns hold zeros and are not stored
     const int j = lane & 15, kq = lane >> 4;
     const int mapj = gm[j >> 1];
-    gcdouble* __restrict__ aj = (gcdouble*)(maps[mapj >= 0 ? mapj : gm[0]].alm + base) + (j & 1);
+    gcdouble* __restrict__ aj = (gcdouble*)(maps[mapj >= 0 ? mapj : gm[0]].alm + (aoff(L, m) - m)) + (j & 1);
     auto load_b = [&](int c0, double(&bE)[4], double(&bO)[4]) {
         const int sE = (c0 - m) & 1;
 #pragma unroll
@@ -2062,7 +1664,7 @@ __global__ __launch_bounds__(64, 2) void k_synth_mma(const WorkItem* __restrict_
         if (c0 + kMmaSteps <= L) load_b(c0 + kMmaSteps, nE, nO);
         // tile rows past L hold finite values whose B operands are zero
         if (c0 == l0)
-            mma_fill_first<kMmaRowS>(T, sA[buf], lane, 0, x, mu1, mu2, sc, g, all);
+            mma_fill_first(T, sA[buf], lane, x, mu1, mu2, sc, g, all);
         else if (all)
             mma_fill<false, kMmaRowS>(T, sA[buf], lane, x, mu1, mu2, sc, g, all);
         else
@@ -2110,7 +1712,23 @@ __global__ __launch_bounds__(64, 2) void k_synth_mma(const WorkItem* __restrict_
 }
 
 // -------------------------------------------------------------- set-up passes
-// Both run the scaled recurrence from the seed lambda_mm.
+// All run the scaled recurrence from the seed lambda_mm.
+
+// One step of the start states' recurrence (odd members divided by cos theta
+// = c), x^2 = y + lo exactly.
+template <int K>
+__device__ __forceinline__ void capture_step(LegState<K>& st, const double (&c)[K], bool odd, double Al)
+{
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const double y = c[k] * c[k], lo = fma(c[k], c[k], -y);
+        const double nu = odd ? fma(Al, st.mu1[k], -st.mu2[k])
+                              : fma(Al * y, st.mu1[k], fma(Al * lo, st.mu1[k], -st.mu2[k]));
+        st.mu2[k] = st.mu1[k];
+        st.mu1[k] = nu;
+    }
+}
+
 // k_scan: first l at which each ring pair becomes live (L+1 if never).
 template <int K>
 __global__ __launch_bounds__(64) void k_scan(const WorkItem* __restrict__ items, const MapDesc* __restrict__ maps,
@@ -2125,11 +1743,12 @@ __global__ __launch_bounds__(64) void k_scan(const WorkItem* __restrict__ items,
         const int m = it.m0 + mi;
         const double* __restrict__ A = md.A + moff(L, m) - m;
         LegState<K> st;
+        double x[K];
         int p[K], ls[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             p[k] = it.rb * 64 * K + k * 64 + lane;
-            st.x[k] = md.ring_x[p[k]];
+            x[k] = md.ring_x[p[k]];
             st.mu1[k] = md.seed_v[(long)m * npad + p[k]];
             st.sc[k] = md.seed_k[(long)m * npad + p[k]];
             st.mu2[k] = 0.0;
@@ -2139,7 +1758,12 @@ __global__ __launch_bounds__(64) void k_scan(const WorkItem* __restrict__ items,
         int l = m;
         while (!all && l < L) {
             ++l;
-            st.advance(A[l]);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const double nu = fma(A[l] * x[k], st.mu1[k], -st.mu2[k]);
+                st.mu2[k] = st.mu1[k];
+                st.mu1[k] = nu;
+            }
             if (rescale<K>(st.mu1, st.mu2, st.sc)) {
 #pragma unroll
                 for (int k = 0; k < K; ++k)
@@ -2152,8 +1776,7 @@ __global__ __launch_bounds__(64) void k_scan(const WorkItem* __restrict__ items,
     }
 }
 
-// k_capture: the state (mu_{l-1}, mu_l, scale count) at l = item.lfirst, in
-// slot sidx (adjoint segments) or at (m, pair).
+// k_capture: the state (mu_{l-1}, mu_l, scale count) at l = item.lfirst.
 template <int K>
 __global__ __launch_bounds__(64) void k_capture(const WorkItem* __restrict__ items, const MapDesc* __restrict__ maps,
                                                 double* __restrict__ prev, double* __restrict__ cur,
@@ -2169,25 +1792,53 @@ __global__ __launch_bounds__(64) void k_capture(const WorkItem* __restrict__ ite
     const double* __restrict__ A = md.A + moff(L, m) - m;
     LegState<K> st;
     int p[K];
+    double c[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         p[k] = it.rb * 64 * K + k * 64 + lane;
-        st.x[k] = md.ring_x[p[k]];
+        c[k] = md.ring_x[p[k]];
         st.mu1[k] = md.seed_v[(long)m * npad + p[k]];
         st.sc[k] = md.seed_k[(long)m * npad + p[k]];
         st.mu2[k] = 0.0;
     }
     for (int l = m + 1; l <= it.lfirst; ++l) {
-        st.advance(A[l]);
+        capture_step<K>(st, c, ((l - m) & 1) != 0, A[l]);
         rescale<K>(st.mu1, st.mu2, st.sc);
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const long q = it.sidx >= 0 ? (long)it.sidx * 64 * K + k * 64 + lane : (long)m * npad + p[k];
+        const long q = (long)m * npad + p[k];
         prev[q] = st.mu2[k];
         cur[q] = st.mu1[k];
         kout[q] = st.sc[k];
     }
+}
+
+// k_adj_capture: the adjoint's start state of 64 ring pairs of degree m at row
+// start l (even l - m): (mu_{l-2}, mu_{l-1}) and the scale count; (-mu_m, 0) at
+// l = m, from which the first step gives mu_m.
+__global__ __launch_bounds__(64) void k_adj_capture(const AdjCap* __restrict__ caps, const MapDesc* __restrict__ md_)
+{
+    const AdjCap c = caps[blockIdx.x];
+    const MapDesc& md = *md_;
+    const int L = md.L, m = c.m;
+    const double* __restrict__ A = md.A + moff(L, m) - m;
+    const int p = c.p0 + threadIdx.x;
+    LegState<1> s;
+    const double x[1] = {md.ring_x[p]};
+    s.mu1[0] = md.seed_v[(long)m * md.npair_pad + p];
+    s.sc[0] = md.seed_k[(long)m * md.npair_pad + p];
+    s.mu2[0] = 0.0;
+    if (c.l == m) {
+        s.mu2[0] = -s.mu1[0];
+        s.mu1[0] = 0.0;
+    }
+    for (int l = m + 1; l < c.l; ++l) {
+        capture_step<1>(s, x, ((l - m) & 1) != 0, A[l]);
+        rescale<1>(s.mu1, s.mu2, s.sc);
+    }
+    c.st[threadIdx.x] = make_double2(s.mu2[0], s.mu1[0]);
+    c.sk[threadIdx.x] = s.sc[0];
 }
 
 // ================================================================== ring stage
@@ -3220,6 +2871,19 @@ __global__ __launch_bounds__(1024) void k_dot_final(const double* __restrict__ p
 
 // ================================================================== launchers
 
+// Raise a kernel's dynamic-LDS limit to kMaxLds once per device (function
+// attributes belong to a device; one bit per device id in `done`).
+static int allow_dynamic_lds(const void* fn, std::atomic<unsigned long long>& done)
+{
+    int dev = 0;
+    CMBL_HIP(hipGetDevice(&dev));
+    const unsigned long long bit = 1ull << (dev & 63);
+    if (done.load(std::memory_order_acquire) & bit) return CMBL_OK;
+    CMBL_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+    done.fetch_or(bit, std::memory_order_acq_rel);
+    return CMBL_OK;
+}
+
 int lm_tiles(int L)
 {
     const int nt = (L + kLM) / kLM;
@@ -3237,15 +2901,20 @@ template <int K>
 static int synth_k(const WorkItem* items, int n, const MapDesc* d_maps, hipStream_t s)
 {
     if (n <= 0) return CMBL_OK;
-    hipLaunchKernelGGL(k_synth<K>, dim3(n), dim3(64), 0, s, items, d_maps);
+    hipLaunchKernelGGL((k_synth<K, 1>), dim3(n), dim3(64), 0, s, items, d_maps, (const int*)nullptr);
     CMBL_HIP(hipGetLastError());
     return CMBL_OK;
 }
-template <int K>
-static int adj_k(const WorkItem* items, int n, const MapDesc* d_maps, hipStream_t s)
+int launch_adj(int K, const AdjItem* items, int n, hipStream_t s)
 {
     if (n <= 0) return CMBL_OK;
-    hipLaunchKernelGGL(k_adj<K>, dim3(n), dim3(64), 0, s, items, d_maps);
+    switch (K) {
+    case 1: hipLaunchKernelGGL(k_adj<1>, dim3(n), dim3(64), 0, s, items); break;
+    case 2: hipLaunchKernelGGL(k_adj<2>, dim3(n), dim3(64), 0, s, items); break;
+    case 4: hipLaunchKernelGGL(k_adj<4>, dim3(n), dim3(64), 0, s, items); break;
+    case 8: hipLaunchKernelGGL(k_adj<8>, dim3(n), dim3(64), 0, s, items); break;
+    default: return fail(CMBL_ERR_ARG, "unsupported rings-per-lane K");
+    }
     CMBL_HIP(hipGetLastError());
     return CMBL_OK;
 }
@@ -3278,31 +2947,16 @@ static int scan_k(const WorkItem* items, int n, const MapDesc* d_maps, int* d_ls
     return CMBL_OK;
 }
 
-template <int K, int G>
-static int synth_g(const WorkItem* items, int n, const MapDesc* d_maps, const int* d_groups, hipStream_t s)
+int launch_synth_pairs(int K, const WorkItem* items, int n, const MapDesc* d_maps, const int* d_groups, hipStream_t s)
 {
     if (n <= 0) return CMBL_OK;
-    hipLaunchKernelGGL((k_synth_g<K, G>), dim3(n), dim3(64), 0, s, items, d_maps, d_groups);
+    switch (K) {
+    case 1: hipLaunchKernelGGL((k_synth<1, 2>), dim3(n), dim3(64), 0, s, items, d_maps, d_groups); break;
+    case 2: hipLaunchKernelGGL((k_synth<2, 2>), dim3(n), dim3(64), 0, s, items, d_maps, d_groups); break;
+    default: return fail(CMBL_ERR_ARG, "unsupported shared-synthesis shape");
+    }
     CMBL_HIP(hipGetLastError());
     return CMBL_OK;
-}
-
-int launch_synth_group(int K, int G, const WorkItem* items, int n, const MapDesc* d_maps, const int* d_groups,
-                       hipStream_t s)
-{
-    if (G == 4) {
-        switch (K) {
-        case 1: return synth_g<1, 4>(items, n, d_maps, d_groups, s);
-        case 2: return synth_g<2, 4>(items, n, d_maps, d_groups, s);
-        }
-    } else if (G == 2) {
-        switch (K) {
-        case 1: return synth_g<1, 2>(items, n, d_maps, d_groups, s);
-        case 2: return synth_g<2, 2>(items, n, d_maps, d_groups, s);
-        case 4: return synth_g<4, 2>(items, n, d_maps, d_groups, s);
-        }
-    }
-    return fail(CMBL_ERR_ARG, "unsupported shared-synthesis shape");
 }
 
 int launch_synth(int K, const WorkItem* items, int n, const MapDesc* d_maps, hipStream_t s)
@@ -3312,16 +2966,6 @@ int launch_synth(int K, const WorkItem* items, int n, const MapDesc* d_maps, hip
     case 2: return synth_k<2>(items, n, d_maps, s);
     case 4: return synth_k<4>(items, n, d_maps, s);
     case 8: return synth_k<8>(items, n, d_maps, s);
-    }
-    return fail(CMBL_ERR_ARG, "unsupported rings-per-lane K");
-}
-int launch_adj(int K, const WorkItem* items, int n, const MapDesc* d_maps, hipStream_t s)
-{
-    switch (K) {
-    case 1: return adj_k<1>(items, n, d_maps, s);
-    case 2: return adj_k<2>(items, n, d_maps, s);
-    case 4: return adj_k<4>(items, n, d_maps, s);
-    case 8: return adj_k<8>(items, n, d_maps, s);
     }
     return fail(CMBL_ERR_ARG, "unsupported rings-per-lane K");
 }
@@ -3346,6 +2990,14 @@ int launch_capture(int K, const WorkItem* items, int n, const MapDesc* d_maps, d
     return fail(CMBL_ERR_ARG, "unsupported rings-per-lane K");
 }
 
+int launch_adj_capture(const AdjCap* caps, int n, const MapDesc* d_md, hipStream_t s)
+{
+    if (n <= 0) return CMBL_OK;
+    hipLaunchKernelGGL(k_adj_capture, dim3(n), dim3(64), 0, s, caps, d_md);
+    CMBL_HIP(hipGetLastError());
+    return CMBL_OK;
+}
+
 int launch_scan(int K, const WorkItem* items, int n, const MapDesc* d_maps, int* d_lstart, hipStream_t s)
 {
     switch (K) {
@@ -3355,19 +3007,6 @@ int launch_scan(int K, const WorkItem* items, int n, const MapDesc* d_maps, int*
     case 8: return scan_k<8>(items, n, d_maps, d_lstart, s);
     }
     return fail(CMBL_ERR_ARG, "unsupported rings-per-lane K");
-}
-
-// Raise a kernel's dynamic-LDS limit to kMaxLds once per device (function
-// attributes belong to a device; one bit per device id in `done`).
-static int allow_dynamic_lds(const void* fn, std::atomic<unsigned long long>& done)
-{
-    int dev = 0;
-    CMBL_HIP(hipGetDevice(&dev));
-    const unsigned long long bit = 1ull << (dev & 63);
-    if (done.load(std::memory_order_acquire) & bit) return CMBL_OK;
-    CMBL_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
-    done.fetch_or(bit, std::memory_order_acq_rel);
-    return CMBL_OK;
 }
 
 template <int MODE, int MAXM>
@@ -3445,26 +3084,13 @@ int launch_pre_pol(const MapDesc& md, const MapDesc* d_md, const double* t, cons
     return CMBL_OK;
 }
 
-template <int K>
-static int synth_pol_k(const WorkItem* items, int n, const MapDesc* d_md, const double2* rec, double* pt, double* pq,
-                       double* pu, hipStream_t s)
-{
-    if (n <= 0) return CMBL_OK;
-    hipLaunchKernelGGL(k_synth_pol<K>, dim3(n), dim3(64), 0, s, items, d_md, rec, pt, pq, pu);
-    CMBL_HIP(hipGetLastError());
-    return CMBL_OK;
-}
-
 int launch_synth_pol(int K, const WorkItem* items, int n, const MapDesc* d_md, const double2* d_rec, double* d_pt,
                      double* d_pq, double* d_pu, hipStream_t s)
 {
-    switch (K) {
-    case 1: return synth_pol_k<1>(items, n, d_md, d_rec, d_pt, d_pq, d_pu, s);
-    case 2: return synth_pol_k<2>(items, n, d_md, d_rec, d_pt, d_pq, d_pu, s);
-    case 4: return synth_pol_k<4>(items, n, d_md, d_rec, d_pt, d_pq, d_pu, s);
-    case 8: return synth_pol_k<8>(items, n, d_md, d_rec, d_pt, d_pq, d_pu, s);
-    }
-    return fail(CMBL_ERR_ARG, "unsupported rings-per-lane K");
+    if (n <= 0) return CMBL_OK;
+    hipLaunchKernelGGL(k_synth_pol, dim3(n, K), dim3(64), 0, s, items, d_md, d_rec, d_pt, d_pq, d_pu);
+    CMBL_HIP(hipGetLastError());
+    return CMBL_OK;
 }
 
 int launch_reorder(const double* in, double* out, long nside, int to_ring, hipStream_t s)

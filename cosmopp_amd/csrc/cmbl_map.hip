@@ -133,8 +133,6 @@ static int dupload(cmbl_map* mp, T** p, const std::vector<T>& h)
     return CMBL_OK;
 }
 
-
-
 // Work lists for a Legendre stage with K rings per lane.  One item per live
 // (m, ring block); lfirst is the first l at which any of its pairs is live.
 // The cost estimate counts VALU work per lane: 3 per scaled step, 4 per live
@@ -159,41 +157,122 @@ static void build_items(const cmbl_map* mp, int K, const std::vector<int>& lstar
             }
             if (lmin > L) continue;
             const double cost = K * (3.0 * (lmax - lmin) + 4.0 * (L - lmax + 1)) + 64.0 * K;
-            out->push_back(ItemCost{WorkItem{map_index, m, 1, rb, lmin, L, -1, 0}, cost});
+            out->push_back(ItemCost{WorkItem{map_index, m, 1, rb, lmin, 0, {0, 0}}, cost});
         }
     }
 }
 
-// Adjoint items cut along l into segments of at most S steps, each starting
-// from its own captured recurrence state (slot sidx): the adjoint's outputs
-// are per l, so segments of one (m, ring block) write disjoint parts of its
-// row, and the long low-m items no longer set the launch's tail.
-static int adj_segment_len(int L) { return std::max(256, ((L / 4 + 127) / 128) * 128); }
-// Segments only where the adjoint has few items: below this count a launch
-// is a few waves per SIMD (three fit at once) and its longest items set its
-// length; at nside 512 / lmax 1024 (4,100 items) segments took the adjoint
-// from 0.153 to 0.122 ms, at nside 1024 / lmax 2048 (16,000) they changed
-// nothing and at nside 2048 (65,000) cost up to 4%.
-static const size_t kSegmentBelow = 12288;
-
-static void segment_items(std::vector<ItemCost>* v, int L, int S, int K, std::vector<ItemCost>* whole)
+// Longest segment (l-steps, a multiple of 8) of a launch of `live` whole
+// items: enough items for three rounds of two waves per SIMD, but no segments
+// under 64 steps, where an item's fixed part (its loads, about two
+// microseconds) would outweigh its rows.
+static int adj_segment(size_t live, int L)
 {
-    std::vector<ItemCost> out;
-    whole->clear();
-    for (const ItemCost& c : *v) {
-        whole->push_back(c);
-        whole->back().it.sidx = (int)out.size();  // the first segment's start state is the item's
-        const double len = (double)(L - c.it.lfirst + 1);
-        for (int l0 = c.it.lfirst; l0 <= L; l0 += S) {
-            ItemCost sg = c;
-            sg.it.lfirst = l0;
-            sg.it.lend = std::min(L, l0 + S - 1);
-            sg.it.sidx = (int)out.size();
-            sg.cost = (c.cost - 64.0 * K) * (double)(sg.it.lend - l0 + 1) / len + 64.0 * K;
-            out.push_back(sg);
+    const size_t want = 3 * 2048;
+    if (live >= want) return (L + 16) / 8 * 8;
+    const long len = (long)(L / 2 + 1) * (long)live / (long)want;
+    return std::max(64, (int)((len + 63) / 64 * 64));
+}
+
+// Adjoint items of a map's geometry with K ring pairs per lane (state
+// addresses as indices until fill_adj; map, Q and u set by adj_for).  One item
+// per live (m, block of 64 K ring pairs), cut along l into segments (unless
+// `whole`) where there are too few items to fill the chip: the outputs are per
+// l, so the segments of one (m, block) write disjoint parts of its row.
+// Each group of 64 pairs joins at the row of its first live l.
+static void build_adj(const cmbl_map* mp, int K, bool whole, std::vector<AdjCost>* out, std::vector<AdjCap>* caps)
+{
+    const int L = mp->L, n64 = mp->npair_pad / 64;
+    // blocks of the real ring pairs only
+    const int nb = (mp->npair + 64 * K - 1) / (64 * K);
+    std::vector<int> first((size_t)nb * (L + 1), L + 1);
+    size_t live = 0;
+    for (int b = 0; b < nb; ++b)
+        for (int m = 0; m <= L; ++m) {
+            int& f = first[(size_t)b * (L + 1) + m];
+            for (int k = 0; k < K && b * K + k < n64; ++k) f = std::min(f, mp->lmin64[(size_t)m * n64 + b * K + k]);
+            live += f <= L;
         }
+    const int seg = whole ? (L + 16) / 8 * 8 : adj_segment(live, L);
+    for (int b = 0; b < nb; ++b)
+        for (int m = 0; m <= L; ++m) {
+            const int lf = first[(size_t)b * (L + 1) + m];
+            if (lf > L) continue;
+            const int lb = lf - ((lf - m) & 1);  // rows start at even l - m
+            for (int l0 = lb; l0 <= L; l0 += seg) {
+                AdjItem it{};
+                it.A = mp->desc.A + (moff(L, m) - m);
+                it.x = mp->desc.ring_x;
+                it.m0 = m;
+                it.l0 = l0;
+                it.nrow = (std::min(seg, L - l0 + 1) + 7) / 8;
+                it.p0 = b * 64 * K;
+                it.npair = mp->npair;
+                it.L = L;
+                it.lend = std::min(L, l0 + seg - 1);
+                it.part = b;
+                it.seg = (l0 - lb) / seg;
+                const size_t at = caps->size() * 64;
+                it.st = reinterpret_cast<const double2*>(at * sizeof(double2));
+                it.sk = reinterpret_cast<const int*>(at * sizeof(int));
+                double cost = 300.0;
+                int top = it.nrow;
+                for (int k = 0; k < K; ++k) {
+                    const int u = b * K + k;
+                    const int lk = u < n64 ? mp->lmin64[(size_t)m * n64 + u] : L + 1;
+                    int row = lk > it.lend ? it.nrow : std::max(0, (lk - l0) / 8);
+                    // groups join in the order K - 1, .., 0
+                    top = std::min(top, row);
+                    row = top;
+                    it.row[k] = (unsigned short)row;
+                    cost += 28.0 * (it.nrow - row);
+                    // a group that never joins gets a state too (unused)
+                    caps->push_back(AdjCap{nullptr, nullptr, m, std::min(u, n64 - 1) * 64,
+                                           row < it.nrow ? l0 + 8 * row : m, 0});
+                }
+                cost += 60.0 * (it.nrow - top);
+                // rows before the first group's are not run
+                out->push_back(AdjCost{it, cost});
+            }
+        }
+}
+
+// Allocates and fills the start states of build_adj's items (their st and sk
+// become pointers); the buffers are appended to allocs.
+static int fill_adj(const cmbl_map* mp, std::vector<AdjCost>* items, std::vector<AdjCap>* caps, std::vector<void*>* allocs)
+{
+    const size_t n = std::max<size_t>(caps->size(), 1) * 64;
+    void *ps = nullptr, *pk = nullptr, *dc = nullptr;
+    CMBL_HIP(hipMalloc(&ps, n * sizeof(double2)));
+    allocs->push_back(ps);
+    CMBL_HIP(hipMalloc(&pk, n * sizeof(int)));
+    allocs->push_back(pk);
+    for (AdjCost& c : *items) {
+        c.it.st = reinterpret_cast<const double2*>((char*)ps + reinterpret_cast<size_t>(c.it.st));
+        c.it.sk = reinterpret_cast<const int*>((char*)pk + reinterpret_cast<size_t>(c.it.sk));
     }
-    *v = out;
+    for (size_t i = 0; i < caps->size(); ++i) {
+        (*caps)[i].st = (double2*)ps + i * 64;
+        (*caps)[i].sk = (int*)pk + i * 64;
+    }
+    if (caps->empty()) return CMBL_OK;
+    CMBL_HIP(hipMalloc(&dc, caps->size() * sizeof(AdjCap)));
+    int rc = CMBL_OK;
+    if (hipMemcpy(dc, caps->data(), caps->size() * sizeof(AdjCap), hipMemcpyHostToDevice) != hipSuccess)
+        rc = fail(CMBL_ERR_HIP, "adjoint set-up");
+    if (rc == CMBL_OK) rc = launch_adj_capture((const AdjCap*)dc, (int)caps->size(), mp->d_desc, nullptr);
+    if (rc == CMBL_OK && hipDeviceSynchronize() != hipSuccess) rc = fail(CMBL_ERR_HIP, "adjoint set-up");
+    (void)hipFree(dc);
+    return rc;
+}
+
+// A geometry's adjoint item for map `index` of its list.
+static AdjCost adj_for(AdjCost c, int index, const MapDesc& d)
+{
+    c.it.map = index;
+    c.it.Q = d.Q + 4 * (long)c.it.m0;
+    c.it.u = d.upart + 2 * ((long)c.it.part * d.nalm + moff(d.L, c.it.m0) - c.it.m0);
+    return c;
 }
 
 // XCD-aware order.  Workgroup i runs on XCD i % 8, so the list is built as
@@ -201,9 +280,16 @@ static void segment_items(std::vector<ItemCost>* v, int L, int S, int K, std::ve
 // (which share the 128-byte lines of the pair-major stage buffers) go to the
 // same XCD; groups are spread over the XCDs by total cost; each XCD list is
 // ordered by cost, largest first; short lists are padded with empty items.
-static std::vector<WorkItem> order_items(std::vector<ItemCost>& v)
+// Items that stay together: the synthesis' quads of m (they write parts of the
+// same lines: nside 512 88 -> 82 us); the adjoint's items each on their own
+// (its reads are spread over the whole item: together 109, by cost 105 us).
+static std::tuple<int, int, int> item_quad(const WorkItem& it) { return {it.map, it.m0 >> 2, it.rb}; }
+static std::tuple<int, int, int> item_quad(const AdjItem& it) { return {it.map, it.m0, it.part << 16 | it.seg}; }
+
+template <typename Cost>
+static auto order_items(const std::vector<Cost>& v)
 {
-    std::vector<WorkItem> out;
+    std::vector<decltype(Cost::it)> out;
     if (v.empty()) return out;
     std::vector<std::pair<long, double>> groups;  // (key, cost)
     std::vector<long> keys(v.size());
@@ -229,17 +315,33 @@ static std::vector<WorkItem> order_items(std::vector<ItemCost>& v)
         assign.push_back({g.first, x});
     }
     std::sort(assign.begin(), assign.end());
-    std::vector<std::vector<ItemCost>> lists(kXcds);
+    std::vector<std::vector<Cost>> lists(kXcds);
     for (size_t i = 0; i < v.size(); ++i) {
         const auto itx = std::lower_bound(assign.begin(), assign.end(), std::make_pair(keys[i], -1));
         lists[itx->second].push_back(v[i]);
     }
     size_t len = 0;
     for (auto& l : lists) {
-        std::stable_sort(l.begin(), l.end(), [](const ItemCost& a, const ItemCost& b) { return a.cost > b.cost; });
+        // by the largest cost of the items that stay together
+        auto quad = [](const Cost& c) { return item_quad(c.it); };
+        std::map<decltype(quad(l[0])), double> top;
+        for (const Cost& c : l) {
+            double& t = top[quad(c)];
+            t = std::max(t, c.cost);
+        }
+        std::vector<std::pair<double, size_t>> order;
+        for (size_t i = 0; i < l.size(); ++i) order.push_back({top[quad(l[i])], i});
+        std::sort(order.begin(), order.end(), [&](const auto& a, const auto& b) {
+            if (a.first != b.first) return a.first > b.first;
+            return std::make_tuple(quad(l[a.second]), l[a.second].it.m0, a.second) <
+                   std::make_tuple(quad(l[b.second]), l[b.second].it.m0, b.second);
+        });
+        std::vector<Cost> sorted;
+        for (const auto& o : order) sorted.push_back(l[o.second]);
+        l.swap(sorted);
         len = std::max(len, l.size());
     }
-    out.resize(len * kXcds, WorkItem{0, 0, 0, 0, 0, 0, -1, 0});
+    out.resize(len * kXcds, decltype(Cost::it){});  // empty items: mcnt = 0, nrow = 0
     for (int x = 0; x < kXcds; ++x)
         for (size_t j = 0; j < lists[x].size(); ++j) out[j * kXcds + x] = lists[x][j].it;
     return out;
@@ -304,13 +406,6 @@ static int run_ring(int mode, const RingItem* d_items, const std::vector<RingCla
     for (const RingClass& c : classes)
         CMBL_TRY(launch_ring(mode, d_items + c.first, c.count, d_maps, c.lds, out, in, tw, s));
     return CMBL_OK;
-}
-
-static int choose_k(int npair, int kmax)
-{
-    int k = 1;
-    while (k < kmax && npair >= 64 * k * 2 * 4) k *= 2;  // keep >= 4 ring blocks per m
-    return k;
 }
 
 // ------------------------------------------------------------------ launch-shape tuning
@@ -384,6 +479,18 @@ static void tuning_load_default(const std::string& arch)
     }
 }
 
+// Launch shapes by size.  Synthesis: no cross-lane reduction, so one ring pair
+// per lane (more items, less mixed live / negligible work per wave) until
+// there are items enough for two (n512: 82 against 88 us; n1024: 475 against
+// 440 us).  Adjoint: the reduction's share halves with each doubling of the
+// ring pairs per lane, as long as the blocks keep items for the chip (n1024:
+// 570 us at 4, 527 at 8; n512 107 and 105; n256 28, 28 and 31 at 2, 4, 8).
+static cmbl_tuning rule_tuning(int nside)
+{
+    const int npair = 2 * nside;
+    return cmbl_tuning{npair >= 2048 ? 2 : 1, npair >= 1024 ? 8 : npair >= 512 ? 4 : npair >= 128 ? 2 : 1, 4096};
+}
+
 // The tuning a new map of this geometry gets: the table's entry, else the rule.
 static cmbl_tuning default_tuning(int nside, int lmax)
 {
@@ -394,10 +501,7 @@ static cmbl_tuning default_tuning(int nside, int lmax)
         for (const TuneEntry& e : g_tune)
             if (e.arch == arch && e.nside == nside && e.lmax == lmax) return e.t;
     }
-    // synthesis: no cross-lane reduction, so small ring blocks (less mixed
-    // live/negligible work per wave); adjoint: four rings per lane amortise
-    // the per-l lane reduction
-    return cmbl_tuning{choose_k(2 * nside, 2), choose_k(2 * nside, 4), 4096};
+    return rule_tuning(nside);
 }
 
 static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune)
@@ -418,7 +522,6 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     const int kmax = std::max(mp->K1, mp->K5);
     mp->npair_pad = ((mp->npair + 64 * kmax - 1) / (64 * kmax)) * (64 * kmax);
     mp->nrb1 = mp->npair_pad / (64 * mp->K1);
-    mp->nrb5 = mp->npair_pad / (64 * mp->K5);
     const int npad = mp->npair_pad;
 
     // Bluestein rings longer than split_limit are split into two half-length
@@ -471,7 +574,8 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     mp->lds_ring = lds_bytes(std::max(maxM, 2 * kRingThreads));
 
     // ---- recurrence tables (long double on the host, rounded once)
-    std::vector<double> A(mp->nalm, 0.0), Nrm(mp->nalm, 1.0);
+    // A is read up to two rows of eight past the last degree (k_adj)
+    std::vector<double> A(mp->nalm + 16, 0.0), Nrm(mp->nalm, 1.0);
     for (int m = 0; m <= L; ++m) {
         const long b = moff(L, m) - m;
         long double Nm2 = 1.0L, Nm1 = 1.0L;  // N_{l-2}, N_{l-1}
@@ -535,7 +639,6 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     d.npair = mp->npair;
     d.npair_pad = npad;
     d.nring = mp->nring;
-    d.nrb5 = mp->nrb5;
     d.npix = mp->npix;
     d.nalm = mp->nalm;
     double *p_rx, *p_A, *p_N, *p_sv;
@@ -558,6 +661,7 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     CMBL_TRY(dupload(mp, &p_so, scrofs));
     d.ring_scrofs = p_so;
     CMBL_TRY(dalloc(mp, &d.ring_scr, (size_t)std::max<long>(scr_total, 1)));
+    A.resize(A.size() + 64, 0.0);  // room for the loads ahead of use past the last row
     CMBL_TRY(dupload(mp, &p_A, A));
     CMBL_TRY(dupload(mp, &p_N, Nrm));
     CMBL_TRY(dupload(mp, &p_sv, seed_v));
@@ -592,12 +696,15 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     d.d = mp->d_data;
     d.w = mp->d_w;
     // workspace
-    CMBL_TRY(dalloc(mp, &d.alm, mp->nalm));
+    {
+        // zero row ends, and room past the last row for loads ahead of use
+        const size_t n = (size_t)mp->nalm + (size_t)kAlmPad * (L + 1) + 64;
+        CMBL_TRY(dalloc(mp, &d.alm, n));
+        CMBL_HIP(hipMemset(d.alm, 0, sizeof(double2) * n));
+    }
     CMBL_TRY(dalloc(mp, &d.P, (size_t)mp->npair * (L + 1) * 4));
     CMBL_HIP(hipMemset(d.P, 0, sizeof(double) * (size_t)mp->npair * (L + 1) * 4));
     CMBL_TRY(dalloc(mp, &d.Q, (size_t)mp->npair * (L + 1) * 4));
-    CMBL_TRY(dalloc(mp, &d.upart, (size_t)mp->nrb5 * mp->nalm * 2));
-    CMBL_HIP(hipMemset(d.upart, 0, sizeof(double) * (size_t)mp->nrb5 * mp->nalm * 2));
     CMBL_TRY(dalloc(mp, &d.chi, mp->npair));
     d.nprior = lm_tiles(L);
     CMBL_TRY(dalloc(mp, &d.prior, d.nprior));
@@ -625,7 +732,7 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     // ---- scan: first live l per (m, pair); work lists; start states
     std::vector<WorkItem> all;
     for (int rb = 0; rb < mp->nrb1; ++rb)
-        for (int m = 0; m <= L; m += 4) all.push_back(WorkItem{0, m, std::min(4, L + 1 - m), rb, m, L, -1, 0});
+        for (int m = 0; m <= L; m += 4) all.push_back(WorkItem{0, m, std::min(4, L + 1 - m), rb, m, 0, {0, 0}});
     WorkItem* d_all;
     int* d_ls;
     CMBL_TRY(dupload(mp, &d_all, all));
@@ -637,45 +744,44 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     for (int m = 0; m <= L; ++m)
         for (int p = mp->npair; p < npad; ++p) lstart[(size_t)m * npad + p] = L + 1;
 
-    std::vector<ItemCost> c1, c5;
+    mp->lmin64.assign((size_t)(L + 1) * (npad / 64), L + 1);
+    for (int m = 0; m <= L; ++m)
+        for (int q = 0; q < npad; ++q) {
+            int& v = mp->lmin64[(size_t)m * (npad / 64) + q / 64];
+            v = std::min(v, lstart[(size_t)m * npad + q]);
+        }
+    std::vector<ItemCost> c1;
     build_items(mp, mp->K1, lstart, 0, &c1);
-    build_items(mp, mp->K5, lstart, 0, &c5);
-    std::vector<ItemCost> c5whole;  // batches take whole items: they have items enough
-    if (c5.size() < kSegmentBelow) {
-        segment_items(&c5, L, adj_segment_len(L), mp->K5, &c5whole);
-    } else {
-        for (size_t i = 0; i < c5.size(); ++i) c5[i].it.sidx = (int)i;  // whole items, one slot each
-        c5whole = c5;
-    }
     mp->cost1 = c1;
-    mp->cost5 = c5whole;
     mp->items1 = order_items(c1);
-    mp->items5 = order_items(c5);
     mp->nitems1 = (int)mp->items1.size();
-    mp->nitems5 = (int)mp->items5.size();
     CMBL_TRY(dupload(mp, &mp->d_items1, mp->items1));
-    CMBL_TRY(dupload(mp, &mp->d_items5, mp->items5));
     {
         const size_t nst = (size_t)(L + 1) * npad;
-        const size_t nst5 = std::max<size_t>(c5.size(), 1) * 64 * mp->K5;  // one slot per segment
-        double *p1, *c1p, *p5, *c5p;
-        int *k1, *k5;
+        double *p1, *c1p;
+        int* k1;
         CMBL_TRY(dalloc(mp, &p1, nst));
         CMBL_TRY(dalloc(mp, &c1p, nst));
         CMBL_TRY(dalloc(mp, &k1, nst));
-        CMBL_TRY(dalloc(mp, &p5, nst5));
-        CMBL_TRY(dalloc(mp, &c5p, nst5));
-        CMBL_TRY(dalloc(mp, &k5, nst5));
         CMBL_TRY(launch_capture(mp->K1, mp->d_items1, mp->nitems1, mp->d_desc, p1, c1p, k1, nullptr));
-        CMBL_TRY(launch_capture(mp->K5, mp->d_items5, mp->nitems5, mp->d_desc, p5, c5p, k5, nullptr));
         d.s1_prev = p1;
         d.s1_cur = c1p;
         d.s1_k = k1;
-        d.s5_prev = p5;
-        d.s5_cur = c5p;
-        d.s5_k = k5;
-        CMBL_HIP(hipMemcpy(mp->d_desc, &d, sizeof(d), hipMemcpyHostToDevice));
     }
+    // adjoint: partial sums (zero where no item writes), items and start states
+    mp->nrb5 = d.nrb5 = (mp->npair + 64 * mp->K5 - 1) / (64 * mp->K5);
+    CMBL_TRY(dalloc(mp, &d.upart, (size_t)mp->nrb5 * mp->nalm * 2));
+    CMBL_HIP(hipMemset(d.upart, 0, sizeof(double) * (size_t)mp->nrb5 * mp->nalm * 2));
+    {
+        std::vector<AdjCap> caps;
+        build_adj(mp, mp->K5, false, &mp->cost5, &caps);
+        CMBL_TRY(fill_adj(mp, &mp->cost5, &caps, &mp->allocs));
+        for (AdjCost& c : mp->cost5) c = adj_for(c, 0, d);
+        const std::vector<AdjItem> items5 = order_items(mp->cost5);
+        mp->nitems5 = (int)items5.size();
+        CMBL_TRY(dupload(mp, &mp->d_items5, items5));
+    }
+    CMBL_HIP(hipMemcpy(mp->d_desc, &d, sizeof(d), hipMemcpyHostToDevice));
     // ring items: largest transform first
     for (int p = 0; p < mp->npair; ++p) mp->ring_items.push_back(RingItem{0, p});
     mp->ring_M.assign(Mfft.begin(), Mfft.begin() + mp->npair);
@@ -772,7 +878,7 @@ int eval_device(cmbl_map* mp, const double* x, double* f, double* g, hipStream_t
     CMBL_TRY(t.mark(2));
     CMBL_TRY(run_ring(kRingLike, mp->d_ring_items, mp->ring_classes, mp->d_desc, nullptr, nullptr, mp->d_tw, s));
     CMBL_TRY(t.mark(3));
-    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, mp->d_desc, s));
+    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, s));
     CMBL_TRY(t.mark(4));
     CMBL_TRY(launch_post(d, mp->d_desc, x, g, kPostLike, s));
     CMBL_TRY(t.mark(5));
@@ -912,7 +1018,7 @@ int cmbl_tune(int nside, int lmax, int reps, cmbl_tuning* best, double* times)
     if (reps < 1) return fail(CMBL_ERR_ARG, "reps must be >= 1");
     if (nside < 1 || !is_pow2(nside) || lmax < 2 || lmax > 4 * nside)
         return fail(CMBL_ERR_ARG, "nside must be a power of two and lmax in [2, 4*nside]");
-    const cmbl_tuning rule{choose_k(2 * nside, 2), choose_k(2 * nside, 4), 4096};
+    const cmbl_tuning rule = rule_tuning(nside);
     double t[11];
     for (double& v : t) v = -1.0;
     // ring pairs per lane: candidates 1, 2, 4, 8 for both Legendre stages
@@ -1109,7 +1215,7 @@ int cmbl_backward_device(cmbl_map* mp, const double* v, double* g, void* stream)
     if (!v || !g) return fail(CMBL_ERR_ARG, "null pointer");
     hipStream_t s = (hipStream_t)stream;
     CMBL_TRY(run_ring(kRingAna, mp->d_ring_items, mp->ring_classes, mp->d_desc, nullptr, v, mp->d_tw, s));
-    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, mp->d_desc, s));
+    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, s));
     CMBL_TRY(launch_post(mp->desc, mp->d_desc, nullptr, g, kPostGrad, s));
     return CMBL_OK;
 }
@@ -1131,7 +1237,7 @@ int cmbl_map2alm_quadrature_device(cmbl_map* mp, const double* map, double* alm,
     if (!map || !alm) return fail(CMBL_ERR_ARG, "null pointer");
     hipStream_t s = (hipStream_t)stream;
     CMBL_TRY(run_ring(kRingAna, mp->d_ring_items, mp->ring_classes, mp->d_desc, nullptr, map, mp->d_tw, s));
-    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, mp->d_desc, s));
+    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, s));
     CMBL_TRY(launch_post(mp->desc, mp->d_desc, nullptr, alm, kPostQuad, s, 4.0 * 3.141592653589793 / (double)mp->npix));
     return CMBL_OK;
 }
@@ -1155,7 +1261,10 @@ static int pol_setup(cmbl_map* mp)
 {
     if (mp->d_desc_pol) return CMBL_OK;
     const size_t pstride = (size_t)mp->npair * (mp->L + 1) * 4;
-    CMBL_TRY(dalloc(mp, &mp->d_pol_rec, (size_t)kPolRec * mp->nalm));
+    // padded like alm: the synthesis reads whole blocks of 16 l-steps
+    const size_t nrec = ((size_t)mp->nalm + (size_t)kAlmPad * (mp->L + 1) + 64) * (kPolRec / 2);
+    CMBL_TRY(dalloc(mp, &mp->d_pol_rec, nrec));
+    CMBL_HIP(hipMemset(mp->d_pol_rec, 0, sizeof(double2) * nrec));
     CMBL_TRY(dalloc(mp, &mp->d_pol_P, 3 * pstride));
     CMBL_HIP(hipMemset(mp->d_pol_P, 0, sizeof(double) * 3 * pstride));
     std::vector<MapDesc> v(3, mp->desc);
@@ -1315,7 +1424,7 @@ int cmbl_gibbs_apply_device(cmbl_gibbs* gb, const double* x, double* y, void* st
     CMBL_TRY(launch_pre(mp->desc, mp->d_desc, x, s));
     CMBL_TRY(launch_synth(mp->K1, mp->d_items1, mp->nitems1, mp->d_desc, s));
     CMBL_TRY(run_ring(kRingWeight, mp->d_ring_items, mp->ring_classes, mp->d_desc, nullptr, nullptr, mp->d_tw, s));
-    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, mp->d_desc, s));
+    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, s));
     CMBL_TRY(launch_post(mp->desc, mp->d_desc, x, y, kPostGibbs, s));
     return CMBL_OK;
 }
@@ -1339,11 +1448,11 @@ int cmbl_gibbs_rhs_device(cmbl_gibbs* gb, const double* d, const double* omega0,
     CMBL_TRY(cmbl_vec_axpy(gb->d_m0, omega1, gb->sigma, gb->npix, s));
     CMBL_TRY(cmbl_vec_mul(gb->d_m0, mp->d_w, gb->npix, s));
     CMBL_TRY(run_ring(kRingAna, mp->d_ring_items, mp->ring_classes, mp->d_desc, nullptr, gb->d_m0, mp->d_tw, s));
-    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, mp->d_desc, s));
+    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, s));
     CMBL_TRY(launch_post(mp->desc, mp->d_desc, nullptr, b, kPostAlm, s));
     // + sqrt(4pi/Npix) Y^T omega0 (map2alm with ring weight sqrt(Npix/4pi), :479)
     CMBL_TRY(run_ring(kRingAna, mp->d_ring_items, mp->ring_classes, mp->d_desc, nullptr, omega0, mp->d_tw, s));
-    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, mp->d_desc, s));
+    CMBL_TRY(launch_adj(mp->K5, mp->d_items5, mp->nitems5, s));
     CMBL_TRY(launch_post(mp->desc, mp->d_desc, nullptr, b, kPostAddAlm, s,
                          std::sqrt(4.0 * 3.141592653589793 / (double)gb->npix)));
     return CMBL_OK;
@@ -1407,20 +1516,18 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
         return rc;
     };
     std::vector<MapDesc> descs;
-    std::vector<ItemCost> w1[4], w5[4];
+    std::vector<ItemCost> w1[4];
+    std::vector<AdjCost> w5[4];
     std::vector<RingItem> rings;
     // maps of one geometry (nside, lmax, synthesis ring pairs per lane) share
-    // the synthesis recurrence in groups of four (then two)
-    // (groups of up to kAdjG such maps, at least kSynMinG, run the synthesis
-    // on the matrix cores first; CMBL_BATCH_MMA=0 turns that off)
+    // the synthesis recurrence: groups of up to kSynG maps, at least kSynMinG,
+    // on the matrix cores (CMBL_BATCH_MMA=0 turns that off), then pairs
     const char* mma_env = getenv("CMBL_BATCH_MMA");
     const bool mma_on = !(mma_env && mma_env[0] == '0');
-    std::vector<int> group_of(nmaps, -1);
-    std::vector<int> gtable;                   // G map indices per group
-    std::vector<std::pair<int, int>> gshape;   // (K, G) per group
+    std::vector<int> pair_of(nmaps, -1);
+    std::vector<int> ptable;                   // two map indices per pair
     std::vector<int> sgroup_of(nmaps, -1);
-    std::vector<int> stable;                   // kAdjG map indices per matrix-core synthesis group (-1: empty)
-    std::vector<int> sK;                       // its ring pairs per lane
+    std::vector<int> stable;                   // kSynG map indices per matrix-core synthesis group (-1: empty)
     {
         std::map<std::tuple<int, int, int>, std::vector<int>> byg;
         for (int i = 0; i < nmaps; ++i)
@@ -1428,57 +1535,56 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
         for (auto& kv : byg) {
             const std::vector<int>& v = kv.second;
             const int K = std::get<2>(kv.first);
+            if (K > 2) continue;
             size_t at = 0;
-            while (mma_on && (K == 1 || K == 2) && v.size() - at >= (size_t)kSynMinG) {
-                const size_t n = std::min<size_t>(kAdjG, v.size() - at);
-                const int sid = (int)sK.size();
-                sK.push_back(K);
-                for (size_t j = 0; j < (size_t)kAdjG; ++j) {
+            while (mma_on && v.size() - at >= (size_t)kSynMinG) {
+                const size_t n = std::min<size_t>(kSynG, v.size() - at);
+                const int sid = (int)stable.size() / kSynG;
+                for (size_t j = 0; j < (size_t)kSynG; ++j) {
                     stable.push_back(j < n ? v[at + j] : -1);
                     if (j < n) sgroup_of[v[at + j]] = sid;
                 }
                 at += n;
             }
-            for (int G : {4, 2}) {
-                const bool ok = (G == 4 && (K == 1 || K == 2)) || (G == 2 && K <= 4);
-                for (; ok && at + G <= v.size(); at += G) {
-                    const int gid = (int)gshape.size();
-                    gshape.push_back({K, G});
-                    for (int j = 0; j < G; ++j) {
-                        gtable.push_back(v[at + j]);
-                        group_of[v[at + j]] = gid;
-                    }
-                    gtable.resize(gtable.size() + 4 - G, -1);  // table rows of 4
-                }
+            for (; at + 2 <= v.size(); at += 2) {
+                pair_of[v[at]] = pair_of[v[at + 1]] = (int)ptable.size() / 2;
+                ptable.push_back(v[at]);
+                ptable.push_back(v[at + 1]);
             }
         }
     }
-    // maps of one geometry whose adjoint runs one ring pair per lane share it
-    // on the matrix cores in groups of kAdjG (CMBL_BATCH_MMA=0 turns this off)
+    std::vector<ItemCost> wp[2];  // items of the pairs by K - 1, map = the pair
+    // the adjoint: groups of at least kSynMinG maps of one geometry on the
+    // matrix cores; the others map by map with eight ring pairs per lane
+    // (there are items enough in a batch).  Start states and partial sums that
+    // the maps do not have belong to the batch, the states once per geometry
     std::vector<int> agroup_of(nmaps, -1);
-    std::vector<int> atable;  // kAdjG map indices per group
+    std::vector<int> atable;  // kSynG map indices per group (-1: empty)
     {
         std::map<std::pair<int, int>, std::vector<int>> bya;
         for (int i = 0; mma_on && i < nmaps; ++i)
-            if (maps[i] && maps[i]->K5 == 1) bya[std::make_pair(maps[i]->nside, maps[i]->L)].push_back(i);
-        // full groups, then the rest as one group with empty columns when it
-        // holds at least kAdjMinG maps (below that the one-pair-per-lane
-        // adjoint of each map is cheaper than the products' fixed cost)
-        for (auto& kv : bya)
-            for (size_t at = 0; at < kv.second.size(); at += kAdjG) {
-                const size_t n = std::min<size_t>(kAdjG, kv.second.size() - at);
-                if (n < (size_t)kAdjMinG) break;
-                const int gid = (int)(atable.size() / kAdjG);
-                for (size_t j = 0; j < kAdjG; ++j) {
-                    atable.push_back(j < n ? kv.second[at + j] : -1);
-                    if (j < n) agroup_of[kv.second[at + j]] = gid;
+            if (maps[i]) bya[std::make_pair(maps[i]->nside, maps[i]->L)].push_back(i);
+        for (auto& kv : bya) {
+            const std::vector<int>& v = kv.second;
+            for (size_t at = 0; v.size() - at >= (size_t)kSynMinG; at += kSynG) {
+                const size_t n = std::min<size_t>(kSynG, v.size() - at);
+                const int gid = (int)atable.size() / kSynG;
+                for (size_t j = 0; j < (size_t)kSynG; ++j) {
+                    atable.push_back(j < n ? v[at + j] : -1);
+                    if (j < n) agroup_of[v[at + j]] = gid;
                 }
+                if (n < (size_t)kSynG) break;
             }
+        }
     }
-    std::vector<ItemCost> ws[2];  // items of the matrix-core synthesis by K - 1, map = its group
-    std::vector<ItemCost> wa;  // items of the shared adjoint, map = group, sidx = entry of subs
+    struct AdjSet {
+        std::vector<AdjCost> items;
+        int K;
+    };
+    std::map<std::tuple<int, int, bool>, AdjSet> adj_sets;  // (nside, lmax, matrix cores)
+    std::vector<ItemCost> wa;  // items of the matrix-core adjoint, map = group
     std::vector<MmaSub> subs;
-    std::map<std::pair<int, int>, std::vector<ItemCost>> wg;  // (K, G) -> items
+    std::vector<ItemCost> ws[2];  // items of the matrix-core synthesis by K - 1, map = its group
     for (int i = 0; i < nmaps; ++i) {
         cmbl_map* mp = maps[i];
         if (!mp) return cleanup(fail(CMBL_ERR_ARG, "null map in batch"));
@@ -1499,74 +1605,79 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
                 descs.back().ring_chofs = descs[j].ring_chofs;
                 break;
             }
-        if (agroup_of[i] >= 0) {
-            // the shared adjoint writes one partial per kMmaWaves ring blocks
-            // (the last group may be partial), into the batch's own buffer
-            // (the map's is laid out per block)
-            const int nrb = (mp->npair_pad + 64 * kMmaWaves - 1) / (64 * kMmaWaves);
-            const size_t n = (size_t)nrb * mp->nalm * 2;
-            void* pb = nullptr;
-            if (hipMalloc(&pb, sizeof(double) * n) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
-            b->allocs.push_back(pb);
-            if (hipMemset(pb, 0, sizeof(double) * n) != hipSuccess) return cleanup(fail(CMBL_ERR_HIP, "batch"));
-            descs.back().upart = (double*)pb;
-            descs.back().nrb5 = nrb;
-        }
-        int k1 = 0, k5 = 0;
+        int k1 = 0;
         while ((1 << k1) < mp->K1) ++k1;
-        while ((1 << k5) < mp->K5) ++k5;
-        const int gid = group_of[i];
-        const int sid = sgroup_of[i];
-        if (sid >= 0) {
-            if (stable[(size_t)kAdjG * sid] == i)  // the group's first map brings the group's items
+        if (sgroup_of[i] >= 0) {
+            if (stable[(size_t)kSynG * sgroup_of[i]] == i)  // the group's first map brings the group's items
                 for (ItemCost ic : mp->cost1) {
-                    ic.it.map = sid;
+                    ic.it.map = sgroup_of[i];
                     ws[mp->K1 - 1].push_back(ic);
                 }
-        } else if (gid < 0) {
+        } else if (pair_of[i] >= 0) {
+            if (ptable[(size_t)2 * pair_of[i]] == i)
+                for (ItemCost ic : mp->cost1) {
+                    ic.it.map = pair_of[i];
+                    wp[mp->K1 - 1].push_back(ic);
+                }
+        } else {
             for (ItemCost ic : mp->cost1) {
                 ic.it.map = i;
                 w1[k1].push_back(ic);
             }
-        } else if (gtable[4 * gid] == i) {  // the group's first map brings the group's items
-            for (ItemCost ic : mp->cost1) {
-                ic.it.map = gid;
-                ic.cost *= 0.5 + 0.5 * gshape[gid].second;  // recurrence once, sums G times
-                wg[gshape[gid]].push_back(ic);
-            }
         }
-        const int agid = agroup_of[i];
-        if (agid < 0) {
-            for (ItemCost ic : mp->cost5) {
-                ic.it.map = i;
-                w5[k5].push_back(ic);
+        {
+            const bool mma = agroup_of[i] >= 0;
+            const auto key = std::make_tuple(mp->nside, mp->L, mma);
+            auto f = adj_sets.find(key);
+            if (f == adj_sets.end()) {
+                f = adj_sets.emplace(key, AdjSet{{}, 1}).first;
+                AdjSet& as = f->second;
+                while (!mma && as.K < 8 && 64 * as.K < mp->npair) as.K *= 2;
+                std::vector<AdjCap> caps;
+                build_adj(mp, as.K, mma, &as.items, &caps);
+                const int rc = fill_adj(mp, &as.items, &caps, &b->allocs);
+                if (rc != CMBL_OK) return cleanup(rc);
             }
-        } else if (atable[(size_t)kAdjG * agid] == i) {
-            // the group's first map brings its items, merged per (m, kMmaWaves
-            // consecutive ring blocks)
-            std::map<std::pair<int, int>, size_t> at;
-            for (const ItemCost& ic : mp->cost5) {
-                const std::pair<int, int> key(ic.it.m0, ic.it.rb / kMmaWaves);
-                auto f = at.find(key);
-                if (f == at.end()) {
-                    f = at.emplace(key, wa.size()).first;
-                    ItemCost g = ic;
-                    g.it.map = agid;
-                    g.it.rb = key.second;
-                    g.it.lend = mp->L;
-                    g.it.sidx = (int)subs.size();
-                    g.cost = 0.0;
-                    wa.push_back(g);
-                    MmaSub sb;
-                    for (int w = 0; w < kMmaWaves; ++w) sb.lf[w] = sb.sidx[w] = -1;
-                    subs.push_back(sb);
+            const AdjSet& as = f->second;
+            const int per = 64 * (mma ? kMmaWaves : as.K);  // ring pairs of a partial sum
+            if (mma || as.K != mp->K5) {
+                const int nrb = (mp->npair + per - 1) / per;
+                const size_t n = (size_t)nrb * mp->nalm * 2;
+                void* pb = nullptr;
+                if (hipMalloc(&pb, sizeof(double) * n) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
+                b->allocs.push_back(pb);
+                if (hipMemset(pb, 0, sizeof(double) * n) != hipSuccess) return cleanup(fail(CMBL_ERR_HIP, "batch"));
+                descs.back().upart = (double*)pb;
+                descs.back().nrb5 = nrb;
+            }
+            if (!mma) {
+                int k5 = 0;
+                while ((1 << k5) < as.K) ++k5;
+                for (const AdjCost& c : as.items) w5[k5].push_back(adj_for(c, i, descs.back()));
+            } else if (atable[(size_t)kSynG * agroup_of[i]] == i) {
+                // the group's first map brings its items, merged per (m,
+                // kMmaWaves consecutive blocks)
+                std::map<std::pair<int, int>, size_t> at;
+                for (const AdjCost& c : as.items) {
+                    const std::pair<int, int> mb(c.it.m0, c.it.part / kMmaWaves);
+                    auto g = at.find(mb);
+                    if (g == at.end()) {
+                        g = at.emplace(mb, wa.size()).first;
+                        wa.push_back(ItemCost{WorkItem{agroup_of[i], mb.first, 1, mb.second, c.it.l0, (int)subs.size(),
+                                                       {0, 0}}, 0.0});
+                        MmaSub sb{};
+                        for (int& l : sb.lf) l = -1;
+                        subs.push_back(sb);
+                    }
+                    ItemCost& ic = wa[g->second];
+                    MmaSub& sb = subs[ic.it.sub];
+                    const int w = c.it.part % kMmaWaves;
+                    sb.lf[w] = c.it.l0;
+                    sb.st[w] = c.it.st;
+                    sb.sk[w] = c.it.sk;
+                    ic.it.lfirst = std::min(ic.it.lfirst, c.it.l0);
+                    ic.cost += c.cost;
                 }
-                ItemCost& g = wa[f->second];
-                MmaSub& sb = subs[g.it.sidx];
-                sb.lf[ic.it.rb % kMmaWaves] = ic.it.lfirst;
-                sb.sidx[ic.it.rb % kMmaWaves] = ic.it.sidx;
-                g.it.lfirst = std::min(g.it.lfirst, ic.it.lfirst);
-                g.cost += ic.cost;
             }
         }
         // the map's own two-ring workgroups are cut again for the batch's launches
@@ -1584,35 +1695,34 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
     if (hipMemcpy(b->d_descs, descs.data(), sizeof(MapDesc) * descs.size(), hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
     for (int k = 0; k < 4; ++k) {
-        for (int stage = 0; stage < 2; ++stage) {
-            std::vector<ItemCost>& wc = stage ? w5[k] : w1[k];
-            if (wc.empty()) continue;
-            const std::vector<WorkItem> w = order_items(wc);
-            if (hipMalloc(&q, sizeof(WorkItem) * w.size()) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
-            b->allocs.push_back(q);
-            if (hipMemcpy(q, w.data(), sizeof(WorkItem) * w.size(), hipMemcpyHostToDevice) != hipSuccess)
-                return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
-            if (stage) {
-                b->d_items5[k] = (WorkItem*)q;
-                b->n5[k] = (int)w.size();
-            } else {
-                b->d_items1[k] = (WorkItem*)q;
-                b->n1[k] = (int)w.size();
-            }
-        }
-    }
-    for (auto& kv : wg) {
-        const std::vector<WorkItem> w = order_items(kv.second);
+        if (w1[k].empty()) continue;
+        const std::vector<WorkItem> w = order_items(w1[k]);
         if (hipMalloc(&q, sizeof(WorkItem) * w.size()) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
         b->allocs.push_back(q);
         if (hipMemcpy(q, w.data(), sizeof(WorkItem) * w.size(), hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
-        cmbl_batch::SynGroupList gl;
-        gl.K = kv.first.first;
-        gl.G = kv.first.second;
-        gl.n = (int)w.size();
-        gl.d_items = (WorkItem*)q;
-        b->syn_groups.push_back(gl);
+        b->d_items1[k] = (WorkItem*)q;
+        b->n1[k] = (int)w.size();
+    }
+    for (int k = 0; k < 4; ++k) {
+        if (w5[k].empty()) continue;
+        const std::vector<AdjItem> w = order_items(w5[k]);
+        if (hipMalloc(&q, sizeof(AdjItem) * w.size()) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
+        b->allocs.push_back(q);
+        if (hipMemcpy(q, w.data(), sizeof(AdjItem) * w.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
+        b->d_items5[k] = (AdjItem*)q;
+        b->n5[k] = (int)w.size();
+    }
+    for (int k = 0; k < 2; ++k) {
+        if (wp[k].empty()) continue;
+        const std::vector<WorkItem> w = order_items(wp[k]);
+        if (hipMalloc(&q, sizeof(WorkItem) * w.size()) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
+        b->allocs.push_back(q);
+        if (hipMemcpy(q, w.data(), sizeof(WorkItem) * w.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
+        b->d_items_pair[k] = (WorkItem*)q;
+        b->n_pair[k] = (int)w.size();
     }
     for (int k = 0; k < 2; ++k) {
         if (ws[k].empty()) continue;
@@ -1650,14 +1760,12 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
             return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
         b->d_amaps = (int*)q;
     }
-    if (!gtable.empty()) {
-        // rows of four entries; a G = 2 group reads the first two of its row
-        if (hipMalloc(&q, sizeof(int) * gtable.size()) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
+    if (!ptable.empty()) {
+        if (hipMalloc(&q, sizeof(int) * ptable.size()) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
         b->allocs.push_back(q);
-        if (hipMemcpy(q, gtable.data(), sizeof(int) * gtable.size(), hipMemcpyHostToDevice) != hipSuccess)
+        if (hipMemcpy(q, ptable.data(), sizeof(int) * ptable.size(), hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
         b->d_gmaps = (int*)q;
-        b->ngroups = (int)gshape.size();
     }
     b->ring_classes = ring_classes(
         &rings, [&](const RingItem& r) { return maps[r.map]->ring_M[r.pair]; },
@@ -1724,12 +1832,12 @@ int cmbl_batch_value_and_grad_device(cmbl_batch* b, const double* const* x, doub
     for (size_t q = 0; q < groups.size(); ++q)
         CMBL_TRY(launch_pre_batch(b->d_descs + q * kBatchGroup, groups[q], s));
     for (int k = 0; k < 4; ++k) CMBL_TRY(launch_synth(1 << k, b->d_items1[k], b->n1[k], b->d_descs, s));
-    for (const cmbl_batch::SynGroupList& gl : b->syn_groups)
-        CMBL_TRY(launch_synth_group(gl.K, gl.G, gl.d_items, gl.n, b->d_descs, b->d_gmaps, s));
+    for (int k = 0; k < 2; ++k)
+        CMBL_TRY(launch_synth_pairs(k + 1, b->d_items_pair[k], b->n_pair[k], b->d_descs, b->d_gmaps, s));
     for (int k = 0; k < 2; ++k) CMBL_TRY(launch_synth_mma(k + 1, b->d_items_smma[k], b->n_smma[k], b->d_descs, b->d_smaps, s));
     CMBL_TRY(run_ring(kRingLike, b->d_ring_items, b->ring_classes, b->d_descs, nullptr, nullptr, b->d_tw, s));
     CMBL_TRY(launch_adj_mma(b->d_items_mma, b->d_subs_mma, b->n_mma, b->d_descs, b->d_amaps, s));
-    for (int k = 0; k < 4; ++k) CMBL_TRY(launch_adj(1 << k, b->d_items5[k], b->n5[k], b->d_descs, s));
+    for (int k = 3; k >= 0; --k) CMBL_TRY(launch_adj(1 << k, b->d_items5[k], b->n5[k], s));
     for (size_t q = 0; q < groups.size(); ++q) {
         CMBL_TRY(launch_post_batch(b->d_descs + q * kBatchGroup, groups[q], kPostLike, s));
         CMBL_TRY(launch_final_batch(b->d_descs + q * kBatchGroup, groups[q], s));
