@@ -342,7 +342,7 @@ int launch_pre_pol(const MapDesc& md, const MapDesc* d_md, const double* t, cons
 int launch_synth_pol(int K, const WorkItem* items, int nitems, const MapDesc* d_md, const double2* d_rec,
                      double* d_pt, double* d_pq, double* d_pu, hipStream_t s);
 int launch_reorder(const double* in, double* out, long nside, int to_ring, hipStream_t s);
-int launch_coupling(const double* w, int L, double* s0, double* M, hipStream_t s);
+int launch_coupling(const double* w, int L, double* M, hipStream_t s);
 int launch_ring(int mode, const RingItem* items, int nitems, const MapDesc* d_maps, int lds_bytes,
                 double* d_map_out, const double* d_map_in, const double2* d_tw, hipStream_t s);
 int launch_post(const MapDesc& md, const MapDesc* d_md, const double* d_x, double* d_g, int mode,

@@ -56,6 +56,28 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Compile-time loops: every index is a constant when the accumulators are laid
+// out, so they stay in registers (a runtime loop, even one that is unrolled
+// later, left them in scratch).
+template <class F, int... I>
+__device__ __forceinline__ void for_each_map(std::integer_sequence<int, I...>, F&& f)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+// acc += c x (or -= c x), c taken from lane N of the lane's row of 16.  The
+// rows hold the same 16 coefficients, so one register pair feeds 16 steps.  A
+// DPP operand must not have been written by the VALU in the last two
+// instructions: coefficients come straight from memory.
+template <int N, bool NEG>
+__device__ __forceinline__ void fmac_row(double& acc, double c, double x)
+{
+    if (NEG)
+        asm("v_fmac_f64_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(N));
+    else
+        asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(N));
+}
+
 // Global-address-space views of device memory: loads and stores through them
 // compile to global_* instructions (counted by vmcnt only) rather than flat_*
 // ones, whose lgkmcnt share makes every LDS wait also wait for memory, and
@@ -389,50 +411,168 @@ __global__ __launch_bounds__(256) void k_pre_pol(const MapDesc* __restrict__ md_
 // ================================================================== MASTER coupling
 // Mode-coupling matrix of a mask with pseudo spectrum W (source/master.cpp:180-215):
 //   M[l1][l2] = (2 l2 + 1) / (4 pi) sum_{l3 <= L} (2 l3 + 1) W_l3 (l1 l2 l3; 0 0 0)^2.
-// Only squares of the 3j symbols enter, and with g = (l1 + l2 + l3) / 2,
-// a = g - l1, b = g - l2, c = g - l3 their closed form gives two rational
-// recursions (no square roots):
-//   (l1 l2 l1-l2)^2:  1 / (2 l1 + 1) at l2 = 0, times (2c+1) b / ((c+1)(2b-1)) per l2 step;
-//   l3 -> l3 + 2:     times (2a+1)(2b+1) c (g+1) / ((a+1)(b+1)(2c-1)(2g+3)).
-// k_w3j_start tabulates the first, one thread per l1 (s0[l1 (L+1) + l2], l2 <= l1).
-__global__ __launch_bounds__(256) void k_w3j_start(int L, double* __restrict__ s0)
-{
-    const int l1 = blockIdx.x * 256 + threadIdx.x;
-    if (l1 > L) return;
-    double s = 1.0 / (2.0 * l1 + 1.0);
-    double* row = s0 + (long)l1 * (L + 1);
-    row[0] = s;
-    for (int k = 0; k < l1; ++k) {
-        const double b = l1 - k, c = k;
-        s *= (2.0 * c + 1.0) * b / ((c + 1.0) * (2.0 * b - 1.0));
-        row[k + 1] = s;
+// The symbol's closed form, with g = (l1 + l2 + l3) / 2 and h(n) = (2n)! / (4^n n!^2),
+//   (l1 l2 l3; 0 0 0)^2 = h(g - l1) h(g - l2) h(g - l3) / ((2g + 1) h(g)),
+// makes the sum of the pair l2, l1 = l2 + d, over l3 = d + 2 t, t <= l2,
+//   sum_t F_d(t) h(l2 - t) k(l2 + d + t),  F_d(t) = (2 l3 + 1) W_l3 h(t) h(d + t),
+//   k(g) = 1 / ((2g + 1) h(g)):
+// two FP64 instructions per term and no division in the loop.
+
+// C(2n, n), an integer below 2^53 for n <= 28.
+struct CentralBinomials {
+    double c[29];
+    constexpr CentralBinomials() : c{}
+    {
+        unsigned long long v = 1;
+        c[0] = 1.0;
+        for (unsigned long long n = 1; n <= 28; ++n) {
+            v = v * (2 * (2 * n - 1)) / n;
+            c[n] = (double)v;
+        }
     }
+};
+__constant__ const CentralBinomials kCentral;
+
+// h(n) = s r, r = 1 / sqrt(pi (n + 1/4)), with the series s of Gamma(n + 1/2) /
+// Gamma(n + 1) in u = 1 / (n + 1/4)^2 (its next term is below 1e-17 from n = 29);
+// h(n < 0) = 0.
+__device__ __forceinline__ double central_series(double r)
+{
+    const double v = 3.141592653589793 * (r * r), u = v * v;
+    return fma(u, fma(u, fma(u, fma(u, 180323.0 / 134217728.0, -671.0 / 524288.0), 21.0 / 8192.0), -1.0 / 64.0), 1.0);
+}
+__device__ __forceinline__ double central_h(int n)
+{
+    if (n < 29) return n < 0 ? 0.0 : ldexp(kCentral.c[n], -2 * n);
+    const double r = rsqrt(3.141592653589793 * (n + 0.25));
+    return central_series(r) * r;
+}
+__device__ __forceinline__ double central_k(int g)
+{
+    if (g < 29) return ldexp(1.0, 2 * g) / ((2.0 * g + 1.0) * kCentral.c[g]);
+    const double y = 3.141592653589793 * (g + 0.25), r = rsqrt(y);
+    return y * r / ((2.0 * g + 1.0) * central_series(r));
 }
 
-// One thread per pair l2 <= l1 (consecutive threads: consecutive l2, so the
-// l3 loops of a wavefront have similar lengths); writes M[l1][l2] and M[l2][l1].
-__global__ __launch_bounds__(256) void k_coupling(int L, const double* __restrict__ W, const double* __restrict__ s0,
-                                                  double* __restrict__ M)
+// A workgroup takes kCoupD distances d (a wave each) and 64 kCoupR degrees l2,
+// kCoupR consecutive ones per lane: when t advances, a lane's h and k move on by
+// one degree, so a step reads one new value of each from LDS for kCoupR terms.
+// Both are stored by degree modulo kCoupR, which puts the lanes of a read on
+// consecutive doubles.  F comes through the DPP operand, 16 steps per row of
+// lanes.  Bound by FP64 issue (a product and a sum per term; LDS reads take
+// about as long).  The results cross LDS so that the stores of both triangles
+// write runs of kCoupD entries.
+// lmax 1535: 994 -> 75 us (a recursion over l3 with a division per term before;
+// kCoupD 8 3% more, 16 8%; kCoupR 2 8%, 8 three times, out of registers).  Two thirds of
+// that is issue, 128 + 22 instructions per 16 steps, and the tables.
+constexpr int kCoupR = 4;
+constexpr int kCoupD = 4;
+constexpr int kCoupL = 64 * kCoupR;  // degrees l2 of a workgroup
+constexpr int kCoupT = 512;          // steps t per staging of the tables
+constexpr int kCoupS = (kCoupL + kCoupT) / kCoupR + 4;  // entries of one residue
+
+// 16 steps: F of step s in lane s of each row; ho and ko[c] index the lane's next
+// values in hC and kD (indices: pointers in an array would lose that they are LDS).  TRI: some lanes' sums end here; step s ends the sum of degree
+// index kCoupR q + s of the block, whose value is kept in end.
+template <bool TRI>
+__device__ __forceinline__ void coupling_steps(double (&acc)[kCoupR], double (&end)[kCoupR], double (&hv)[kCoupR],
+                                               double (&kv)[kCoupR], double F, const double* hC, int ho,
+                                               const double* kD, const int (&ko)[kCoupR], int q, int lane)
 {
-    const long np = (long)(L + 1) * (L + 2) / 2;
-    for (long p = blockIdx.x * 256L + threadIdx.x; p < np; p += (long)gridDim.x * 256L) {
-        long l1 = (long)((sqrt(8.0 * p + 1.0) - 1.0) * 0.5);
-        while (l1 * (l1 + 1) / 2 > p) --l1;
-        while ((l1 + 1) * (l1 + 2) / 2 <= p) ++l1;
-        const int i1 = (int)l1, i2 = (int)(p - l1 * (l1 + 1) / 2);
-        double s = s0[l1 * (L + 1) + i2];
-        double acc = 0.0;
-        const int top = min(i1 + i2, L);
-        for (int l3 = i1 - i2; l3 <= top; l3 += 2) {
-            acc = fma((2.0 * l3 + 1.0) * W[l3], s, acc);
-            const int g = (i1 + i2 + l3) >> 1;
-            const double a = g - i1, b = g - i2, c = g - l3;
-            s *= (2.0 * a + 1.0) * (2.0 * b + 1.0) * c * (g + 1.0) /
-                 ((a + 1.0) * (b + 1.0) * (2.0 * c - 1.0) * (2.0 * g + 3.0));
+    for_each_map(std::make_integer_sequence<int, 16>{}, [&](auto si) {
+        constexpr int s = decltype(si)::value;
+        constexpr int hs = (kCoupR * 16 - s) % kCoupR;  // slot of degree index 0; degree r: (r - s) mod kCoupR
+        constexpr int ks = (kCoupR - 1 + s) % kCoupR;   // slot of degree index kCoupR - 1; r: (r + s) mod kCoupR
+        hv[hs] = hC[ho + hs * kCoupS - (s + hs) / kCoupR];
+        kv[ks] = kD[ko[s % kCoupR] + s / kCoupR];
+#pragma unroll
+        for (int r = 0; r < kCoupR; ++r)
+            fmac_row<s, false>(acc[r], F, hv[(r - s + 16 * kCoupR) % kCoupR] * kv[(r + s) % kCoupR]);
+        if (TRI) end[s % kCoupR] = lane == q + s / kCoupR ? acc[s % kCoupR] : end[s % kCoupR];
+    });
+}
+
+__global__ __launch_bounds__(64 * kCoupD, 4) void k_coupling(int L, const double* __restrict__ W, double* __restrict__ M)
+{
+    constexpr int kTab = 2 * kCoupR * kCoupS + 2 * kCoupT + kCoupD, kOut = kCoupD * (kCoupL + 1);
+    __shared__ double lds[kTab > kOut ? kTab : kOut];
+    double* hC = lds;                    // h(l2 - t)
+    double* kD = hC + kCoupR * kCoupS;   // k(l2 + d + t)
+    double* hA = kD + kCoupR * kCoupS;   // h(t)
+    double* hB = hA + kCoupT;            // h(d + t)
+    const int d0 = kCoupD * blockIdx.y, b = kCoupL * blockIdx.x;
+    if (b > L - d0) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int d = d0 + w;
+    // steps of the workgroup and of this wave
+    auto steps = [&](int dd) { return dd > L ? 0 : min(b + kCoupL - 1, (L - dd) / 2) + 1; };
+    const int n0 = steps(d0), nw = (steps(d) + 15) & ~15;
+    double acc[kCoupR], end[kCoupR];
+#pragma unroll
+    for (int r = 0; r < kCoupR; ++r) acc[r] = end[r] = 0.0;
+    for (int t0 = 0; t0 < n0; t0 += kCoupT) {
+        const int nt = min(kCoupT, (n0 - t0 + 15) & ~15);  // staged steps
+        __syncthreads();
+        // hC: degree index i <-> l2 - t = b - t0 - nt + i; kD: l2 + d + t = b + d0 + t0 + i
+        for (int i = tid; i < kCoupL + nt; i += 64 * kCoupD) hC[(i % kCoupR) * kCoupS + i / kCoupR] = central_h(b - t0 - nt + i);
+        for (int i = tid; i < kCoupL + nt + kCoupD; i += 64 * kCoupD)
+            kD[(i % kCoupR) * kCoupS + i / kCoupR] = central_k(b + d0 + t0 + i);
+        for (int i = tid; i < nt; i += 64 * kCoupD) hA[i] = central_h(t0 + i);
+        for (int i = tid; i < nt + kCoupD; i += 64 * kCoupD) hB[i] = central_h(d0 + t0 + i);
+        __syncthreads();
+        const int ne = min(nt, nw - t0);
+        if (ne <= 0) continue;
+        int ho = nt / kCoupR + lane, ko[kCoupR];
+#pragma unroll
+        for (int c = 0; c < kCoupR; ++c) {
+            const int i = kCoupR - 1 + w + c;
+            ko[c] = (i % kCoupR) * kCoupS + i / kCoupR + lane;
         }
-        const double inv4pi = 0.25 / 3.141592653589793;
-        M[l1 * (L + 1) + i2] = (2.0 * i2 + 1.0) * inv4pi * acc;
-        M[(long)i2 * (L + 1) + l1] = (2.0 * i1 + 1.0) * inv4pi * acc;
+        double hv[kCoupR], kv[kCoupR];
+        // the first step's values but the ones it reads itself
+#pragma unroll
+        for (int r = 1; r < kCoupR; ++r) hv[r] = hC[ho + r * kCoupS];
+#pragma unroll
+        for (int r = 0; r < kCoupR - 1; ++r) {
+            const int i = r + w;
+            kv[r] = kD[(i % kCoupR) * kCoupS + i / kCoupR + lane];
+        }
+        const int j = lane & 15;
+        auto weight = [&](int t) { const int l3 = d + 2 * (t0 + t); return l3 <= L ? (2.0 * l3 + 1.0) * W[l3] : 0.0; };
+        double f = weight(j);
+        for (int t = 0; t < ne; t += 16) {
+            // past L the weight is zero, and so is F whatever the tables hold
+            double F = f * (hA[t + j] * hB[w + t + j]);
+            f = t + 16 < ne ? weight(t + 16 + j) : 0.0;
+            // two wait states between the VALU write and the first DPP read
+            asm volatile("s_nop 1" : "+v"(F));
+            const int q = (t0 + t - b) / kCoupR;
+            if (t0 + t < b)
+                coupling_steps<false>(acc, end, hv, kv, F, hC, ho, kD, ko, q, lane);
+            else
+                coupling_steps<true>(acc, end, hv, kv, F, hC, ho, kD, ko, q, lane);
+            ho -= 16 / kCoupR;
+#pragma unroll
+            for (int c = 0; c < kCoupR; ++c) ko[c] += 16 / kCoupR;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kCoupR; ++r) {
+        const int i = kCoupR * lane + r;
+        lds[w * (kCoupL + 1) + i] = b + i < nw ? end[r] : acc[r];
+    }
+    __syncthreads();
+    const double inv4pi = 0.25 / 3.141592653589793;
+    // row l2: the entries l1 = l2 + d0 .. of this workgroup
+    for (int u = tid; u < kCoupL * kCoupD; u += 64 * kCoupD) {
+        const int i = u / kCoupD, e = u % kCoupD, l2 = b + i, l1 = l2 + d0 + e;
+        if (l1 <= L) M[(long)l2 * (L + 1) + l1] = (2.0 * l1 + 1.0) * inv4pi * lds[e * (kCoupL + 1) + i];
+    }
+    // row l1: the entries l2 = l1 - d0 - e
+    for (int u = tid; u < (kCoupL + kCoupD - 1) * kCoupD; u += 64 * kCoupD) {
+        const int e = kCoupD - 1 - u % kCoupD, i = u / kCoupD - e, l2 = b + i, l1 = l2 + d0 + e;
+        if (i >= 0 && i < kCoupL && l1 <= L) M[(long)l1 * (L + 1) + l2] = (2.0 * l2 + 1.0) * inv4pi * lds[e * (kCoupL + 1) + i];
     }
 }
 
@@ -540,33 +680,11 @@ struct LegState {
     }
 };
 
-// Compile-time loops over the maps of a group: every index is a constant
-// when the accumulators are laid out, so they stay in registers (a runtime
-// loop, even one that is unrolled later, left them in scratch).
-template <class F, int... I>
-__device__ __forceinline__ void for_each_map(std::integer_sequence<int, I...>, F&& f)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
-
 // -------------------------------------------------------------- synthesis
 template <int K>
 struct SynAcc {
     double er[K], ei[K], orr[K], oi[K];
 };
-
-// acc += c x (or -= c x), c taken from lane N of the lane's row of 16.  The
-// rows hold the same 16 coefficients, so one register pair feeds 16 steps.  A
-// DPP operand must not have been written by the VALU in the last two
-// instructions: coefficients come straight from memory.
-template <int N, bool NEG>
-__device__ __forceinline__ void fmac_row(double& acc, double c, double x)
-{
-    if (NEG)
-        asm("v_fmac_f64_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(N));
-    else
-        asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(N));
-}
 
 // Synthesis state of a lane's K ring pairs.  With step q = l - l0 of the item,
 // the recurrence runs in place on v_q = s_q mu_{l0 + q}, s = + + - - + + - -
@@ -3065,13 +3183,9 @@ int launch_post(const MapDesc& md, const MapDesc* d_md, const double* d_x, doubl
     return CMBL_OK;
 }
 
-int launch_coupling(const double* w, int L, double* s0, double* M, hipStream_t s)
+int launch_coupling(const double* w, int L, double* M, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_w3j_start, dim3((L + 256) / 256), dim3(256), 0, s, L, s0);
-    CMBL_HIP(hipGetLastError());
-    const long np = (long)(L + 1) * (L + 2) / 2;
-    const int blocks = (int)std::min<long>((np + 255) / 256, 16384);
-    hipLaunchKernelGGL(k_coupling, dim3(blocks), dim3(256), 0, s, L, w, s0, M);
+    hipLaunchKernelGGL(k_coupling, dim3(L / kCoupL + 1, L / kCoupD + 1), dim3(64 * kCoupD), 0, s, L, w, M);
     CMBL_HIP(hipGetLastError());
     return CMBL_OK;
 }

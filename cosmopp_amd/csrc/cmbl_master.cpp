@@ -63,19 +63,17 @@ void lu_solve(const std::vector<double>& A, const std::vector<int>& piv, int n, 
 int coupling_host(const double* w, int L, std::vector<double>* M)
 {
     const size_t n = (size_t)(L + 1);
-    double *d_w = nullptr, *d_s0 = nullptr, *d_M = nullptr;
+    double *d_w = nullptr, *d_M = nullptr;
     M->assign(n * n, 0.0);
     int rc = CMBL_OK;
-    if (hipMalloc(&d_w, sizeof(double) * n) != hipSuccess || hipMalloc(&d_s0, sizeof(double) * n * n) != hipSuccess ||
-        hipMalloc(&d_M, sizeof(double) * n * n) != hipSuccess)
+    if (hipMalloc(&d_w, sizeof(double) * n) != hipSuccess || hipMalloc(&d_M, sizeof(double) * n * n) != hipSuccess)
         rc = fail(CMBL_ERR_ALLOC, "hipMalloc failed for the coupling matrix");
     if (rc == CMBL_OK && hipMemcpy(d_w, w, sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess)
         rc = fail(CMBL_ERR_HIP, "copy of W failed");
-    if (rc == CMBL_OK) rc = launch_coupling(d_w, L, d_s0, d_M, nullptr);
+    if (rc == CMBL_OK) rc = launch_coupling(d_w, L, d_M, nullptr);
     if (rc == CMBL_OK && hipMemcpy(M->data(), d_M, sizeof(double) * n * n, hipMemcpyDeviceToHost) != hipSuccess)
         rc = fail(CMBL_ERR_HIP, "copy of the coupling matrix failed");
     if (d_w) (void)hipFree(d_w);
-    if (d_s0) (void)hipFree(d_s0);
     if (d_M) (void)hipFree(d_M);
     return rc;
 }
@@ -114,7 +112,7 @@ int cmbl_coupling_matrix(const double* w, int lmax, double* M)
 int cmbl_coupling_matrix_device(const double* d_w, int lmax, double* d_work, double* d_M, void* stream)
 {
     if (!d_w || !d_work || !d_M || lmax < 0) return fail(CMBL_ERR_ARG, "bad arguments");
-    return launch_coupling(d_w, lmax, d_work, d_M, (hipStream_t)stream);
+    return launch_coupling(d_w, lmax, d_M, (hipStream_t)stream);
 }
 
 void cmbl_master_destroy(cmbl_master* m)

@@ -359,7 +359,7 @@ int cmbl_pseudo_cl(const double* alm, int lmax, double* cl);
 /* Mode-coupling matrix of Master::calculateCouplingKernel (source/master.cpp:180-249):
  * M[l1][l2] = (2 l2 + 1)/(4pi) sum_{l3 <= lmax} (2 l3 + 1) W_l3 (l1 l2 l3; 0 0 0)^2,
  * row-major (lmax+1)^2, from the mask pseudo spectrum W (lmax+1 values).  The
- * device variant needs a workspace of (lmax+1)^2 doubles. */
+ * device variant takes a workspace of (lmax+1)^2 doubles, which it leaves as it is. */
 int cmbl_coupling_matrix(const double* w, int lmax, double* M);
 int cmbl_coupling_matrix_device(const double* d_w, int lmax, double* d_work, double* d_M, void* stream);
 
