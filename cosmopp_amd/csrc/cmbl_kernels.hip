@@ -1232,40 +1232,6 @@ __device__ __forceinline__ bool adj_rescale(AdjState<K>& st, const AdjItem& it, 
     return __all(ok);
 }
 
-// Lanes 0..31 get a summed over lanes (j, j + 32), lanes 32..63 get b summed
-// likewise (v_permlane32_swap exchanges lanes 32..63 of its first operand
-// with lanes 0..31 of its second).
-__device__ __forceinline__ double swap32_add(double a, double b)
-{
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b),
-                                                     false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b),
-                                                     false, false);
-    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-
-// Rows of 16 lanes: rows 0 and 2 get a summed over row pairs (0,1) and (2,3),
-// rows 1 and 3 get b summed likewise (v_permlane16_swap exchanges the odd rows
-// of its first operand with the even rows of its second).
-__device__ __forceinline__ double swap16_add(double a, double b)
-{
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b),
-                                                     false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b),
-                                                     false, false);
-    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-
-// s plus s rotated by N lanes within each row of 16 (DPP row_ror:N); for
-// N = 8 that is s plus s of lane j ^ 8.
-template <int N>
-__device__ __forceinline__ double ror_add(double s)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(s), 0x120 + N, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(s), 0x120 + N, 0xF, 0xF, false);
-    return s + __hiloint2double(hi, lo);
-}
-
 // Rows of eight steps.  Steps 2p and 2p + 1 are folded as soon as both exist,
 // once over lane pairs (j, j + 32) with permlane32 swaps (fold_pair): z[2p + c]
 // then holds step 2p in lanes 0..31 and step 2p + 1 in lanes 32..63 (c = 0

@@ -1285,8 +1285,9 @@ int cmbl_hmc_position(cmbl_hmc* hm, double* d_out)
 // Math::ConjugateGradient::solve (include/conjugate_gradient.hpp:45-102) on
 // a Gibbs system with every vector and scalar on the device: each iteration
 // is the operator, then three fused passes (p . Ap; the x and r updates with
-// r . r, the preconditioner and r . z; the new direction), with alpha, beta
-// and the stopping test formed by the passes' final kernels.  Blocks of
+// r . r, the preconditioner and r . z; the new direction; one workgroup for
+// short vectors: k_cg_step), with alpha, beta and the stopping test formed by
+// the passes' final kernels.  Blocks of
 // kCgBlock iterations are captured in one HIP graph and replayed; the host
 // reads the iteration count and the stop flag after each block.  Once the
 // stop flag is set (|r|^2 <= precision^2, the iteration limit, or a
@@ -1461,6 +1462,133 @@ struct OpCgDir {
     __device__ void finish(const double*) {}
 };
 
+// The three passes of an iteration (OpCgPap, OpCgUpdate, OpCgDir) in one
+// workgroup that holds the vectors in registers, for n <= kCgOne: five launches
+// become one.  Such vectors occupy at most 16 of a pass's 1024 blocks, with one
+// element per thread, so the passes take their time for launching, for the
+// scalars' way through memory and for summing empty blocks.  Sums keep the
+// passes' order (wave, block of 256, then the blocks), so every iterate is the
+// same, bit for bit.  An iteration at n = 961, 2601 and 3969: 51, 52 and 52 us
+// with the passes, 37, 42 and 45 with this; with twice the elements per thread
+// the vectors no longer fit in registers.
+constexpr int kCgOneE = 4;
+constexpr long kCgOne = 1024 * kCgOneE;
+
+// The product whose terms' wave sums (64 consecutive elements each) are in sw:
+// block sums of four, their wave sum, added to 0 (the other blocks are empty).
+// Called by one wave; result in its lane 0.
+__device__ __forceinline__ double cg_one_sum(const double* sw)
+{
+    const int b = threadIdx.x & 63;
+    double part = 0.0;
+    if (b < 4 * kCgOneE)
+        for (int i = 0; i < 4; ++i) part += sw[4 * b + i];
+    double a = 0.0;
+    a += part;
+    return 0.0 + wave_sum(a);
+}
+
+__global__ __launch_bounds__(1024) void k_cg_step(CgView c, int n)
+{
+    __shared__ double sw[2][16 * kCgOneE];
+    __shared__ double sc;
+    __shared__ int stop;
+    const int tid = threadIdx.x, w = tid >> 6;
+    CgScalars st = *c.st;
+    if (st.done) return;
+    double x[kCgOneE], p[kCgOneE], r[kCgOneE], ap[kCgOneE], dl[kCgOneE];
+#pragma unroll
+    for (int u = 0; u < kCgOneE; ++u) {
+        const int e = u * 1024 + tid;
+        x[u] = p[u] = r[u] = ap[u] = 0.0;
+        dl[u] = 1.0;
+        if (e < n) {
+            p[u] = c.p[e];
+            ap[u] = c.ap[e];
+            x[u] = c.x[e];
+            r[u] = c.r[e];
+            dl[u] = c.dl[packed_l_of(e)];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kCgOneE; ++u) {
+        const double a = u * 1024 < n ? wave_sum(fma(p[u], ap[u], 0.0)) : 0.0;
+        if ((tid & 63) == 0) sw[0][16 * u + w] = a;
+    }
+    __syncthreads();
+    if (w == 0) {
+        const double pap = cg_one_sum(sw[0]);
+        if (tid == 0) {
+            stop = pap == 0.0;
+            if (pap == 0.0) {
+                st.error = 1;
+                st.done = 1;
+                *c.st = st;
+                *c.host = st;
+            } else {
+                st.alpha = st.rz / pap;
+                sc = st.alpha;
+            }
+        }
+    }
+    __syncthreads();
+    if (stop) return;
+    const double alpha = sc;
+    double z[kCgOneE];
+#pragma unroll
+    for (int u = 0; u < kCgOneE; ++u) {
+        z[u] = 0.0;
+        double a0 = 0.0, a1 = 0.0;
+        if (u * 1024 < n) {
+            x[u] = fma(alpha, p[u], x[u]);
+            r[u] = fma(-alpha, ap[u], r[u]);
+            z[u] = r[u] / dl[u];
+            a0 = wave_sum(fma(r[u], r[u], 0.0));
+            a1 = wave_sum(fma(r[u], z[u], 0.0));
+        }
+        if ((tid & 63) == 0) {
+            sw[0][16 * u + w] = a0;
+            sw[1][16 * u + w] = a1;
+        }
+    }
+    __syncthreads();
+    if (w == 0) {
+        const double rr = cg_one_sum(sw[0]), rz = cg_one_sum(sw[1]);
+        if (tid == 0) {
+            st.eps = rr;
+            st.iters += 1;
+            if (!isfinite(rr)) {
+                st.error = 2;
+                st.done = 1;
+            } else if (st.rz == 0.0) {
+                st.error = 3;
+                st.done = 1;
+            } else {
+                st.beta = rz / st.rz;
+                st.rz = rz;
+                if (!(rr > st.prec2) || st.iters >= st.max_iter) st.done = 1;
+            }
+            *c.st = st;
+            *c.host = st;
+            sc = st.beta;
+            stop = st.done;
+        }
+    }
+    __syncthreads();
+    const double beta = sc;
+    const bool last = stop;
+#pragma unroll
+    for (int u = 0; u < kCgOneE; ++u) {
+        const int e = u * 1024 + tid;
+        if (e < n) {
+            c.x[e] = x[u];
+            c.r[e] = r[u];
+            c.z[e] = z[u];
+            if (!last) c.p[e] = fma(1.0, z[u], beta * p[u]);
+        }
+    }
+}
+
 struct GibbsCg {
     hipStream_t stream = nullptr;
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
@@ -1517,6 +1645,11 @@ static int gibbs_cg_block(cmbl_gibbs* gb, hipStream_t s)
     const long n = gb->n;
     for (int i = 0; i < kCgBlock; ++i) {
         CMBL_TRY(cmbl_gibbs_apply_device(gb, v.p, v.ap, s));
+        if (n <= kCgOne) {
+            hipLaunchKernelGGL(k_cg_step, dim3(1), dim3(1024), 0, s, v, (int)n);
+            CMBL_HIP(hipGetLastError());
+            continue;
+        }
         CMBL_TRY(run_pass(OpCgPap{v, n}, gb->cg->ps, s));
         CMBL_TRY(run_pass(OpCgUpdate{v, n, 0.0, 0}, gb->cg->ps, s));
         CMBL_TRY(run_pass(OpCgDir{v, n, 0.0, 0}, gb->cg->ps, s));
