@@ -127,6 +127,19 @@ __device__ __forceinline__ GCView2 gview(const double2* p)
 }
 __device__ __forceinline__ GView2 gview(double2* p) { return GView2{(__attribute__((address_space(1))) dvec2*)p}; }
 
+// Element i of an array below 4 GB: a uniform base and a 32-bit byte offset, one
+// address register and no 64-bit arithmetic per lane.
+__device__ __forceinline__ double2 ld_at(const double2* base, unsigned i)
+{
+    const dvec2 v = *(const __attribute__((address_space(1))) dvec2*)((const __attribute__((address_space(1))) char*)base +
+                                                                     (i << 4));
+    return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ double ld_at(const double* base, unsigned i)
+{
+    return *(gcdouble*)((const __attribute__((address_space(1))) char*)base + (i << 3));
+}
+
 // ================================================================== k_pre / k_post
 // The packed parameter vector (almToVector: l-major, index l^2 + 2m - 1 + c)
 // and the m-major device arrays (alm, Nrm, upart: index moff(L, m) + l - m)
@@ -1946,7 +1959,7 @@ __device__ __forceinline__ int zp(int e) { return e + (e >> 4); }
 
 __device__ __forceinline__ double2 tw_get(const double2* __restrict__ tw, int t, int sign)
 {
-    double2 w = gview(tw)[t];
+    double2 w = ld_at(tw, t);
     if (sign > 0) w.y = -w.y;
     return w;
 }
@@ -1973,11 +1986,16 @@ __device__ __forceinline__ double2 tw16(double2 x, int j)
 
 // In-register R-point DFT (R <= 16), radix-2 decimation in frequency:
 // natural order in, u[bitrev(q)] = sum_r u_r e^{SIGN 2 pi i r q / R} out.
-template <int R, int SIGN>
+// HALF: inputs r >= R / 2 are zero (and not read).
+template <int R, int SIGN, bool HALF = false>
 __device__ __forceinline__ void dft_reg(double2 (&u)[R])
 {
+    if (HALF) {
 #pragma unroll
-    for (int s = R / 2; s >= 1; s /= 2) {
+        for (int a = 0; a < R / 2; ++a) u[a + R / 2] = tw16<SIGN>(u[a], a * (16 / R));
+    }
+#pragma unroll
+    for (int s = HALF ? R / 4 : R / 2; s >= 1; s /= 2) {
 #pragma unroll
         for (int blk = 0; blk < R; blk += 2 * s) {
 #pragma unroll
@@ -2012,7 +2030,9 @@ static_assert((1 << kLogMaxFFT) == kMaxFFT, "twiddle table length");
 // pass of its two FFTs: kFuseChirpIn multiplies each loaded input by the
 // chirp (inputs at n and beyond are zero and not read), kFuseFilt each output
 // by the chirp filter, kFuseChirpOut each output by 1/M and the chirp (outputs
-// at n and beyond are not stored).  OS is the sign of the ring transform: for
+// at n and beyond are not stored).  As M >= 2 n, the upper half of the first
+// pass' inputs and of the last pass' outputs are such: their share of the
+// butterflies is left out.  OS is the sign of the ring transform: for
 // OS > 0 the chirps are conjugated and the filter is read reversed and
 // conjugated.
 enum { kFuseNone = 0, kFuseChirpIn = 1, kFuseFilt = 2, kFuseChirpOut = 3 };
@@ -2030,7 +2050,7 @@ struct BsFuse {
 template <int OS>
 __device__ __forceinline__ double2 bs_chirp(BsFuse f, int j)
 {
-    double2 c = gview(f.chirp)[min(j, f.n - j)];
+    double2 c = ld_at(f.chirp, min(j, f.n - j));
     if (OS > 0) c.y = -c.y;
     return c;
 }
@@ -2038,7 +2058,7 @@ __device__ __forceinline__ double2 bs_chirp(BsFuse f, int j)
 template <int OS>
 __device__ __forceinline__ double2 bs_filt(BsFuse f, int r, int M)
 {
-    double2 g = gview(f.filt)[min(r, M - r)];
+    double2 g = ld_at(f.filt, min(r, M - r));
     if (OS > 0) g.y = -g.y;  // F_{M-r} conjugated, F_{M-r} = F_r
     return g;
 }
@@ -2067,12 +2087,12 @@ __device__ __forceinline__ void stockham_pass(double2* Z, int M, int p, int lp, 
             if (PRE == kFuseChirpIn) {
                 // chirps first (global loads in flight), then the LDS loads
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
+                for (int r = 0; r < R / 2; ++r) {
                     const int e = i + r * nb;
                     u[b][r] = e < fz.n ? bs_chirp<OS>(fz, e) : make_double2(0.0, 0.0);
                 }
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
+                for (int r = 0; r < R / 2; ++r) {
                     const int e = i + r * nb;
                     if (e < fz.n) u[b][r] = cmul(Z[zp(e)], u[b][r]);
                 }
@@ -2097,10 +2117,10 @@ __device__ __forceinline__ void stockham_pass(double2* Z, int M, int p, int lp, 
                     if (r + 1 < R) w = cmul(w, w1);
                 }
             }
-            dft_reg<R, SIGN>(u[b]);
+            dft_reg<R, SIGN, PRE == kFuseChirpIn>(u[b]);
             const int j = (i - k) * R + k;
 #pragma unroll
-            for (int q = 0; q < R; ++q) {
+            for (int q = 0; q < (POST == kFuseChirpOut ? R / 2 : R); ++q) {
                 const int e = j + q * p;
                 double2 v = u[b][brev_c<LR>(q)];
                 if (POST == kFuseFilt) {
@@ -2279,14 +2299,22 @@ __device__ __forceinline__ void fold_aliases(const double2* __restrict__ row, in
 // e^{i pi (k0 + t D) / n} for t = 0, 1, 2, ...: the first two factors from
 // sincospi, each later term by one complex multiply (a thread's bins and
 // samples step by a fixed D; the rounding grows by about an ulp per step, over
-// at most 16 steps).  A phase by sincospi costs a 64-bit remainder, an FP64
-// division and the polynomial, about a hundred instructions.
+// at most 16 steps).  A phase by sincospi costs an FP64 division and the
+// polynomial, about a hundred instructions, so a ring's fold and unfold, whose
+// bins are the same, start from the same pair.
 struct PhaseSeq {
     double2 cur, step;
-    __device__ __forceinline__ void init(long k0, long D, long n)
+    // e^{i pi q / n}, 0 <= q < 2 n
+    static __device__ __forceinline__ double2 cis_pi(int q, int n)
     {
-        cur = cis_pi_frac(k0, n);
-        step = cis_pi_frac(D, n);
+        double s, c;
+        sincospi((double)q / (double)n, &s, &c);
+        return make_double2(c, s);
+    }
+    __device__ __forceinline__ void init(int k0, int D, int n)  // k0 < 2 n
+    {
+        cur = cis_pi(k0, n);
+        step = cis_pi(D % (2 * n), n);
     }
     __device__ __forceinline__ double2 next()
     {
@@ -2479,6 +2507,9 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         oS[r] = mdr[r]->ring_ofsS[pr[r]];
     }
 
+    PhaseSeq phase;  // both rings have n samples
+    if (shf[0] || shf[1]) phase.init(tid, NT, n);
+
     if (MODE != kRingAna) {
         // fold, n > L: at most the alias k and the mirror n - k per bin
         double2 e[CNT], o[CNT];
@@ -2486,12 +2517,12 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
             const int L = mdr[r]->L;
-            auto rw = gview(reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4));
+            const double2* rw = reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4);
             const int k = tid + (t - r * CH) * NT;
             const int m = k <= L ? k : n - k;
             if (k <= L || (k >= 1 && n - k <= L)) {
-                e[t] = rw[2 * m];
-                o[t] = rw[2 * m + 1];
+                e[t] = ld_at(rw, 2 * m);
+                o[t] = ld_at(rw, 2 * m + 1);
             }
         }
         PhaseSeq ps;
@@ -2499,9 +2530,9 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
             const int L = mdr[r]->L;
-            auto rw = gview(reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4));
+            const double2* rw = reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4);
             const int k = tid + (t - r * CH) * NT;
-            if (t % CH == 0 && shf[r]) ps.init(tid, NT, n);
+            if (t % CH == 0) ps = phase;
             const double sg = shf[r] ? -1.0 : 1.0;  // (-1)^{j shift} at j = 1
             const double2 ph = shf[r] ? ps.next() : make_double2(1.0, 0.0);
             double2 gN = make_double2(0.0, 0.0), gS = make_double2(0.0, 0.0);
@@ -2512,8 +2543,8 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
                 gS.x += 1.0 * (e[t].x - o[t].x);
                 gS.y += 1.0 * (e[t].y - o[t].y);
                 if (mirror) {
-                    e[t] = rw[2 * (n - k)];
-                    o[t] = rw[2 * (n - k) + 1];
+                    e[t] = ld_at(rw, 2 * (n - k));
+                    o[t] = ld_at(rw, 2 * (n - k) + 1);
                 }
             }
             if (mirror) {
@@ -2546,14 +2577,12 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
-            gcdouble* dd = gview(mdr[r]->d);
-            gcdouble* ww = gview(mdr[r]->w);
             const int j = tid + (t - r * CH) * NT;
-            dN[t] = dd[oN[r] + j];
-            wN[t] = ww[oN[r] + j];
+            dN[t] = ld_at(mdr[r]->d + oN[r], j);
+            wN[t] = ld_at(mdr[r]->w + oN[r], j);
             if (oS[r] >= 0) {
-                dS[t] = dd[oS[r] + j];
-                wS[t] = ww[oS[r] + j];
+                dS[t] = ld_at(mdr[r]->d + oS[r], j);
+                wS[t] = ld_at(mdr[r]->w + oS[r], j);
             }
         }
         double chi[2] = {0.0, 0.0};
@@ -2583,10 +2612,9 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
-            gcdouble* ww = gview(mdr[r]->w);
             const int j = tid + (t - r * CH) * NT;
-            wN[t] = ww[oN[r] + j];
-            wS[t] = oS[r] >= 0 ? ww[oS[r] + j] : 0.0;
+            wN[t] = ld_at(mdr[r]->w + oN[r], j);
+            wS[t] = oS[r] >= 0 ? ld_at(mdr[r]->w + oS[r], j) : 0.0;
         }
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
@@ -2597,13 +2625,12 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         }
         __syncthreads();
     } else {  // kRingAna
-        gcdouble* in = gview(map_in);
         double2 mv[CNT];
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
             const int j = tid + (t - r * CH) * NT;
-            mv[t] = make_double2(in[oN[r] + j], oS[r] >= 0 ? in[oS[r] + j] : 0.0);
+            mv[t] = make_double2(ld_at(map_in + oN[r], j), oS[r] >= 0 ? ld_at(map_in + oS[r], j) : 0.0);
         }
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
@@ -2620,8 +2647,7 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
     for (int r = 0; r < 2; ++r) {
         const int L = mdr[r]->L;
         double2* qrow = reinterpret_cast<double2*>(mdr[r]->Q + (long)pr[r] * (L + 1) * 4);
-        PhaseSeq ps;
-        if (shf[r]) ps.init(tid, NT, n);
+        PhaseSeq ps = phase;
         for (int k = tid; k < n; k += NT) {
             const double2 ph = shf[r] ? ps.next() : make_double2(1.0, 0.0);
             if (k > L) continue;
@@ -2670,12 +2696,13 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
     const int tid = threadIdx.x;
     constexpr int CNT = (MAXM + NT - 1) / NT;  // ring samples per thread, at most
     gdouble* out = gview(map_out);
-    gcdouble* in = gview(map_in);
-    gcdouble* dd = gview(md.d);
-    gcdouble* ww = gview(md.w);
     // for n < NT the aliases of each bin are split over R thread
     // groups (reads stay coalesced over k), partial sums added in fixed order
     const int R = n < NT ? NT / n : 1;
+    // e^{i pi k/n} of the thread's bins (R > 1: of its one bin)
+    const int k1 = R > 1 ? tid % n : tid;
+    PhaseSeq phase;
+    if (shifted) phase.init(k1, NT, n);
 
     if (MODE != kRingAna) {
         const double2* row = reinterpret_cast<const double2*>(md.P + (long)p * (L + 1) * 4);
@@ -2685,20 +2712,18 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
             // per bin, and both only where n - L <= k <= L: one load per bin
             // issued for every bin of the thread before the sums, the rare
             // second one where the sums need it
-            auto rw = gview(row);
             double2 e[CNT], o[CNT];
 #pragma unroll
             for (int t = 0; t < CNT; ++t) {
                 const int k = tid + t * NT;
                 const int m = k <= L ? k : n - k;
                 if (k < n && (k <= L || (k >= 1 && n - k <= L))) {
-                    e[t] = rw[2 * m];
-                    o[t] = rw[2 * m + 1];
+                    e[t] = ld_at(row, 2 * m);
+                    o[t] = ld_at(row, 2 * m + 1);
                 }
             }
             const double sg = shifted ? -1.0 : 1.0;  // (-1)^{j shift} at j = 1
-            PhaseSeq ps;
-            if (shifted) ps.init(tid, NT, n);
+            PhaseSeq ps = phase;
 #pragma unroll
             for (int t = 0; t < CNT; ++t) {
                 const int k = tid + t * NT;
@@ -2712,8 +2737,8 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
                     gS.x += 1.0 * (e[t].x - o[t].x);
                     gS.y += 1.0 * (e[t].y - o[t].y);
                     if (mirror) {
-                        e[t] = rw[2 * (n - k)];
-                        o[t] = rw[2 * (n - k) + 1];
+                        e[t] = ld_at(row, 2 * (n - k));
+                        o[t] = ld_at(row, 2 * (n - k) + 1);
                     }
                 }
                 if (mirror) {
@@ -2725,8 +2750,7 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
                 fold_store(Z, k, ph, shifted, oS < 0, gN, gS);
             }
         } else if (R == 1) {
-            PhaseSeq ps;
-            if (shifted) ps.init(tid, NT, n);
+            PhaseSeq ps = phase;
             for (int k = tid; k < n; k += NT) {
                 double2 gN, gS;
                 fold_aliases(row, L, n, k, 0, 1, shifted, gN, gS);
@@ -2735,7 +2759,7 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
         } else {
             double2 gN = make_double2(0.0, 0.0), gS = make_double2(0.0, 0.0);
             if (tid < R * n) {
-                fold_aliases(row, L, n, tid % n, tid / n, R, shifted, gN, gS);
+                fold_aliases(row, L, n, k1, tid / n, R, shifted, gN, gS);
                 Z[zp(2 * tid)] = gN;
                 Z[zp(2 * tid + 1)] = gS;
             }
@@ -2750,7 +2774,7 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
             }
             __syncthreads();
             if (tid < n)
-                fold_store(Z, tid, shifted ? cis_pi_frac(tid, n) : make_double2(1.0, 0.0), shifted, oS < 0, gN, gS);
+                fold_store(Z, tid, phase.cur, shifted, oS < 0, gN, gS);
         }
         __syncthreads();
         ring_dft<+1, MAXM>(Z, n, M, logM, pow2, chirp, filt, tw);
@@ -2772,11 +2796,11 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
         for (int t = 0; t < CNT; ++t) {
             const int j = tid + t * NT;
             if (j < n) {
-                dN[t] = dd[oN + j];
-                wN[t] = ww[oN + j];
+                dN[t] = ld_at(md.d + oN, j);
+                wN[t] = ld_at(md.w + oN, j);
                 if (oS >= 0) {
-                    dS[t] = dd[oS + j];
-                    wS[t] = ww[oS + j];
+                    dS[t] = ld_at(md.d + oS, j);
+                    wS[t] = ld_at(md.w + oS, j);
                 }
             }
         }
@@ -2805,8 +2829,8 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
         for (int t = 0; t < CNT; ++t) {
             const int j = tid + t * NT;
             if (j < n) {
-                wN[t] = ww[oN + j];
-                wS[t] = oS >= 0 ? ww[oS + j] : 0.0;
+                wN[t] = ld_at(md.w + oN, j);
+                wS[t] = oS >= 0 ? ld_at(md.w + oS, j) : 0.0;
             }
         }
 #pragma unroll
@@ -2822,7 +2846,7 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int j = tid + t * NT;
-            if (j < n) mv[t] = make_double2(in[oN + j], oS >= 0 ? in[oS + j] : 0.0);
+            if (j < n) mv[t] = make_double2(ld_at(map_in + oN, j), oS >= 0 ? ld_at(map_in + oS, j) : 0.0);
         }
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
@@ -2836,20 +2860,17 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
     // unfold, with the aliases of bin k split over R thread groups as in the fold
     double2* qrow = reinterpret_cast<double2*>(md.Q + (long)p * (L + 1) * 4);
     if (R == 1) {
-        PhaseSeq ps;
-        if (shifted) ps.init(tid, NT, n);
         for (int k = tid; k < n; k += NT) {
-            const double2 ph = shifted ? ps.next() : make_double2(1.0, 0.0);
+            const double2 ph = shifted ? phase.next() : make_double2(1.0, 0.0);
             if (k > L) continue;
             const int nk = (k == 0) ? 0 : n - k;
             unfold_bin(qrow, L, n, k, 0, 1, shifted, ph, Z[zp(k)], Z[zp(nk)]);
         }
     } else if (tid < R * n) {  // R n <= NT: one (bin, group) per thread
-        const int k = tid % n, r = tid / n;
+        const int k = k1, r = tid / n;
         if (k <= L) {
             const int nk = (k == 0) ? 0 : n - k;
-            unfold_bin(qrow, L, n, k, r, R, shifted, shifted ? cis_pi_frac(k, n) : make_double2(1.0, 0.0), Z[zp(k)],
-                       Z[zp(nk)]);
+            unfold_bin(qrow, L, n, k, r, R, shifted, phase.cur, Z[zp(k)], Z[zp(nk)]);
         }
     }
 }
