@@ -2875,6 +2875,259 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
     }
 }
 
+// The ring stage of maps whose transforms all have at most kSmallFFT points
+// (nside <= 128): a launch of some hundred workgroups, bound by the latency of
+// one.  So, against k_ring: radix-4 passes, which keep four times as many
+// threads busy as radix 8 on a chain half as long, between two LDS buffers, one
+// barrier each; twiddles, chirps, filters and pixels loaded at the start, at
+// once with the parity sums, into LDS or the registers of the thread that uses
+// them in both directions (Bluestein's chirp products move to the steps that
+// write and read the samples, where thread k holds c_k = c_{n-k}).
+// us per call by events, before and after: nside 8 17.1 / 12.9, 32 19.1 / 14.2, 64
+// 20.3 / 15.5, 128 24.4 / 18.5 (an empty kernel: 5).
+constexpr int kSmallFFT = 1024;
+constexpr int kSmallT = 256;
+
+// DFT of the M = 2^logM points of a (those from nin on are zero), natural order
+// in and out, by way of b; returns the buffer that holds it.  sign: +-1; filt:
+// times f[q], its imaginary part times conj, at point tid + q M / 4.  (Signs by
+// value: each copy of the code is fetched once and run once.)
+__device__ __forceinline__ double2* small_fft(double2* a, double2* b, int M, int logM, int nin, const double2* tw,
+                                              double sign, bool filt, const double2 (&f)[4], double conj)
+{
+    const int i = threadIdx.x;
+    const double2 zero = make_double2(0.0, 0.0);
+    int p = 1, lp = 0;
+    if (logM & 1) {
+        const int nb = M / 2;  // at most kSmallT: logM <= 9
+        if (i < nb) {
+            const double2 x0 = i < nin ? a[zp(i)] : zero, x1 = i + nb < nin ? a[zp(i + nb)] : zero;
+            b[zp(2 * i)] = cadd(x0, x1);
+            b[zp(2 * i + 1)] = csub(x0, x1);
+        }
+        __syncthreads();
+        double2* t = a;
+        a = b;
+        b = t;
+        nin = M;
+        p = 2;
+        lp = 1;
+    }
+    const int nb = M / 4;
+    for (; p < M; p <<= 2, lp += 2) {
+        if (i < nb) {
+            double2 u[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u[r] = i + r * nb < nin ? a[zp(i + r * nb)] : zero;
+            const int k = i & (p - 1);
+            if (p > 1) {
+                double2 w1 = tw[k << (logM - 2 - lp)];  // e^{-2 pi i k / (4 p)}
+                w1.y *= -sign;
+                const double2 w2 = cmul(w1, w1);
+                u[1] = cmul(u[1], w1);
+                u[2] = cmul(u[2], w2);
+                u[3] = cmul(u[3], cmul(w2, w1));
+            }
+            const double2 s0 = cadd(u[0], u[2]), d0 = csub(u[0], u[2]), s1 = cadd(u[1], u[3]), d1 = csub(u[1], u[3]);
+            const double2 e1 = make_double2(-sign * d1.y, sign * d1.x);
+            double2 y[4] = {cadd(s0, s1), cadd(d0, e1), csub(s0, s1), csub(d0, e1)};
+            const int j = (i - k) * 4 + k;
+            const bool last = filt && 4 * p == M;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (last) y[q] = cmul(y[q], make_double2(f[q].x, conj * f[q].y));
+                b[zp(j + q * p)] = y[q];
+            }
+        }
+        __syncthreads();
+        double2* t = a;
+        a = b;
+        b = t;
+        nin = M;
+    }
+    return a;
+}
+
+// The ring's DFT of that sign: the FFT for power-of-two n, else Bluestein's two,
+// whose filter is conjugated for the + sign.  Z: data and result, Y: the other
+// buffer.
+__device__ __forceinline__ void small_dft(double2*& Z, double2*& Y, int n, int M, int logM, const double2* tw,
+                                          double sign, const double2 (&f)[4])
+{
+    const bool pow2 = M == n;
+    for (int h = pow2 ? 1 : 0; h < 2; ++h) {
+        double2* r = small_fft(Z, Y, M, logM, h == 0 ? n : M, tw, pow2 ? sign : h == 0 ? -1.0 : 1.0, h == 0, f, -sign);
+        if (r != Z) {
+            Y = Z;
+            Z = r;
+        }
+    }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kSmallT) void k_ring_small(const RingItem* __restrict__ items,
+                                                        const MapDesc* __restrict__ maps,
+                                                        double* __restrict__ map_out,
+                                                        const double* __restrict__ map_in,
+                                                        const double2* __restrict__ tw)
+{
+    // rings of up to 2 NT samples: 4 nside, and below 512 where the transform is longer
+    constexpr int NT = kSmallT, CNT = 2, kZ = kSmallFFT + kSmallFFT / 16;
+    __shared__ double2 Zs[2 * kZ];
+    __shared__ double2 tws[kSmallFFT / 4];
+    __shared__ double sh[NT / 64];
+    const RingItem it = items[blockIdx.x];
+    const MapDesc& md = maps[it.map];
+    const int tid = threadIdx.x;
+    const int L = md.L;
+    const int p = it.pair;
+    const int n = md.ring_nph[p];
+    const int M = md.ring_M[p];
+    const int logM = 31 - __builtin_clz(M);
+    const bool pow2 = (M == n);
+    const bool shifted = md.ring_shift[p] != 0;
+    const long oN = md.ring_ofsN[p];
+    const long oS = md.ring_ofsS[p];
+    // aliases of a bin over R groups of threads as in k_ring; k1: the thread's
+    // first bin and (where it is below n) sample
+    const int R = n < NT ? NT / n : 1;
+    const int k1 = R > 1 ? tid % n : tid;
+
+    const double2 one = make_double2(1.0, 0.0);
+    double2 f[4] = {one, one, one, one}, c[CNT];
+    double dN[CNT], wN[CNT], dS[CNT], wS[CNT];
+    double2 twv = one;
+    if (tid < M / 4) twv = ld_at(tw, tid << (kLogMaxFFT - logM));
+    if (!pow2) {
+        const BsFuse fz{md.bs_chirp + md.ring_chofs[p], md.bs_filt + md.ring_bsofs[p], n, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (tid < M / 4) f[q] = bs_filt<-1>(fz, tid + q * (M / 4), M);
+#pragma unroll
+        for (int t = 0; t < CNT; ++t)
+            if (k1 + t * NT < n) c[t] = bs_chirp<-1>(fz, k1 + t * NT);
+    }
+#pragma unroll
+    for (int t = 0; t < CNT; ++t) {
+        const int j = tid + t * NT;
+        dN[t] = wN[t] = dS[t] = wS[t] = 0.0;
+        if (t * NT < n && j < n && MODE != kRingSyn) {
+            if (MODE == kRingLike) dN[t] = ld_at(md.d + oN, j);
+            if (MODE == kRingAna)
+                dN[t] = ld_at(map_in + oN, j);
+            else
+                wN[t] = ld_at(md.w + oN, j);
+            if (oS >= 0) {
+                if (MODE == kRingLike) dS[t] = ld_at(md.d + oS, j);
+                if (MODE == kRingAna)
+                    dS[t] = ld_at(map_in + oS, j);
+                else
+                    wS[t] = ld_at(md.w + oS, j);
+            }
+        }
+    }
+    PhaseSeq phase;
+    if (shifted) phase.init(k1, NT, n);
+    if (tid < M / 4) tws[tid] = twv;
+    double2 *Z = Zs, *Y = Zs + kZ;
+
+    if (MODE != kRingAna) {
+        const double2* row = reinterpret_cast<const double2*>(md.P + (long)p * (L + 1) * 4);
+        if (R == 1) {
+            PhaseSeq ps = phase;
+#pragma unroll
+            for (int t = 0; t < CNT; ++t) {
+                const int k = tid + t * NT;
+                if (k >= n) continue;
+                double2 gN, gS;
+                fold_aliases(row, L, n, k, 0, 1, shifted, gN, gS);
+                fold_store(Z, k, shifted ? ps.next() : one, shifted, oS < 0, gN, gS);
+                if (!pow2) Z[zp(k)] = cmulc(Z[zp(k)], c[t]);
+            }
+        } else {
+            double2 gN, gS;
+            if (tid < R * n) {
+                fold_aliases(row, L, n, k1, tid / n, R, shifted, gN, gS);
+                Y[zp(2 * tid)] = gN;
+                Y[zp(2 * tid + 1)] = gS;
+            }
+            __syncthreads();
+            if (tid < n) {
+                gN = gS = make_double2(0.0, 0.0);
+                for (int r = 0; r < R; ++r) {
+                    gN = cadd(gN, Y[zp(2 * (r * n + tid))]);
+                    gS = cadd(gS, Y[zp(2 * (r * n + tid) + 1)]);
+                }
+                fold_store(Z, tid, phase.cur, shifted, oS < 0, gN, gS);
+                if (!pow2) Z[zp(tid)] = cmulc(Z[zp(tid)], c[0]);
+            }
+        }
+        __syncthreads();
+        small_dft(Z, Y, n, M, logM, tws, 1.0, f);
+    }
+
+    const double inv = ldexp(1.0, -logM);
+    double chi = 0.0;
+#pragma unroll
+    for (int t = 0; t < CNT; ++t) {
+        const int j = tid + t * NT;
+        if (j >= n) continue;
+        double2 v = make_double2(dN[t], dS[t]);  // kRingAna
+        if (MODE != kRingAna) {
+            v = Z[zp(j)];
+            if (!pow2) v = cmulc(make_double2(v.x * inv, v.y * inv), c[t]);
+        }
+        if (MODE == kRingSyn) {
+            map_out[oN + j] = v.x;
+            if (oS >= 0) map_out[oS + j] = v.y;
+            continue;
+        }
+        if (MODE == kRingLike) {
+            const double rN = dN[t] - v.x, fN = wN[t] * rN;
+            chi = fma(fN, rN, chi);
+            double fS = 0.0;
+            if (oS >= 0) {
+                const double rS = dS[t] - v.y;
+                fS = wS[t] * rS;
+                chi = fma(fS, rS, chi);
+            }
+            v = make_double2(fN, fS);
+        } else if (MODE == kRingWeight) {
+            v = make_double2(wN[t] * v.x, oS >= 0 ? wS[t] * v.y : 0.0);
+        }
+        Z[zp(j)] = pow2 ? v : cmul(v, c[t]);
+    }
+    if (MODE == kRingSyn) return;
+    if (MODE == kRingLike) {
+        const double t = block_sum<NT>(chi, sh);
+        if (tid == 0) md.chi[p] = t;
+    } else {
+        __syncthreads();
+    }
+    small_dft(Z, Y, n, M, logM, tws, -1.0, f);
+
+    // unfold
+    double2* qrow = reinterpret_cast<double2*>(md.Q + (long)p * (L + 1) * 4);
+    auto bin = [&](int k, int t, int r, double2 ph) {
+        if (k > L) return;
+        double2 y = Z[zp(k)], z2 = Z[zp(k == 0 ? 0 : n - k)];
+        if (!pow2) {
+            y = cmul(make_double2(y.x * inv, y.y * inv), c[t]);
+            z2 = cmul(make_double2(z2.x * inv, z2.y * inv), c[t]);
+        }
+        unfold_bin(qrow, L, n, k, r, R, shifted, ph, y, z2);
+    };
+    if (R == 1) {
+#pragma unroll
+        for (int t = 0; t < CNT; ++t) {
+            const int k = tid + t * NT;
+            if (k < n) bin(k, t, 0, shifted ? phase.next() : one);
+        }
+    } else if (tid < R * n) {
+        bin(k1, 0, tid / n, phase.cur);
+    }
+}
+
 // Bluestein set-up for one ring pair of Bluestein length n (nph, or nph/2 for
 // a split ring; even): chirp[j] = e^{-i pi j^2/n} for j <= n/2 and filt =
 // FFT_M of b_j = e^{+i pi j^2/n} for |j| < n wrapped mod M, entries 0..M/2 (the
@@ -3133,6 +3386,11 @@ static int ring_m(const RingItem* items, int n, const MapDesc* d_maps, int lds, 
 {
     if (n <= 0) return CMBL_OK;
     if (lds > kMaxLds) return fail(CMBL_ERR_ARG, "ring transform longer than the LDS FFT");
+    if (lds <= lds_bytes(kSmallFFT)) {
+        hipLaunchKernelGGL(k_ring_small<MODE>, dim3(n), dim3(kSmallT), 0, s, items, d_maps, out, in, tw);
+        CMBL_HIP(hipGetLastError());
+        return CMBL_OK;
+    }
     if (lds > lds_bytes(4096)) return ring_mm<MODE, 8192>(items, n, d_maps, lds, out, in, tw, s);
     if (lds > lds_bytes(2048)) return ring_mm<MODE, 4096>(items, n, d_maps, lds, out, in, tw, s);
     return ring_mm<MODE, 2048>(items, n, d_maps, lds, out, in, tw, s);
