@@ -476,7 +476,8 @@ __device__ __forceinline__ double central_k(int g)
 // about as long).  The results cross LDS so that the stores of both triangles
 // write runs of kCoupD entries.
 // lmax 1535: 994 -> 75 us (a recursion over l3 with a division per term before;
-// kCoupD 8 3% more, 16 8%; kCoupR 2 8%, 8 three times, out of registers).  Two thirds of
+// kCoupD 8 3% more, 16 8%; kCoupR 2 8%, 8 three times, out of registers; a bound
+// of four waves per SIMD, which spills: the same).  Two thirds of
 // that is issue, 128 + 22 instructions per 16 steps, and the tables.
 constexpr int kCoupR = 4;
 constexpr int kCoupD = 4;
@@ -505,7 +506,7 @@ __device__ __forceinline__ void coupling_steps(double (&acc)[kCoupR], double (&e
     });
 }
 
-__global__ __launch_bounds__(64 * kCoupD, 4) void k_coupling(int L, const double* __restrict__ W, double* __restrict__ M)
+__global__ __launch_bounds__(64 * kCoupD, 3) void k_coupling(int L, const double* __restrict__ W, double* __restrict__ M)
 {
     constexpr int kTab = 2 * kCoupR * kCoupS + 2 * kCoupT + kCoupD, kOut = kCoupD * (kCoupL + 1);
     __shared__ double lds[kTab > kOut ? kTab : kOut];
@@ -2299,22 +2300,14 @@ __device__ __forceinline__ void fold_aliases(const double2* __restrict__ row, in
 // e^{i pi (k0 + t D) / n} for t = 0, 1, 2, ...: the first two factors from
 // sincospi, each later term by one complex multiply (a thread's bins and
 // samples step by a fixed D; the rounding grows by about an ulp per step, over
-// at most 16 steps).  A phase by sincospi costs an FP64 division and the
-// polynomial, about a hundred instructions, so a ring's fold and unfold, whose
-// bins are the same, start from the same pair.
+// at most 16 steps).  A phase by sincospi costs a 64-bit remainder, an FP64
+// division and the polynomial, about a hundred instructions.
 struct PhaseSeq {
     double2 cur, step;
-    // e^{i pi q / n}, 0 <= q < 2 n
-    static __device__ __forceinline__ double2 cis_pi(int q, int n)
+    __device__ __forceinline__ void init(long k0, long D, long n)
     {
-        double s, c;
-        sincospi((double)q / (double)n, &s, &c);
-        return make_double2(c, s);
-    }
-    __device__ __forceinline__ void init(int k0, int D, int n)  // k0 < 2 n
-    {
-        cur = cis_pi(k0, n);
-        step = cis_pi(D % (2 * n), n);
+        cur = cis_pi_frac(k0, n);
+        step = cis_pi_frac(D, n);
     }
     __device__ __forceinline__ double2 next()
     {
@@ -2507,9 +2500,6 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         oS[r] = mdr[r]->ring_ofsS[pr[r]];
     }
 
-    PhaseSeq phase;  // both rings have n samples
-    if (shf[0] || shf[1]) phase.init(tid, NT, n);
-
     if (MODE != kRingAna) {
         // fold, n > L: at most the alias k and the mirror n - k per bin
         double2 e[CNT], o[CNT];
@@ -2517,12 +2507,12 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
             const int L = mdr[r]->L;
-            const double2* rw = reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4);
+            auto rw = gview(reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4));
             const int k = tid + (t - r * CH) * NT;
             const int m = k <= L ? k : n - k;
             if (k <= L || (k >= 1 && n - k <= L)) {
-                e[t] = ld_at(rw, 2 * m);
-                o[t] = ld_at(rw, 2 * m + 1);
+                e[t] = rw[2 * m];
+                o[t] = rw[2 * m + 1];
             }
         }
         PhaseSeq ps;
@@ -2530,9 +2520,9 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
             const int L = mdr[r]->L;
-            const double2* rw = reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4);
+            auto rw = gview(reinterpret_cast<const double2*>(mdr[r]->P + (long)pr[r] * (L + 1) * 4));
             const int k = tid + (t - r * CH) * NT;
-            if (t % CH == 0) ps = phase;
+            if (t % CH == 0 && shf[r]) ps.init(tid, NT, n);
             const double sg = shf[r] ? -1.0 : 1.0;  // (-1)^{j shift} at j = 1
             const double2 ph = shf[r] ? ps.next() : make_double2(1.0, 0.0);
             double2 gN = make_double2(0.0, 0.0), gS = make_double2(0.0, 0.0);
@@ -2543,8 +2533,8 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
                 gS.x += 1.0 * (e[t].x - o[t].x);
                 gS.y += 1.0 * (e[t].y - o[t].y);
                 if (mirror) {
-                    e[t] = ld_at(rw, 2 * (n - k));
-                    o[t] = ld_at(rw, 2 * (n - k) + 1);
+                    e[t] = rw[2 * (n - k)];
+                    o[t] = rw[2 * (n - k) + 1];
                 }
             }
             if (mirror) {
@@ -2577,12 +2567,14 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
+            gcdouble* dd = gview(mdr[r]->d);
+            gcdouble* ww = gview(mdr[r]->w);
             const int j = tid + (t - r * CH) * NT;
-            dN[t] = ld_at(mdr[r]->d + oN[r], j);
-            wN[t] = ld_at(mdr[r]->w + oN[r], j);
+            dN[t] = dd[oN[r] + j];
+            wN[t] = ww[oN[r] + j];
             if (oS[r] >= 0) {
-                dS[t] = ld_at(mdr[r]->d + oS[r], j);
-                wS[t] = ld_at(mdr[r]->w + oS[r], j);
+                dS[t] = dd[oS[r] + j];
+                wS[t] = ww[oS[r] + j];
             }
         }
         double chi[2] = {0.0, 0.0};
@@ -2612,9 +2604,10 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
+            gcdouble* ww = gview(mdr[r]->w);
             const int j = tid + (t - r * CH) * NT;
-            wN[t] = ld_at(mdr[r]->w + oN[r], j);
-            wS[t] = oS[r] >= 0 ? ld_at(mdr[r]->w + oS[r], j) : 0.0;
+            wN[t] = ww[oN[r] + j];
+            wS[t] = oS[r] >= 0 ? ww[oS[r] + j] : 0.0;
         }
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
@@ -2625,12 +2618,13 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
         }
         __syncthreads();
     } else {  // kRingAna
+        gcdouble* in = gview(map_in);
         double2 mv[CNT];
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int r = t / CH;
             const int j = tid + (t - r * CH) * NT;
-            mv[t] = make_double2(ld_at(map_in + oN[r], j), oS[r] >= 0 ? ld_at(map_in + oS[r], j) : 0.0);
+            mv[t] = make_double2(in[oN[r] + j], oS[r] >= 0 ? in[oS[r] + j] : 0.0);
         }
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
@@ -2647,7 +2641,8 @@ __device__ void ring_two(const RingItem& it, const MapDesc* __restrict__ maps, d
     for (int r = 0; r < 2; ++r) {
         const int L = mdr[r]->L;
         double2* qrow = reinterpret_cast<double2*>(mdr[r]->Q + (long)pr[r] * (L + 1) * 4);
-        PhaseSeq ps = phase;
+        PhaseSeq ps;
+        if (shf[r]) ps.init(tid, NT, n);
         for (int k = tid; k < n; k += NT) {
             const double2 ph = shf[r] ? ps.next() : make_double2(1.0, 0.0);
             if (k > L) continue;
@@ -2696,13 +2691,12 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
     const int tid = threadIdx.x;
     constexpr int CNT = (MAXM + NT - 1) / NT;  // ring samples per thread, at most
     gdouble* out = gview(map_out);
+    gcdouble* in = gview(map_in);
+    gcdouble* dd = gview(md.d);
+    gcdouble* ww = gview(md.w);
     // for n < NT the aliases of each bin are split over R thread
     // groups (reads stay coalesced over k), partial sums added in fixed order
     const int R = n < NT ? NT / n : 1;
-    // e^{i pi k/n} of the thread's bins (R > 1: of its one bin)
-    const int k1 = R > 1 ? tid % n : tid;
-    PhaseSeq phase;
-    if (shifted) phase.init(k1, NT, n);
 
     if (MODE != kRingAna) {
         const double2* row = reinterpret_cast<const double2*>(md.P + (long)p * (L + 1) * 4);
@@ -2712,18 +2706,20 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
             // per bin, and both only where n - L <= k <= L: one load per bin
             // issued for every bin of the thread before the sums, the rare
             // second one where the sums need it
+            auto rw = gview(row);
             double2 e[CNT], o[CNT];
 #pragma unroll
             for (int t = 0; t < CNT; ++t) {
                 const int k = tid + t * NT;
                 const int m = k <= L ? k : n - k;
                 if (k < n && (k <= L || (k >= 1 && n - k <= L))) {
-                    e[t] = ld_at(row, 2 * m);
-                    o[t] = ld_at(row, 2 * m + 1);
+                    e[t] = rw[2 * m];
+                    o[t] = rw[2 * m + 1];
                 }
             }
             const double sg = shifted ? -1.0 : 1.0;  // (-1)^{j shift} at j = 1
-            PhaseSeq ps = phase;
+            PhaseSeq ps;
+            if (shifted) ps.init(tid, NT, n);
 #pragma unroll
             for (int t = 0; t < CNT; ++t) {
                 const int k = tid + t * NT;
@@ -2737,8 +2733,8 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
                     gS.x += 1.0 * (e[t].x - o[t].x);
                     gS.y += 1.0 * (e[t].y - o[t].y);
                     if (mirror) {
-                        e[t] = ld_at(row, 2 * (n - k));
-                        o[t] = ld_at(row, 2 * (n - k) + 1);
+                        e[t] = rw[2 * (n - k)];
+                        o[t] = rw[2 * (n - k) + 1];
                     }
                 }
                 if (mirror) {
@@ -2750,7 +2746,8 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
                 fold_store(Z, k, ph, shifted, oS < 0, gN, gS);
             }
         } else if (R == 1) {
-            PhaseSeq ps = phase;
+            PhaseSeq ps;
+            if (shifted) ps.init(tid, NT, n);
             for (int k = tid; k < n; k += NT) {
                 double2 gN, gS;
                 fold_aliases(row, L, n, k, 0, 1, shifted, gN, gS);
@@ -2759,7 +2756,7 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
         } else {
             double2 gN = make_double2(0.0, 0.0), gS = make_double2(0.0, 0.0);
             if (tid < R * n) {
-                fold_aliases(row, L, n, k1, tid / n, R, shifted, gN, gS);
+                fold_aliases(row, L, n, tid % n, tid / n, R, shifted, gN, gS);
                 Z[zp(2 * tid)] = gN;
                 Z[zp(2 * tid + 1)] = gS;
             }
@@ -2774,7 +2771,7 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
             }
             __syncthreads();
             if (tid < n)
-                fold_store(Z, tid, phase.cur, shifted, oS < 0, gN, gS);
+                fold_store(Z, tid, shifted ? cis_pi_frac(tid, n) : make_double2(1.0, 0.0), shifted, oS < 0, gN, gS);
         }
         __syncthreads();
         ring_dft<+1, MAXM>(Z, n, M, logM, pow2, chirp, filt, tw);
@@ -2796,11 +2793,11 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
         for (int t = 0; t < CNT; ++t) {
             const int j = tid + t * NT;
             if (j < n) {
-                dN[t] = ld_at(md.d + oN, j);
-                wN[t] = ld_at(md.w + oN, j);
+                dN[t] = dd[oN + j];
+                wN[t] = ww[oN + j];
                 if (oS >= 0) {
-                    dS[t] = ld_at(md.d + oS, j);
-                    wS[t] = ld_at(md.w + oS, j);
+                    dS[t] = dd[oS + j];
+                    wS[t] = ww[oS + j];
                 }
             }
         }
@@ -2829,8 +2826,8 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
         for (int t = 0; t < CNT; ++t) {
             const int j = tid + t * NT;
             if (j < n) {
-                wN[t] = ld_at(md.w + oN, j);
-                wS[t] = oS >= 0 ? ld_at(md.w + oS, j) : 0.0;
+                wN[t] = ww[oN + j];
+                wS[t] = oS >= 0 ? ww[oS + j] : 0.0;
             }
         }
 #pragma unroll
@@ -2846,7 +2843,7 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
             const int j = tid + t * NT;
-            if (j < n) mv[t] = make_double2(ld_at(map_in + oN, j), oS >= 0 ? ld_at(map_in + oS, j) : 0.0);
+            if (j < n) mv[t] = make_double2(in[oN + j], oS >= 0 ? in[oS + j] : 0.0);
         }
 #pragma unroll
         for (int t = 0; t < CNT; ++t) {
@@ -2860,17 +2857,20 @@ __global__ __launch_bounds__(ring_threads(MAXM), MAXM > 4096 ? 1 : 4) void k_rin
     // unfold, with the aliases of bin k split over R thread groups as in the fold
     double2* qrow = reinterpret_cast<double2*>(md.Q + (long)p * (L + 1) * 4);
     if (R == 1) {
+        PhaseSeq ps;
+        if (shifted) ps.init(tid, NT, n);
         for (int k = tid; k < n; k += NT) {
-            const double2 ph = shifted ? phase.next() : make_double2(1.0, 0.0);
+            const double2 ph = shifted ? ps.next() : make_double2(1.0, 0.0);
             if (k > L) continue;
             const int nk = (k == 0) ? 0 : n - k;
             unfold_bin(qrow, L, n, k, 0, 1, shifted, ph, Z[zp(k)], Z[zp(nk)]);
         }
     } else if (tid < R * n) {  // R n <= NT: one (bin, group) per thread
-        const int k = k1, r = tid / n;
+        const int k = tid % n, r = tid / n;
         if (k <= L) {
             const int nk = (k == 0) ? 0 : n - k;
-            unfold_bin(qrow, L, n, k, r, R, shifted, phase.cur, Z[zp(k)], Z[zp(nk)]);
+            unfold_bin(qrow, L, n, k, r, R, shifted, shifted ? cis_pi_frac(k, n) : make_double2(1.0, 0.0), Z[zp(k)],
+                       Z[zp(nk)]);
         }
     }
 }
