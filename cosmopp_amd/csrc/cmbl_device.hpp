@@ -7,6 +7,16 @@
 
 namespace cmbl {
 
+// A wave-uniform value that the kernel itself stores to later.  A plain load of
+// it may become a scalar load, which is not ordered with the wave's vector
+// stores: a store issued after it can reach memory first.  Atomic loads go
+// through vector memory, in order with them.
+template <class T>
+__device__ __forceinline__ T load_before_store(const T* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // Lanes 0..31 get a summed over lanes (j, j + 32), lanes 32..63 get b summed
 // likewise (v_permlane32_swap exchanges lanes 32..63 of its first operand
 // with lanes 0..31 of its second).

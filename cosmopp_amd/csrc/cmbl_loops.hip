@@ -280,8 +280,11 @@ struct OpHistory {
     }
     __device__ void finish(const double* r)
     {
-        const int k = d.slot[d.m - 1];
-        for (int i = d.m - 1; i > 0; --i) d.slot[i] = d.slot[i - 1];
+        // (with k by a scalar load the rotation's first store sometimes passed
+        // it: k was then slot[m - 2], one slot was held twice from there on and
+        // one lost, and directions with enough pairs were wrong)
+        const int k = load_before_store(d.slot + d.m - 1);
+        for (int i = d.m - 1; i > 0; --i) d.slot[i] = load_before_store(d.slot + i - 1);
         d.slot[0] = k;
         const double ys = r[0];
         double yy = sqrt(r[1]);
