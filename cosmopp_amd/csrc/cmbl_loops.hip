@@ -744,7 +744,9 @@ void cmbl_lbfgs_destroy(cmbl_lbfgs* lb)
 int cmbl_lbfgs_set_starting(cmbl_lbfgs* lb, const double* d_x0)
 {
     if (!lb || !d_x0) return fail(CMBL_ERR_ARG, "null pointer");
-    CMBL_HIP(hipStreamSynchronize(lb->stream));
+    // as at creation: the caller's x0 may still be in flight on its streams,
+    // with which this context's stream does not order
+    CMBL_HIP(hipDeviceSynchronize());
     CMBL_HIP(hipMemcpyAsync(lb->d.x, d_x0, sizeof(double) * lb->n, hipMemcpyDeviceToDevice, lb->stream));
     return lb_start(lb);
 }

@@ -75,3 +75,26 @@ def test_directions(nside, lmax, graphs):
         assert f == ends[0][0] and np.array_equal(x, ends[0][1])
     lb.close()
     mp.close()
+
+
+@pytest.mark.parametrize("side", [False, True])
+def test_set_starting_waits_for_the_callers_stream(side):
+    """A point still being written on the caller's stream: the value at the start
+    is that of the finished point."""
+    import torch
+
+    print("case lbfgs set_starting in flight", side, flush=True)
+    c = Case(16, 32, 5400.0 / 32 / 60.0, 20.0, 20.0, seed=5)
+    mp = c.make_map()
+    want, _ = mp.value_and_grad(c.x)
+    x1 = torch.from_numpy(c.x).to("cuda:0")
+    x0 = torch.zeros_like(x1)
+    lb = cm.LBFGS(mp, x0.data_ptr(), m=M)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream() if side else torch.cuda.current_stream()):
+        torch.cuda._sleep(20_000_000)  # about 10 ms
+        x0.copy_(x1)
+        lb.set_starting(x0.data_ptr())
+    assert lb.state()["f"] == want
+    lb.close()
+    mp.close()
