@@ -67,8 +67,9 @@ __device__ __forceinline__ void for_each_map(std::integer_sequence<int, I...>, F
 
 // acc += c x (or -= c x), c taken from lane N of the lane's row of 16.  The
 // rows hold the same 16 coefficients, so one register pair feeds 16 steps.  A
-// DPP operand must not have been written by the VALU in the last two
-// instructions: coefficients come straight from memory.
+// DPP operand must not have been written by the VALU in the last two wait
+// states, which the compiler does not see to for operands of an asm: every c
+// passes dpp_ready() after its last copy and before its first use.
 template <int N, bool NEG>
 __device__ __forceinline__ void fmac_row(double& acc, double c, double x)
 {
@@ -77,6 +78,8 @@ __device__ __forceinline__ void fmac_row(double& acc, double c, double x)
     else
         asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(N));
 }
+
+__device__ __forceinline__ void dpp_ready(double& c) { asm volatile("s_nop 1" : "+v"(c)); }
 
 // Global-address-space views of device memory: loads and stores through them
 // compile to global_* instructions (counted by vmcnt only) rather than flat_*
@@ -558,8 +561,7 @@ __global__ __launch_bounds__(64 * kCoupD, 3) void k_coupling(int L, const double
             // past L the weight is zero, and so is F whatever the tables hold
             double F = f * (hA[t + j] * hB[w + t + j]);
             f = t + 16 < ne ? weight(t + 16 + j) : 0.0;
-            // two wait states between the VALU write and the first DPP read
-            asm volatile("s_nop 1" : "+v"(F));
+            dpp_ready(F);
             const int q = (t0 + t - b) / kCoupR;
             if (t0 + t < b)
                 coupling_steps<false>(acc, end, hv, kv, F, hC, ho, kD, ko, q, lane);
@@ -821,6 +823,7 @@ __device__ __forceinline__ void syn_block(SynState<K>& st, SynAcc<K> (&ac)[G], c
                                           scdouble* const (&a)[G], long o, double (&xr)[G][NS], double (&xi)[G][NS])
 {
     double yr[G][NS], yi[G][NS];
+    dpp_ready(A);
     if constexpr (NS == 8) {
         syn_group<K, G, P1, 0, NS>(st, ac, xa, A, xr, xi, a, o + 8, yr, yi);
         if (SCALED) syn_rescale<K, G>(st, ac);
@@ -976,12 +979,16 @@ struct PolRow {
 #pragma unroll
         for (int i = 0; i < kPolRec; ++i) c[i] = R[(long)l * kPolRec + i];
     }
-    // two wait states between these VALU writes and the first DPP read
+    // to be called before a row's first use (the c may just have been copied)
     __device__ __forceinline__ void ready(int l, double m2)
     {
         const double fl = l;
         e = fl - m2;
         h = 0.5 * (fl * (fl - 1.0));
+#pragma unroll
+        for (int i = 0; i < kPolRec; i += 7)
+            asm volatile("" : "+v"(c[i]), "+v"(c[i + 1]), "+v"(c[i + 2]), "+v"(c[i + 3]), "+v"(c[i + 4]),
+                              "+v"(c[i + 5]), "+v"(c[i + 6]));
         asm volatile("s_nop 1" : "+v"(A), "+v"(e), "+v"(h));
     }
 };

@@ -4,6 +4,10 @@ up in the compiler's assembly of the loop and sampler kernels.
 A scalar load and a later vector store of one wave are not ordered with each
 other.  Where a kernel may write what it reads, no scalar load other than of the
 kernel's arguments may therefore be outstanding at a store.
+
+A DPP operand must not have been written by the VALU in the last two wait states.
+The compiler sees to it for its own instructions, not for those in inline asm
+(row_newbcast): there an s_nop has to stand between, whatever else happens to.
 """
 import os
 import re
@@ -100,3 +104,49 @@ def test_no_scalar_load_outstanding_at_a_store(source, tmp_path):
     assert found
     bad = {k: v for k, v in ((k, loads_at_stores(*f)) for k, f in found.items()) if v}
     assert not bad, bad
+
+
+def mask(regs):
+    return sum(1 << i for kind, i in regs if kind == "v")
+
+
+def unguarded_rows(ins, succ):
+    """row_newbcast instructions whose DPP operand may come from the VALU with no s_nop of two wait states or more
+    since (a bit per register written by the VALU, followed along every path)."""
+    state, work, bad = {0: 0}, [0], set()
+    while work:
+        i = work.pop()
+        s, out = ins[i], state[i]
+        ops = [o.strip() for o in s.split(None, 1)[1].split(",")] if " " in s else []
+        if "row_newbcast" in s and out & mask(registers(ops[1].lstrip("-").split()[0])):
+            bad.add(s)
+        nop = re.match(r"s_nop\s+(\d+)", s)
+        if nop and int(nop.group(1)) >= 1:
+            out = 0
+        elif s.startswith("v_") and ops:
+            out |= mask(registers(ops[0].split()[0]))
+            if "swap" in s:
+                out |= mask(registers(ops[1].split()[0]))
+        elif s.startswith(("global_load", "ds_read", "flat_load")):
+            out &= ~mask(registers(ops[0].split()[0]))
+        for j in succ[i]:
+            new = state.get(j, 0) | out
+            if j not in state or new != state[j]:
+                state[j] = new
+                work.append(j)
+    return sorted(bad)
+
+
+def test_the_row_check_itself():
+    use = " v_fmac_f64_dpp v[0:1], v[2:3], v[4:5] row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+    far = " v_mov_b64_e32 v[6:7], 0\n" * 9
+    for body, n in ((" v_mov_b64_e32 v[2:3], v[8:9]\n" + far, 1), (" v_mov_b64_e32 v[2:3], v[8:9]\n s_nop 1\n", 0),
+                    (" v_mov_b64_e32 v[2:3], v[8:9]\n global_load_dwordx2 v[2:3], v[8:9], off\n", 0)):
+        assert len(unguarded_rows(*kernels("_Zk: ; @k\n" + body + use + " s_endpgm\n.Lfunc_end0:\n")["_Zk"])) == n
+
+
+def test_row_coefficients_are_guarded(tmp_path):
+    found = assembly("cmbl_kernels.hip", tmp_path)
+    rows = sum("row_newbcast" in s for ins, _ in found.values() for s in ins)
+    bad = {k: v for k, v in ((k, unguarded_rows(*f)) for k, f in found.items()) if v}
+    assert rows > 1000 and not bad, {k: (len(v), v[:2]) for k, v in bad.items()}
