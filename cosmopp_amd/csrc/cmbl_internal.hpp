@@ -254,11 +254,10 @@ struct AdjCost {
     AdjItem it;
     double cost;
 };
-// Set-up of one group of 64 ring pairs from p0: its state at row start l.
+// Set-up of one group of 64 ring pairs from p0: entry `at` of the state buffers
+// (64 values each) takes its state of degree m at row start l.
 struct AdjCap {
-    double2* st;
-    int* sk;
-    int m, p0, l, pad_;
+    int at, m, p0, l;
 };
 
 // A ring pair of a map; with pair2 >= 0 also a second ring pair (of map2) of
@@ -365,7 +364,8 @@ int launch_post_batch(const MapDesc* d_mds, const BatchArgs& a, int mode, hipStr
 int launch_final_batch(const MapDesc* d_mds, const BatchArgs& a, hipStream_t s);
 int launch_bluestein_setup(const MapDesc* d_md, const int* d_pairs, int npairs_bs, double2* d_out,
                            double2* d_chirp, int lds_bytes, const double2* d_tw, hipStream_t s);
-int launch_adj_capture(const AdjCap* caps, int n, const MapDesc* d_md, hipStream_t s);
+int launch_adj_capture(const AdjCap* caps, const int* runs, int nruns, double2* st, int* sk, const MapDesc* d_md,
+                       hipStream_t s);
 int launch_scan(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, int* d_lstart,
                 hipStream_t s);
 int launch_capture(int K, const WorkItem* items, int nitems, const MapDesc* d_maps, double* d_prev, double* d_cur,
@@ -408,7 +408,6 @@ struct cmbl_map {
     std::vector<int> ring_two;  // n for power-of-two unsplit pairs with n > lmax (two may share a workgroup), else 0
     std::vector<cmbl::WorkItem> items1;      // launch order (XCD-interleaved)
     std::vector<cmbl::ItemCost> cost1;       // live items with cost estimates
-    std::vector<cmbl::AdjCost> cost5;
     std::vector<int> lmin64;      // first live l (L + 1: none) per m and 64 ring pairs
     std::vector<cmbl::RingItem> ring_items;
     double2* d_tw = nullptr;

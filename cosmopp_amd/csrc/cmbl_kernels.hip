@@ -1919,31 +1919,35 @@ __global__ __launch_bounds__(64) void k_capture(const WorkItem* __restrict__ ite
     }
 }
 
-// k_adj_capture: the adjoint's start state of 64 ring pairs of degree m at row
-// start l (even l - m): (mu_{l-2}, mu_{l-1}) and the scale count; (-mu_m, 0) at
-// l = m, from which the first step gives mu_m.
-__global__ __launch_bounds__(64) void k_adj_capture(const AdjCap* __restrict__ caps, const MapDesc* __restrict__ md_)
+// k_adj_capture: the adjoint's start states of 64 ring pairs of degree m at the
+// row starts l (even l - m) of a run of entries, by l: (mu_{l-2}, mu_{l-1}) and
+// the scale count; (-mu_m, 0) at l = m, from which the first step gives mu_m.
+// The recurrence runs once for the run (its entries are the segments of one
+// group; once for each of them, from l = m, took up to eight times the steps).
+__global__ __launch_bounds__(64) void k_adj_capture(const AdjCap* __restrict__ caps, const int* __restrict__ runs,
+                                                    double2* __restrict__ st, int* __restrict__ sk,
+                                                    const MapDesc* __restrict__ md_)
 {
-    const AdjCap c = caps[blockIdx.x];
     const MapDesc& md = *md_;
-    const int L = md.L, m = c.m;
+    const int i0 = runs[blockIdx.x], i1 = runs[blockIdx.x + 1];
+    const int L = md.L, m = caps[i0].m, p = caps[i0].p0 + threadIdx.x;
     const double* __restrict__ A = md.A + moff(L, m) - m;
-    const int p = c.p0 + threadIdx.x;
     LegState<1> s;
     const double x[1] = {md.ring_x[p]};
     s.mu1[0] = md.seed_v[(long)m * md.npair_pad + p];
     s.sc[0] = md.seed_k[(long)m * md.npair_pad + p];
     s.mu2[0] = 0.0;
-    if (c.l == m) {
-        s.mu2[0] = -s.mu1[0];
-        s.mu1[0] = 0.0;
+    int l = m + 1;
+    for (int i = i0; i < i1; ++i) {
+        const AdjCap c = caps[i];
+        for (; l < c.l; ++l) {
+            capture_step<1>(s, x, ((l - m) & 1) != 0, A[l]);
+            rescale<1>(s.mu1, s.mu2, s.sc);
+        }
+        const long q = 64L * c.at + threadIdx.x;
+        st[q] = c.l == m ? make_double2(-s.mu1[0], 0.0) : make_double2(s.mu2[0], s.mu1[0]);
+        sk[q] = s.sc[0];
     }
-    for (int l = m + 1; l < c.l; ++l) {
-        capture_step<1>(s, x, ((l - m) & 1) != 0, A[l]);
-        rescale<1>(s.mu1, s.mu2, s.sc);
-    }
-    c.st[threadIdx.x] = make_double2(s.mu2[0], s.mu1[0]);
-    c.sk[threadIdx.x] = s.sc[0];
 }
 
 // ================================================================== ring stage
@@ -3355,10 +3359,11 @@ int launch_capture(int K, const WorkItem* items, int n, const MapDesc* d_maps, d
     return fail(CMBL_ERR_ARG, "unsupported rings-per-lane K");
 }
 
-int launch_adj_capture(const AdjCap* caps, int n, const MapDesc* d_md, hipStream_t s)
+int launch_adj_capture(const AdjCap* caps, const int* runs, int nruns, double2* st, int* sk, const MapDesc* d_md,
+                       hipStream_t s)
 {
-    if (n <= 0) return CMBL_OK;
-    hipLaunchKernelGGL(k_adj_capture, dim3(n), dim3(64), 0, s, caps, d_md);
+    if (nruns <= 0) return CMBL_OK;
+    hipLaunchKernelGGL(k_adj_capture, dim3(nruns), dim3(64), 0, s, caps, runs, st, sk, d_md);
     CMBL_HIP(hipGetLastError());
     return CMBL_OK;
 }

@@ -139,21 +139,17 @@ static int dupload(cmbl_map* mp, T** p, const std::vector<T>& h)
 // step, K rings.
 static const int kXcds = 8;
 
-static void build_items(const cmbl_map* mp, int K, const std::vector<int>& lstart, int map_index,
+static void build_items(const cmbl_map* mp, int K, const std::vector<int>& lmax64, int map_index,
                         std::vector<ItemCost>* out)
 {
-    const int L = mp->L;
-    const int npad = mp->npair_pad;
-    const int nrb = npad / (64 * K);
-    for (int rb = 0; rb < nrb; ++rb) {
+    const int L = mp->L, n64 = mp->npair_pad / 64;
+    for (int rb = 0; rb < n64 / K; ++rb) {
         for (int m = 0; m <= L; ++m) {
             int lmin = L + 1, lmax = -1;
-            for (int j = 0; j < 64 * K; ++j) {
-                const int v = lstart[(size_t)m * npad + rb * 64 * K + j];
-                if (v <= L) {
-                    lmin = std::min(lmin, v);
-                    lmax = std::max(lmax, v);
-                }
+            for (int k = 0; k < K; ++k) {
+                const size_t u = (size_t)m * n64 + rb * K + k;
+                lmin = std::min(lmin, mp->lmin64[u]);
+                lmax = std::max(lmax, lmax64[u]);
             }
             if (lmin > L) continue;
             const double cost = K * (3.0 * (lmax - lmin) + 4.0 * (L - lmax + 1)) + 64.0 * K;
@@ -162,43 +158,63 @@ static void build_items(const cmbl_map* mp, int K, const std::vector<int>& lstar
     }
 }
 
-// Longest segment (l-steps, a multiple of 8) of a launch of `live` whole
-// items: enough items for three rounds of two waves per SIMD, but no segments
-// under 64 steps, where an item's fixed part (its loads, about two
-// microseconds) would outweigh its rows.
+// Adjoint items of a map's geometry with K ring pairs per lane (state
+// addresses as indices until fill_adj; map, Q and u set by adj_for).  One item
+// per live (m, block of 64 K ring pairs), cut along l into segments of at most
+// `seg` steps where a launch has too few items to fill the chip: the outputs
+// are per l, so the segments of one (m, block) write disjoint parts of its row.
+// Each group of 64 pairs joins at the row of its first live l.
+//
+// Longest segment (a multiple of 8) where a launch has `live` whole items:
+// enough items for three rounds of two waves per SIMD, but no segments under 64
+// steps, where an item's fixed part (its loads, about two microseconds) would
+// outweigh its rows.
+static int adj_whole(int L) { return (L + 16) / 8 * 8; }
 static int adj_segment(size_t live, int L)
 {
     const size_t want = 3 * 2048;
-    if (live >= want) return (L + 16) / 8 * 8;
+    if (live >= want) return adj_whole(L);
     const long len = (long)(L / 2 + 1) * (long)live / (long)want;
     return std::max(64, (int)((len + 63) / 64 * 64));
 }
 
-// Adjoint items of a map's geometry with K ring pairs per lane (state
-// addresses as indices until fill_adj; map, Q and u set by adj_for).  One item
-// per live (m, block of 64 K ring pairs), cut along l into segments (unless
-// `whole`) where there are too few items to fill the chip: the outputs are per
-// l, so the segments of one (m, block) write disjoint parts of its row.
-// Each group of 64 pairs joins at the row of its first live l.
-static void build_adj(const cmbl_map* mp, int K, bool whole, std::vector<AdjCost>* out, std::vector<AdjCap>* caps)
+// The start states to form: a run of entries per (m, 64 ring pairs), by l.
+struct AdjCaps {
+    std::vector<AdjCap> cap;
+    std::vector<int> run;  // first entry of each run
+};
+
+static int adj_blocks(const cmbl_map* mp, int K) { return (mp->npair + 64 * K - 1) / (64 * K); }
+
+// First live l of degree m in block b of 64 K ring pairs (L + 1: none).
+static int adj_first(const cmbl_map* mp, int K, int m, int b)
+{
+    const int n64 = mp->npair_pad / 64;
+    int f = mp->L + 1;
+    for (int k = 0; k < K && b * K + k < n64; ++k) f = std::min(f, mp->lmin64[(size_t)m * n64 + b * K + k]);
+    return f;
+}
+
+// Live (m, block) items of a map.
+static size_t adj_live(const cmbl_map* mp, int K)
+{
+    size_t live = 0;
+    for (int m = 0; m <= mp->L; ++m)
+        for (int b = 0; b < adj_blocks(mp, K); ++b) live += adj_first(mp, K, m, b) <= mp->L;
+    return live;
+}
+
+static void build_adj(const cmbl_map* mp, int K, int seg, std::vector<AdjCost>* out, AdjCaps* caps)
 {
     const int L = mp->L, n64 = mp->npair_pad / 64;
     // blocks of the real ring pairs only
-    const int nb = (mp->npair + 64 * K - 1) / (64 * K);
-    std::vector<int> first((size_t)nb * (L + 1), L + 1);
-    size_t live = 0;
+    const int nb = adj_blocks(mp, K);
     for (int b = 0; b < nb; ++b)
         for (int m = 0; m <= L; ++m) {
-            int& f = first[(size_t)b * (L + 1) + m];
-            for (int k = 0; k < K && b * K + k < n64; ++k) f = std::min(f, mp->lmin64[(size_t)m * n64 + b * K + k]);
-            live += f <= L;
-        }
-    const int seg = whole ? (L + 16) / 8 * 8 : adj_segment(live, L);
-    for (int b = 0; b < nb; ++b)
-        for (int m = 0; m <= L; ++m) {
-            const int lf = first[(size_t)b * (L + 1) + m];
+            const int lf = adj_first(mp, K, m, b);
             if (lf > L) continue;
             const int lb = lf - ((lf - m) & 1);  // rows start at even l - m
+            const size_t at = caps->cap.size();
             for (int l0 = lb; l0 <= L; l0 += seg) {
                 AdjItem it{};
                 it.A = mp->desc.A + (moff(L, m) - m);
@@ -212,9 +228,9 @@ static void build_adj(const cmbl_map* mp, int K, bool whole, std::vector<AdjCost
                 it.lend = std::min(L, l0 + seg - 1);
                 it.part = b;
                 it.seg = (l0 - lb) / seg;
-                const size_t at = caps->size() * 64;
-                it.st = reinterpret_cast<const double2*>(at * sizeof(double2));
-                it.sk = reinterpret_cast<const int*>(at * sizeof(int));
+                const size_t slot = (at + (size_t)it.seg * K) * 64;
+                it.st = reinterpret_cast<const double2*>(slot * sizeof(double2));
+                it.sk = reinterpret_cast<const int*>(slot * sizeof(int));
                 double cost = 300.0;
                 int top = it.nrow;
                 for (int k = 0; k < K; ++k) {
@@ -226,22 +242,32 @@ static void build_adj(const cmbl_map* mp, int K, bool whole, std::vector<AdjCost
                     row = top;
                     it.row[k] = (unsigned short)row;
                     cost += 28.0 * (it.nrow - row);
-                    // a group that never joins gets a state too (unused)
-                    caps->push_back(AdjCap{nullptr, nullptr, m, std::min(u, n64 - 1) * 64,
-                                           row < it.nrow ? l0 + 8 * row : m, 0});
                 }
                 cost += 60.0 * (it.nrow - top);
                 // rows before the first group's are not run
                 out->push_back(AdjCost{it, cost});
             }
+            // the start states of a group in its segments, by l; one that does
+            // not join in a segment gets a state too (unused)
+            const size_t ns = (size_t)((L - lb) / seg + 1), i0 = out->size() - ns;
+            for (int k = 0; k < K; ++k) {
+                const int p0 = std::min(b * K + k, n64 - 1) * 64;
+                caps->run.push_back((int)caps->cap.size());
+                for (size_t j = 0; j < ns; ++j) {
+                    const AdjItem& it = (*out)[i0 + j].it;
+                    const int row = it.row[k];
+                    caps->cap.push_back(AdjCap{(int)(at + j * K + k), m, p0, row < it.nrow ? it.l0 + 8 * row : m});
+                }
+            }
         }
 }
 
-// Allocates and fills the start states of build_adj's items (their st and sk
-// become pointers); the buffers are appended to allocs.
-static int fill_adj(const cmbl_map* mp, std::vector<AdjCost>* items, std::vector<AdjCap>* caps, std::vector<void*>* allocs)
+// Allocates and starts to fill the start states of build_adj's items (their st
+// and sk become pointers); the buffers are appended to allocs.  The caller waits
+// for the device before the items are used.
+static int fill_adj(const cmbl_map* mp, std::vector<AdjCost>* items, AdjCaps* caps, std::vector<void*>* allocs)
 {
-    const size_t n = std::max<size_t>(caps->size(), 1) * 64;
+    const size_t n = std::max<size_t>(caps->cap.size(), 1) * 64;
     void *ps = nullptr, *pk = nullptr, *dc = nullptr;
     CMBL_HIP(hipMalloc(&ps, n * sizeof(double2)));
     allocs->push_back(ps);
@@ -251,19 +277,16 @@ static int fill_adj(const cmbl_map* mp, std::vector<AdjCost>* items, std::vector
         c.it.st = reinterpret_cast<const double2*>((char*)ps + reinterpret_cast<size_t>(c.it.st));
         c.it.sk = reinterpret_cast<const int*>((char*)pk + reinterpret_cast<size_t>(c.it.sk));
     }
-    for (size_t i = 0; i < caps->size(); ++i) {
-        (*caps)[i].st = (double2*)ps + i * 64;
-        (*caps)[i].sk = (int*)pk + i * 64;
-    }
-    if (caps->empty()) return CMBL_OK;
-    CMBL_HIP(hipMalloc(&dc, caps->size() * sizeof(AdjCap)));
-    int rc = CMBL_OK;
-    if (hipMemcpy(dc, caps->data(), caps->size() * sizeof(AdjCap), hipMemcpyHostToDevice) != hipSuccess)
-        rc = fail(CMBL_ERR_HIP, "adjoint set-up");
-    if (rc == CMBL_OK) rc = launch_adj_capture((const AdjCap*)dc, (int)caps->size(), mp->d_desc, nullptr);
-    if (rc == CMBL_OK && hipDeviceSynchronize() != hipSuccess) rc = fail(CMBL_ERR_HIP, "adjoint set-up");
-    (void)hipFree(dc);
-    return rc;
+    if (caps->cap.empty()) return CMBL_OK;
+    const int runs = (int)caps->run.size();
+    caps->run.push_back((int)caps->cap.size());
+    const size_t bc = caps->cap.size() * sizeof(AdjCap), br = caps->run.size() * sizeof(int);
+    CMBL_HIP(hipMalloc(&dc, bc + br));
+    allocs->push_back(dc);  // freed with the others: a hipFree here waits for the device
+    CMBL_HIP(hipMemcpy(dc, caps->cap.data(), bc, hipMemcpyHostToDevice));
+    CMBL_HIP(hipMemcpy((char*)dc + bc, caps->run.data(), br, hipMemcpyHostToDevice));
+    return launch_adj_capture((const AdjCap*)dc, (const int*)((char*)dc + bc), runs, (double2*)ps, (int*)pk, mp->d_desc,
+                              nullptr);
 }
 
 // A geometry's adjoint item for map `index` of its list.
@@ -283,67 +306,69 @@ static AdjCost adj_for(AdjCost c, int index, const MapDesc& d)
 // Items that stay together: the synthesis' quads of m (they write parts of the
 // same lines: nside 512 88 -> 82 us); the adjoint's items each on their own
 // (its reads are spread over the whole item: together 109, by cost 105 us).
-static std::tuple<int, int, int> item_quad(const WorkItem& it) { return {it.map, it.m0 >> 2, it.rb}; }
-static std::tuple<int, int, int> item_quad(const AdjItem& it) { return {it.map, it.m0, it.part << 16 | it.seg}; }
+// (map, m or its quad, block and segment) of an item; items of one key stay together.
+static unsigned long item_key(int map, int m, int rest)
+{
+    return (unsigned long)map << 46 | (unsigned long)m << 32 | (unsigned)rest;
+}
+static unsigned long item_quad(const WorkItem& it) { return item_key(it.map, it.m0 >> 2, it.rb); }
+static unsigned long item_quad(const AdjItem& it) { return item_key(it.map, it.m0, it.part << 16 | it.seg); }
 
 template <typename Cost>
 static auto order_items(const std::vector<Cost>& v)
 {
     std::vector<decltype(Cost::it)> out;
     if (v.empty()) return out;
-    std::vector<std::pair<long, double>> groups;  // (key, cost)
-    std::vector<long> keys(v.size());
-    {
-        std::vector<std::pair<long, size_t>> kv;
-        for (size_t i = 0; i < v.size(); ++i) {
-            keys[i] = ((long)v[i].it.map << 32) | (long)(v[i].it.m0 >> 2);
-            kv.push_back({keys[i], i});
-        }
-        std::sort(kv.begin(), kv.end());
-        for (size_t i = 0; i < kv.size(); ++i) {
-            if (groups.empty() || groups.back().first != kv[i].first) groups.push_back({kv[i].first, 0.0});
-            groups.back().second += v[kv[i].second].cost;
-        }
+    // items by map and quad of m, and these groups' costs
+    std::vector<std::pair<long, unsigned>> kv(v.size());
+    for (size_t i = 0; i < v.size(); ++i) kv[i] = {(long)v[i].it.map << 32 | (long)(v[i].it.m0 >> 2), (unsigned)i};
+    std::sort(kv.begin(), kv.end());
+    struct Group {
+        double cost;
+        size_t first, end;
+    };
+    std::vector<Group> groups;
+    for (size_t i = 0; i < kv.size(); ++i) {
+        if (i == 0 || kv[i].first != kv[i - 1].first) groups.push_back(Group{0.0, i, i});
+        groups.back().cost += v[kv[i].second].cost;
+        groups.back().end = i + 1;
     }
-    std::sort(groups.begin(), groups.end(),
-              [](const std::pair<long, double>& a, const std::pair<long, double>& b) { return a.second > b.second; });
-    std::vector<double> load(kXcds, 0.0);
-    std::vector<std::pair<long, int>> assign;
-    for (const auto& g : groups) {
-        const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        load[x] += g.second;
-        assign.push_back({g.first, x});
-    }
-    std::sort(assign.begin(), assign.end());
-    std::vector<std::vector<Cost>> lists(kXcds);
-    for (size_t i = 0; i < v.size(); ++i) {
-        const auto itx = std::lower_bound(assign.begin(), assign.end(), std::make_pair(keys[i], -1));
-        lists[itx->second].push_back(v[i]);
+    std::sort(groups.begin(), groups.end(), [](const Group& a, const Group& b) {
+        return a.cost != b.cost ? a.cost > b.cost : a.first < b.first;
+    });
+    // an XCD's items as (key, m, index), then by the largest cost of the items that stay together
+    struct Entry {
+        double top;
+        unsigned long key;
+        unsigned m, i;
+    };
+    double load[kXcds] = {};
+    std::vector<Entry> lists[kXcds];
+    for (const Group& g : groups) {
+        const int x = (int)(std::min_element(load, load + kXcds) - load);
+        load[x] += g.cost;
+        for (size_t j = g.first; j < g.end; ++j) {
+            const unsigned i = kv[j].second;
+            lists[x].push_back(Entry{v[i].cost, item_quad(v[i].it), (unsigned)v[i].it.m0, i});
+        }
     }
     size_t len = 0;
     for (auto& l : lists) {
-        // by the largest cost of the items that stay together
-        auto quad = [](const Cost& c) { return item_quad(c.it); };
-        std::map<decltype(quad(l[0])), double> top;
-        for (const Cost& c : l) {
-            double& t = top[quad(c)];
-            t = std::max(t, c.cost);
+        auto by_key = [](const Entry& a, const Entry& b) {
+            return a.key != b.key ? a.key < b.key : a.m != b.m ? a.m < b.m : a.i < b.i;
+        };
+        std::sort(l.begin(), l.end(), by_key);
+        for (size_t i = 0, j; i < l.size(); i = j) {
+            double top = 0.0;
+            for (j = i; j < l.size() && l[j].key == l[i].key; ++j) top = std::max(top, l[j].top);
+            for (size_t k = i; k < j; ++k) l[k].top = top;
         }
-        std::vector<std::pair<double, size_t>> order;
-        for (size_t i = 0; i < l.size(); ++i) order.push_back({top[quad(l[i])], i});
-        std::sort(order.begin(), order.end(), [&](const auto& a, const auto& b) {
-            if (a.first != b.first) return a.first > b.first;
-            return std::make_tuple(quad(l[a.second]), l[a.second].it.m0, a.second) <
-                   std::make_tuple(quad(l[b.second]), l[b.second].it.m0, b.second);
-        });
-        std::vector<Cost> sorted;
-        for (const auto& o : order) sorted.push_back(l[o.second]);
-        l.swap(sorted);
+        std::stable_sort(l.begin(), l.end(), [](const Entry& a, const Entry& b) { return a.top > b.top; });
         len = std::max(len, l.size());
     }
     out.resize(len * kXcds, decltype(Cost::it){});  // empty items: mcnt = 0, nrow = 0
     for (int x = 0; x < kXcds; ++x)
-        for (size_t j = 0; j < lists[x].size(); ++j) out[j * kXcds + x] = lists[x][j].it;
+        for (size_t j = 0; j < lists[x].size(); ++j) out[j * kXcds + x] = v[lists[x][j].i].it;
     return out;
 }
 
@@ -413,7 +438,7 @@ static int run_ring(int mode, const RingItem* d_items, const std::vector<RingCla
 // adjoint (k_adj), and the length above which Bluestein rings are split in
 // two half transforms.  Chosen by cmbl_tune (timed candidates) and kept in a
 // table keyed by (device architecture, nside, lmax); cmbl_map_create takes a
-// geometry's entry, else the rule of choose_k.  The table file next to the
+// geometry's entry, else rule_tuning.  The table file next to the
 // library, tuning_<arch>.txt, is read at the first map creation (or the file
 // named by CMBL_TUNING_FILE).
 struct TuneEntry {
@@ -574,8 +599,9 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     mp->lds_ring = lds_bytes(std::max(maxM, 2 * kRingThreads));
 
     // ---- recurrence tables (long double on the host, rounded once)
-    // A is read up to two rows of eight past the last degree (k_adj)
-    std::vector<double> A(mp->nalm + 16, 0.0), Nrm(mp->nalm, 1.0);
+    // A is read past the last degree: up to two rows of eight (k_adj), and room
+    // for the loads ahead of use
+    std::vector<double> A(mp->nalm + 80, 0.0), Nrm(mp->nalm, 1.0);
     for (int m = 0; m <= L; ++m) {
         const long b = moff(L, m) - m;
         long double Nm2 = 1.0L, Nm1 = 1.0L;  // N_{l-2}, N_{l-1}
@@ -661,7 +687,6 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     CMBL_TRY(dupload(mp, &p_so, scrofs));
     d.ring_scrofs = p_so;
     CMBL_TRY(dalloc(mp, &d.ring_scr, (size_t)std::max<long>(scr_total, 1)));
-    A.resize(A.size() + 64, 0.0);  // room for the loads ahead of use past the last row
     CMBL_TRY(dupload(mp, &p_A, A));
     CMBL_TRY(dupload(mp, &p_N, Nrm));
     CMBL_TRY(dupload(mp, &p_sv, seed_v));
@@ -740,18 +765,24 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     CMBL_TRY(launch_scan(mp->K1, d_all, (int)all.size(), mp->d_desc, d_ls, nullptr));
     std::vector<int> lstart((size_t)(L + 1) * npad);
     CMBL_HIP(hipMemcpy(lstart.data(), d_ls, sizeof(int) * lstart.size(), hipMemcpyDeviceToHost));
-    // padding pairs never constrain liveness
+    // first and last live l of each 64 ring pairs; padding pairs never constrain liveness
+    const int n64 = npad / 64;
+    mp->lmin64.assign((size_t)(L + 1) * n64, L + 1);
+    std::vector<int> lmax64((size_t)(L + 1) * n64, -1);
     for (int m = 0; m <= L; ++m)
-        for (int p = mp->npair; p < npad; ++p) lstart[(size_t)m * npad + p] = L + 1;
-
-    mp->lmin64.assign((size_t)(L + 1) * (npad / 64), L + 1);
-    for (int m = 0; m <= L; ++m)
-        for (int q = 0; q < npad; ++q) {
-            int& v = mp->lmin64[(size_t)m * (npad / 64) + q / 64];
-            v = std::min(v, lstart[(size_t)m * npad + q]);
+        for (int u = 0; u < n64 && 64 * u < mp->npair; ++u) {
+            const int* v = lstart.data() + (size_t)m * npad + 64 * u;
+            const int n = std::min(64, mp->npair - 64 * u);
+            int lo = L + 1, hi = -1;
+            for (int j = 0; j < n; ++j) {
+                lo = std::min(lo, v[j]);
+                hi = std::max(hi, v[j] <= L ? v[j] : -1);
+            }
+            mp->lmin64[(size_t)m * n64 + u] = lo;
+            lmax64[(size_t)m * n64 + u] = hi;
         }
     std::vector<ItemCost> c1;
-    build_items(mp, mp->K1, lstart, 0, &c1);
+    build_items(mp, mp->K1, lmax64, 0, &c1);
     mp->cost1 = c1;
     mp->items1 = order_items(c1);
     mp->nitems1 = (int)mp->items1.size();
@@ -773,11 +804,12 @@ static int map_create(cmbl_map* mp, int nside, int lmax, const cmbl_tuning& tune
     CMBL_TRY(dalloc(mp, &d.upart, (size_t)mp->nrb5 * mp->nalm * 2));
     CMBL_HIP(hipMemset(d.upart, 0, sizeof(double) * (size_t)mp->nrb5 * mp->nalm * 2));
     {
-        std::vector<AdjCap> caps;
-        build_adj(mp, mp->K5, false, &mp->cost5, &caps);
-        CMBL_TRY(fill_adj(mp, &mp->cost5, &caps, &mp->allocs));
-        for (AdjCost& c : mp->cost5) c = adj_for(c, 0, d);
-        const std::vector<AdjItem> items5 = order_items(mp->cost5);
+        AdjCaps caps;
+        std::vector<AdjCost> c5;
+        build_adj(mp, mp->K5, adj_segment(adj_live(mp, mp->K5), L), &c5, &caps);
+        CMBL_TRY(fill_adj(mp, &c5, &caps, &mp->allocs));
+        for (AdjCost& c : c5) c = adj_for(c, 0, d);
+        const std::vector<AdjItem> items5 = order_items(c5);
         mp->nitems5 = (int)items5.size();
         CMBL_TRY(dupload(mp, &mp->d_items5, items5));
     }
@@ -1577,11 +1609,44 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
             }
         }
     }
+    // per geometry (nside, lmax, matrix cores); one segment rule for the launch
+    // that carries all the other maps' items
     struct AdjSet {
         std::vector<AdjCost> items;
-        int K;
+        int K = 1;
+        size_t live = 0;
+        bool built = false;
     };
-    std::map<std::tuple<int, int, bool>, AdjSet> adj_sets;  // (nside, lmax, matrix cores)
+    std::map<std::tuple<int, int, bool>, AdjSet> adj_sets;
+    size_t adj_total = 0;
+    std::vector<size_t> uofs(nmaps, 0);  // partial sums of the batch's own, in one buffer (in doubles)
+    std::vector<int> unrb(nmaps, 0);     // their ring blocks (0: the map's own serve)
+    size_t utotal = 0;
+    for (int i = 0; i < nmaps; ++i) {
+        if (!maps[i]) continue;
+        const bool mma = agroup_of[i] >= 0;
+        AdjSet& as = adj_sets[std::make_tuple(maps[i]->nside, maps[i]->L, mma)];
+        if (!mma) {
+            if (as.live == 0) {
+                while (as.K < 8 && 64 * as.K < maps[i]->npair) as.K *= 2;
+                as.live = adj_live(maps[i], as.K);
+            }
+            adj_total += as.live;
+            if (as.K == maps[i]->K5) continue;
+        }
+        const int per = 64 * (mma ? kMmaWaves : as.K);  // ring pairs of a partial sum
+        unrb[i] = (maps[i]->npair + per - 1) / per;
+        uofs[i] = utotal;
+        utotal += (size_t)unrb[i] * maps[i]->nalm * 2;
+    }
+    double* upart = nullptr;
+    if (utotal > 0) {
+        void* pb = nullptr;
+        if (hipMalloc(&pb, sizeof(double) * utotal) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
+        b->allocs.push_back(pb);
+        if (hipMemset(pb, 0, sizeof(double) * utotal) != hipSuccess) return cleanup(fail(CMBL_ERR_HIP, "batch"));
+        upart = (double*)pb;
+    }
     std::vector<ItemCost> wa;  // items of the matrix-core adjoint, map = group
     std::vector<MmaSub> subs;
     std::vector<ItemCost> ws[2];  // items of the matrix-core synthesis by K - 1, map = its group
@@ -1627,28 +1692,17 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
         }
         {
             const bool mma = agroup_of[i] >= 0;
-            const auto key = std::make_tuple(mp->nside, mp->L, mma);
-            auto f = adj_sets.find(key);
-            if (f == adj_sets.end()) {
-                f = adj_sets.emplace(key, AdjSet{{}, 1}).first;
-                AdjSet& as = f->second;
-                while (!mma && as.K < 8 && 64 * as.K < mp->npair) as.K *= 2;
-                std::vector<AdjCap> caps;
-                build_adj(mp, as.K, mma, &as.items, &caps);
+            AdjSet& as = adj_sets[std::make_tuple(mp->nside, mp->L, mma)];
+            if (!as.built) {
+                AdjCaps caps;
+                build_adj(mp, as.K, mma ? adj_whole(mp->L) : adj_segment(adj_total, mp->L), &as.items, &caps);
                 const int rc = fill_adj(mp, &as.items, &caps, &b->allocs);
                 if (rc != CMBL_OK) return cleanup(rc);
+                as.built = true;
             }
-            const AdjSet& as = f->second;
-            const int per = 64 * (mma ? kMmaWaves : as.K);  // ring pairs of a partial sum
-            if (mma || as.K != mp->K5) {
-                const int nrb = (mp->npair + per - 1) / per;
-                const size_t n = (size_t)nrb * mp->nalm * 2;
-                void* pb = nullptr;
-                if (hipMalloc(&pb, sizeof(double) * n) != hipSuccess) return cleanup(fail(CMBL_ERR_ALLOC, "batch"));
-                b->allocs.push_back(pb);
-                if (hipMemset(pb, 0, sizeof(double) * n) != hipSuccess) return cleanup(fail(CMBL_ERR_HIP, "batch"));
-                descs.back().upart = (double*)pb;
-                descs.back().nrb5 = nrb;
+            if (unrb[i] > 0) {
+                descs.back().upart = upart + uofs[i];
+                descs.back().nrb5 = unrb[i];
             }
             if (!mma) {
                 int k5 = 0;
@@ -1776,6 +1830,8 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
     b->nring_items = (int)rings.size();
     if (hipMemcpy(q, rings.data(), sizeof(RingItem) * rings.size(), hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(CMBL_ERR_HIP, "batch upload"));
+    // the start states are in place
+    if (hipDeviceSynchronize() != hipSuccess) return cleanup(fail(CMBL_ERR_HIP, "batch set-up"));
     *out = b;
     return CMBL_OK;
 }
