@@ -315,6 +315,19 @@ int launch_synth_pairs(int K, const WorkItem* items, int nitems, const MapDesc* 
 int launch_adj(int K, const AdjItem* items, int nitems, hipStream_t s);
 constexpr int kSynG = 8;     // maps of a matrix-core group
 constexpr int kSynMinG = 6;  // fewest maps of such a group
+// Fewest maps of an adjoint group; `rest`: beside full groups of the same maps,
+// whose launch it joins.  The products cost a group of any size about what they
+// cost eight maps, so alone 3, 4 and 5 maps are faster one by one (us, one by
+// one / group: nside 64 52, 48, 56 / 60, 55, 62; nside 256 192, 184, 238 / 212,
+// 198, 245; nside 512 664, 813, 1041 / 833, 921, 1076).  Beside full groups the
+// launch saved decides on small maps: 9 to 13 maps, the rest one by one / as a
+// group, nside 64 80, 87, 97, 91, 101 / 74, 81, 90, 83, 94; nside 256 378, 433,
+// 491, 483, 543 / 403, 443, 491, 480, 527; nside 512 1622, 1799, 2009, 2161,
+// 2383 / 1945, 2053, 2200, 2282, 2428.
+constexpr int adj_min_group(int npair, bool rest)
+{
+    return !rest ? 6 : npair <= 256 ? 1 : npair <= 512 ? 3 : 6;
+}
 constexpr int kMmaWaves = 4;  // waves of a matrix-core adjoint workgroup, 64 ring pairs each
 // Its waves' first l (-1: none) and start states (AdjItem's form).
 struct MmaSub {

@@ -1586,8 +1586,8 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
         }
     }
     std::vector<ItemCost> wp[2];  // items of the pairs by K - 1, map = the pair
-    // the adjoint: groups of at least kSynMinG maps of one geometry on the
-    // matrix cores; the others map by map with eight ring pairs per lane
+    // the adjoint: groups of maps of one geometry (adj_min_group) on the matrix
+    // cores; the others map by map with eight ring pairs per lane
     // (there are items enough in a batch).  Start states and partial sums that
     // the maps do not have belong to the batch, the states once per geometry
     std::vector<int> agroup_of(nmaps, -1);
@@ -1598,14 +1598,14 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
             if (maps[i]) bya[std::make_pair(maps[i]->nside, maps[i]->L)].push_back(i);
         for (auto& kv : bya) {
             const std::vector<int>& v = kv.second;
-            for (size_t at = 0; v.size() - at >= (size_t)kSynMinG; at += kSynG) {
+            for (size_t at = 0; at < v.size(); at += kSynG) {
                 const size_t n = std::min<size_t>(kSynG, v.size() - at);
+                if (n < (size_t)adj_min_group(maps[v[at]]->npair, at > 0)) break;
                 const int gid = (int)atable.size() / kSynG;
                 for (size_t j = 0; j < (size_t)kSynG; ++j) {
                     atable.push_back(j < n ? v[at + j] : -1);
                     if (j < n) agroup_of[v[at + j]] = gid;
                 }
-                if (n < (size_t)kSynG) break;
             }
         }
     }

@@ -79,3 +79,30 @@ def test_pol_edges(nside, lmax, k_synth):
     for got, want in zip(mp.alm2map_pol(t, e, b), oracle.alm2map_pol(nside, lmax, t, e, b)):
         assert rel(got, want) < 1e-10
     mp.close()
+
+
+# the rest of a batch beside a full matrix-core group: one map up to nside 128 and
+# three at nside 256 form a group of their own, fewer and larger maps do not
+@pytest.mark.parametrize("nside,lmax,nmaps", [(64, 65, 9), (128, 100, 11), (256, 130, 10), (256, 130, 11), (512, 60, 13),
+                                              (512, 60, 14)])
+def test_batch_rest_beside_a_group(nside, lmax, nmaps):
+    import torch
+
+    print("case rest", nside, lmax, nmaps, flush=True)
+    cases = [Case(nside, lmax, 5400.0 / lmax / 60.0, 10.0 + i, 12.0, seed=17 * i + nmaps) for i in range(nmaps)]
+    maps = [make_map(c, 1, 1) for c in cases]
+    xs = [torch.from_numpy(c.x).to("cuda:0") for c in cases]
+    gs = [torch.empty_like(x) for x in xs]
+    f = torch.empty(nmaps, dtype=torch.float64, device="cuda:0")
+    b = cm.Batch(maps)
+    b.value_and_grad_device([x.data_ptr() for x in xs], f.data_ptr(), [g.data_ptr() for g in gs],
+                            torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for i in (0, 7, 8, nmaps - 1):
+        c = cases[i]
+        fo, go = oracle.neg2lnL(c.nside, c.lmax, c.x, c.beam, c.cl, c.d, c.w)
+        assert abs(f[i].item() - fo) < 1e-10 * abs(fo)
+        assert rel(gs[i].cpu().numpy(), go) < 1e-10
+    b.close()
+    for mp in maps:
+        mp.close()
