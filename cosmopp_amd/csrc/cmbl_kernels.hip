@@ -642,15 +642,6 @@ __device__ __forceinline__ bool all_live(const int (&sc)[K])
     return __all(ok);
 }
 template <int K>
-__device__ __forceinline__ bool any_live(const int (&sc)[K])
-{
-    int ok = 0;
-#pragma unroll
-    for (int k = 0; k < K; ++k) ok |= (sc[k] == 0);
-    return __any(ok);
-}
-
-template <int K>
 __device__ __forceinline__ bool rescale(double (&mu1)[K], double (&mu2)[K], int (&sc)[K])
 {
     int need = 0;
@@ -680,20 +671,11 @@ struct Ring {
     }
 };
 
-// Recurrence state of the spin-2 and set-up kernels.
+// Recurrence state of the set-up kernels.
 template <int K>
 struct LegState {
     double mu1[K], mu2[K];  // mu_l, mu_{l-1}, odd ones divided by x (k_scan: not)
-    double gate[K];         // 1 for live lanes, 0 otherwise (scaled path only)
     int sc[K];
-    bool live, all;
-    __device__ __forceinline__ void refresh()
-    {
-        live = any_live<K>(sc);
-        all = all_live<K>(sc);
-#pragma unroll
-        for (int k = 0; k < K; ++k) gate[k] = sc[k] == 0 ? 1.0 : 0.0;
-    }
 };
 
 // -------------------------------------------------------------- synthesis
@@ -753,13 +735,14 @@ __device__ __forceinline__ void syn_steps(SynState<K>& st, SynAcc<K> (&ac)[G], c
 // Rescale check after a row of eight steps while some lane is scaled: lanes
 // above 2^900 drop by 2^-1000; a lane whose count reaches 0 clears its sums.
 // Scaled lanes (count > 0) accumulate like live ones: their scaled mu
-// (|mu| < 2^958 between checks) makes meaningless sums, which are cleared when
+// (|mu| < 2^950 between checks) makes meaningless sums, which are cleared when
 // the lane turns live and never stored while it is scaled, so the result
 // equals gating each term by the lane's state at the last check, without the
-// multiplies.  Eight steps multiply |mu| by at most prod (A_l + 1) < 2^45
-// (A_{m+1} = sqrt(2m + 2) is the largest factor), so from 2^900 nothing
-// overflows between checks; a lane whose scale count reaches 0 inside a row
-// joins at the row's end, dropping terms below 2^-42 of O(1) 2^-45.
+// multiplies.  Eight steps multiply |mu| by at most prod (A_l + 1) < 2^50 up to
+// the largest lmax, 8192 (2^49.5 at m = 8184; A_{m+1} = sqrt(2m + 3) is the
+// largest factor), so from 2^900 nothing overflows between checks.  A lane
+// below 2^-100 at one check is below 2^-50 at the next, where it joins: the
+// terms it leaves out are below 2^-50 of lambda's O(1).
 template <int K, int G>
 __device__ __forceinline__ void syn_rescale(SynState<K>& st, SynAcc<K> (&ac)[G])
 {
@@ -1193,7 +1176,7 @@ __global__ __launch_bounds__(64) void k_synth_pol(const WorkItem* __restrict__ i
 // A lane's ring-stage inputs Psi_m (even and odd parts, the odd one times x)
 // of its K ring pairs.  Lanes whose scale count is > 0 hold
 // zeros, so that the same step serves the scaled and the live path: their
-// scaled mu (|mu| < 2^958 between rescale checks) times 0 contributes exactly
+// scaled mu (|mu| < 2^950 between rescale checks) times 0 contributes exactly
 // 0.  A lane that turns live loads its inputs at the rescale check where its
 // count reaches 0.
 template <int K>
@@ -1320,11 +1303,9 @@ __device__ __forceinline__ void adj_step(AdjState<K>& st, bool odd, double A, co
 // row, until every lane is live.  a holds row r's coefficients; a row loads
 // the next one's after its first step (scalar loads return out of order: the
 // wait before that step would otherwise cover them), and reads the previous
-// row's tile there, which it finishes halfway.  Eight steps multiply |mu| by
-// at most prod (A_l + 1) < 2^45 (A_{m+1} = sqrt(2m + 2) is the largest
-// factor), so from 2^900 no value overflows between checks; a lane whose scale
-// count reaches 0 inside a row joins at the row's end, dropping terms below
-// 2^-42 of O(1).
+// row's tile there, which it finishes halfway.  What eight steps can
+// multiply |mu| by, and what a lane that joins at a row's end leaves out, is as
+// in syn_rescale.
 template <int K, int KA, bool SCALED>
 __device__ __forceinline__ bool adj_rows(AdjState<K>& st, AdjRed& rd, const AdjItem& it, scdouble* A, double (&a)[8],
                                          const double* yl, int& r, int rend, bool all)
