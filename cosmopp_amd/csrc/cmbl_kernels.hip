@@ -671,10 +671,10 @@ struct Ring {
     }
 };
 
-// Recurrence state of the set-up kernels.
+// Recurrence state of k_scan.
 template <int K>
 struct LegState {
-    double mu1[K], mu2[K];  // mu_l, mu_{l-1}, odd ones divided by x (k_scan: not)
+    double mu1[K], mu2[K];  // mu_l, mu_{l-1}
     int sc[K];
 };
 
@@ -1800,18 +1800,54 @@ __global__ __launch_bounds__(64, 2) void k_synth_mma(const WorkItem* __restrict_
 // -------------------------------------------------------------- set-up passes
 // All run the scaled recurrence from the seed lambda_mm.
 
-// One step of the start states' recurrence (odd members divided by cos theta
-// = c), x^2 = y + lo exactly.
+// The start states' recurrence (odd members divided by cos theta = c) carries
+// each value as a sum hi + lo and c^2 = y + d exactly: a start state's error is
+// that of every l after it.  (Plain doubles cannot hold the correction of y: the
+// fma that adds it to mu_{l-2} rounds it away, and its drift grew with l.)
 template <int K>
-__device__ __forceinline__ void capture_step(LegState<K>& st, const double (&c)[K], bool odd, double Al)
+struct CaptureState {
+    double h1[K], e1[K], h2[K], e2[K];  // mu_l and mu_{l-1}, hi and lo
+    int sc[K];
+};
+
+// hi + lo of q + b + lo
+__device__ __forceinline__ void two_sum(double q, double b, double lo, double& hi, double& e)
 {
+#pragma clang fp contract(off)
+    const double s = q + b, t = s - q;
+    const double r = ((q - (s - t)) + (b - t)) + lo;
+    hi = s + r;
+    e = r - (hi - s);
+}
+
+template <int K>
+__device__ __forceinline__ void capture_step(CaptureState<K>& st, const double (&c)[K], bool odd, double Al)
+{
+#pragma clang fp contract(off)  // q is rounded before the sum
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const double y = c[k] * c[k], lo = fma(c[k], c[k], -y);
-        const double nu = odd ? fma(Al, st.mu1[k], -st.mu2[k])
-                              : fma(Al * y, st.mu1[k], fma(Al * lo, st.mu1[k], -st.mu2[k]));
-        st.mu2[k] = st.mu1[k];
-        st.mu1[k] = nu;
+        double p = st.h1[k], e = st.e1[k];
+        if (!odd) {
+            const double y = c[k] * c[k], d = fma(c[k], c[k], -y);
+            p = y * st.h1[k];
+            e = fma(y, st.h1[k], -p) + fma(y, st.e1[k], d * st.h1[k]);
+        }
+        const double q = Al * p;
+        const double f = fma(Al, p, -q) + Al * e;
+        double h, l;
+        two_sum(q, -st.h2[k], f - st.e2[k], h, l);
+        st.h2[k] = st.h1[k];
+        st.e2[k] = st.e1[k];
+        st.h1[k] = h;
+        st.e1[k] = l;
+        // as rescale()
+        const bool r = st.sc[k] > 0 && fabs(h) > kScaleHi;
+        const double f2 = r ? kScaleDn : 1.0;
+        st.h1[k] *= f2;
+        st.e1[k] *= f2;
+        st.h2[k] *= f2;
+        st.e2[k] *= f2;
+        st.sc[k] -= r ? 1 : 0;
     }
 }
 
@@ -1876,26 +1912,23 @@ __global__ __launch_bounds__(64) void k_capture(const WorkItem* __restrict__ ite
     const int lane = threadIdx.x;
     const int m = it.m0;
     const double* __restrict__ A = md.A + moff(L, m) - m;
-    LegState<K> st;
+    CaptureState<K> st;
     int p[K];
     double c[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         p[k] = it.rb * 64 * K + k * 64 + lane;
         c[k] = md.ring_x[p[k]];
-        st.mu1[k] = md.seed_v[(long)m * npad + p[k]];
+        st.h1[k] = md.seed_v[(long)m * npad + p[k]];
         st.sc[k] = md.seed_k[(long)m * npad + p[k]];
-        st.mu2[k] = 0.0;
+        st.e1[k] = st.h2[k] = st.e2[k] = 0.0;
     }
-    for (int l = m + 1; l <= it.lfirst; ++l) {
-        capture_step<K>(st, c, ((l - m) & 1) != 0, A[l]);
-        rescale<K>(st.mu1, st.mu2, st.sc);
-    }
+    for (int l = m + 1; l <= it.lfirst; ++l) capture_step<K>(st, c, ((l - m) & 1) != 0, A[l]);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const long q = (long)m * npad + p[k];
-        prev[q] = st.mu2[k];
-        cur[q] = st.mu1[k];
+        prev[q] = st.h2[k];
+        cur[q] = st.h1[k];
         kout[q] = st.sc[k];
     }
 }
@@ -1913,20 +1946,17 @@ __global__ __launch_bounds__(64) void k_adj_capture(const AdjCap* __restrict__ c
     const int i0 = runs[blockIdx.x], i1 = runs[blockIdx.x + 1];
     const int L = md.L, m = caps[i0].m, p = caps[i0].p0 + threadIdx.x;
     const double* __restrict__ A = md.A + moff(L, m) - m;
-    LegState<1> s;
+    CaptureState<1> s;
     const double x[1] = {md.ring_x[p]};
-    s.mu1[0] = md.seed_v[(long)m * md.npair_pad + p];
+    s.h1[0] = md.seed_v[(long)m * md.npair_pad + p];
     s.sc[0] = md.seed_k[(long)m * md.npair_pad + p];
-    s.mu2[0] = 0.0;
+    s.e1[0] = s.h2[0] = s.e2[0] = 0.0;
     int l = m + 1;
     for (int i = i0; i < i1; ++i) {
         const AdjCap c = caps[i];
-        for (; l < c.l; ++l) {
-            capture_step<1>(s, x, ((l - m) & 1) != 0, A[l]);
-            rescale<1>(s.mu1, s.mu2, s.sc);
-        }
+        for (; l < c.l; ++l) capture_step<1>(s, x, ((l - m) & 1) != 0, A[l]);
         const long q = 64L * c.at + threadIdx.x;
-        st[q] = c.l == m ? make_double2(-s.mu1[0], 0.0) : make_double2(s.mu2[0], s.mu1[0]);
+        st[q] = c.l == m ? make_double2(-s.h1[0], 0.0) : make_double2(s.h2[0], s.h1[0]);
         sk[q] = s.sc[0];
     }
 }
