@@ -620,9 +620,10 @@ __global__ __launch_bounds__(256) void k_reorder(const double* __restrict__ in, 
 // of every 16 l-steps the first takes x^2 plus eight times the rounding error
 // (rounded again: Ring::ya), and of every eighth 16 also eight times what that
 // rounding left (yb), so that the mean multiplier is x^2 to 2^-60 and the
-// phase never drifts by more than a few steps' rounding.  The error against
-// higher precision is then that of the plain recurrence (rms over rings,
-// nside 64 to 1024: 0.9 to 1.2 times).
+// phase never drifts by more than a few steps' rounding.  From start states
+// that are right to the last place (CaptureState) the error against higher
+// precision is that of the plain recurrence (by ring 0.8 to 1.25 times; whole
+// results, nside 64 to 1024: 0.93 to 1.07 times).
 // The wave-uniform coefficients (A_lm and, for the synthesis, B_l N_lm a_lm)
 // come through the scalar cache, or from a row of 16 lanes, a step group ahead:
 // read from LDS by every wave they kept its port (128 bytes per clock) as busy
