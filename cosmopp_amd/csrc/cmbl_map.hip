@@ -8,6 +8,7 @@
 #include <dlfcn.h>
 #include <fstream>
 #include <map>
+#include <set>
 #include <mutex>
 #include <sstream>
 #include <random>
@@ -260,6 +261,45 @@ static void build_adj(const cmbl_map* mp, int K, int seg, std::vector<AdjCost>* 
                 }
             }
         }
+}
+
+// Ring pairs per lane of a map's adjoint in a batch, at most `cap`, no more than
+// the map fills.
+static int batch_adj_k(int npair, int cap)
+{
+    int k = 1;
+    while (k < cap && 64 * k < npair) k *= 2;
+    return k;
+}
+
+// The cap for a batch's maps (npair, lmax) outside matrix-core groups.  More ring
+// pairs per lane save reductions, in proportion to the work w = sum npair nalm of
+// the maps that can take them; fewer make more items for the launch's tail, and a
+// launch less where smaller maps are in the batch (each K is a launch of its own).
+// us per batch at cap 2 / 4 / 8.  Equal maps: 1 of nside 128 / lmax 256 (w 8e6) 47.2 /
+// 48.5 / 48.5, 1 and 3 of nside 256 / lmax 512 (7e7, 2e8) 95, 192 / 92, 184 / 95, 193,
+// 1 and 2 of nside 512 / lmax 600 (1.9e8, 3.7e8) 154, 267 / 145, 246 / 152, 250, 1 of
+// nside 512 / lmax 1024 (5.4e8) 285 / 260 / 256, 2 of nside 1024 / lmax 1536 (4.8e9)
+// 1779 / 1547 / 1475.  Maps of nside 64 to 256 together (5e7; 1.3e8) 95 / 100 / 112; 129 /
+// 132 / 147; of nside 64 to 512 (2.3e8; 6.3e8) 216 / 216 / 229; 367 / 351 / 363; of nside
+// 128 to 1024 (1.9e9, 2.4e9) 896, 1118 / 810, 1011 / 809, 1005.
+static int batch_adj_cap(const std::vector<std::pair<int, int>>& maps)
+{
+    int cap = 2;
+    for (int next : {4, 8}) {
+        double w = 0.0;
+        std::set<int> now, then;  // the launches at either cap
+        for (const auto& m : maps) {
+            now.insert(batch_adj_k(m.first, cap));
+            then.insert(batch_adj_k(m.first, next));
+            if (batch_adj_k(m.first, next) == next)
+                w += 0.5 * (m.second + 1.0) * (m.second + 2.0) * m.first;
+        }
+        const bool more = then.size() > now.size();
+        if (w < (next == 4 ? (more ? 1.3e8 : 2.2e7) : (more ? 1.5e9 : 4e8))) break;
+        cap = next;
+    }
+    return cap;
 }
 
 // Allocates and starts to fill the start states of build_adj's items (their st
@@ -1587,8 +1627,8 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
     }
     std::vector<ItemCost> wp[2];  // items of the pairs by K - 1, map = the pair
     // the adjoint: groups of maps of one geometry (adj_min_group) on the matrix
-    // cores; the others map by map with eight ring pairs per lane
-    // (there are items enough in a batch).  Start states and partial sums that
+    // cores; the others map by map with up to eight ring pairs per lane
+    // (batch_adj_cap).  Start states and partial sums that
     // the maps do not have belong to the batch, the states once per geometry
     std::vector<int> agroup_of(nmaps, -1);
     std::vector<int> atable;  // kSynG map indices per group (-1: empty)
@@ -1618,6 +1658,10 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
         bool built = false;
     };
     std::map<std::tuple<int, int, bool>, AdjSet> adj_sets;
+    std::vector<std::pair<int, int>> vmaps;  // (npair, lmax) of the maps outside groups
+    for (int i = 0; i < nmaps; ++i)
+        if (maps[i] && agroup_of[i] < 0) vmaps.push_back({maps[i]->npair, maps[i]->L});
+    const int kcap = batch_adj_cap(vmaps);
     size_t adj_total = 0;
     std::vector<size_t> uofs(nmaps, 0);  // partial sums of the batch's own, in one buffer (in doubles)
     std::vector<int> unrb(nmaps, 0);     // their ring blocks (0: the map's own serve)
@@ -1628,7 +1672,7 @@ int cmbl_batch_create(cmbl_batch** out, cmbl_map* const* maps, int nmaps)
         AdjSet& as = adj_sets[std::make_tuple(maps[i]->nside, maps[i]->L, mma)];
         if (!mma) {
             if (as.live == 0) {
-                while (as.K < 8 && 64 * as.K < maps[i]->npair) as.K *= 2;
+                as.K = batch_adj_k(maps[i]->npair, kcap);
                 as.live = adj_live(maps[i], as.K);
             }
             adj_total += as.live;

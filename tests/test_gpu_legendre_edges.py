@@ -106,3 +106,29 @@ def test_batch_rest_beside_a_group(nside, lmax, nmaps):
     b.close()
     for mp in maps:
         mp.close()
+
+
+# batches whose maps share no geometry, on both sides of the lines between 2, 4 and 8
+# ring pairs per lane, against the maps one by one
+@pytest.mark.parametrize("sizes", [[(64, 130), (128, 133), (256, 300)], [(64, 130), (512, 520), (8, 20)],
+                                   [(256, 140), (128, 60)], [(512, 900)], [(32, 64), (512, 1500), (512, 1400)]])
+def test_batch_ring_pairs_per_lane(sizes):
+    import torch
+
+    print("case ring pairs", sizes, flush=True)
+    cases = [Case(n, l, 5400.0 / l / 60.0, 10.0 + n, 12.0, seed=n + l) for n, l in sizes]
+    maps = [make_map(c, 1, 1) for c in cases]
+    xs = [torch.from_numpy(c.x).to("cuda:0") for c in cases]
+    gs = [torch.empty_like(x) for x in xs]
+    f = torch.empty(len(maps), dtype=torch.float64, device="cuda:0")
+    b = cm.Batch(maps)
+    b.value_and_grad_device([x.data_ptr() for x in xs], f.data_ptr(), [g.data_ptr() for g in gs],
+                            torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for i, (c, mp) in enumerate(zip(cases, maps)):
+        fo, go = mp.value_and_grad(c.x)
+        assert abs(f[i].item() - fo) < 1e-10 * abs(fo)
+        assert rel(gs[i].cpu().numpy(), go) < 1e-10
+    b.close()
+    for mp in maps:
+        mp.close()
